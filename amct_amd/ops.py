@@ -190,6 +190,26 @@ def hessian_update(hessian, x, beta, alpha):
     return hessian
 
 
+def gptq_factor(hessian, perm, damp, bad):
+    """Upper triangular u with (hessian[perm][:, perm] (+ 1 on zero diagonal entries) + damp I)^-1 = u^T u, from one
+    Cholesky factorisation and one triangular inverse on the matrix pipe.  hessian fp32 [C,C], perm int64 [C], damp fp32
+    (one element), bad int32 (one element, zero; becomes 1 when a pivot is not positive)."""
+    dev = _dev(hessian, perm, damp, bad)
+    cols = hessian.shape[0]
+    _need(hessian.dim() == 2 and hessian.shape[1] == cols and hessian.dtype == torch.float32, "gptq_factor: hessian must be a square fp32 matrix")
+    _need(perm.dtype == torch.int64 and perm.numel() == cols, "gptq_factor: perm must hold {} int64 indices", cols)
+    _need(damp.dtype == torch.float32 and damp.numel() == 1, "gptq_factor: damp must be one fp32 value")
+    _need(bad.dtype == torch.int32 and bad.numel() == 1, "gptq_factor: bad must be one int32 value")
+    hessian, perm = _c(hessian), _c(perm)
+    u = torch.empty_like(hessian)
+    lib = _lib.load()
+    nbytes = lib.amct_gptq_factor_workspace_bytes(cols)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    with _on(dev):
+        _lib.check(lib.amct_gptq_factor(_p(hessian), _p(perm), _p(damp), _p(u), _p(bad), cols, _p(ws), nbytes, _stream(dev)))
+    return u
+
+
 def scale_offset(vmax, vmin, bits, symmetric, scope_rule=SCOPE_AMCT, bad=None):
     """Elementwise (max, min) -> (scale fp32, offset int32 | None), same shape as the inputs."""
     dev = _dev(vmax, vmin, bad)

@@ -1,7 +1,7 @@
 """Host-side mirror of the weight optimisation of amct_pytorch/quantize_op/gptq_module.py (:91-155, :161-186)
 with the tensors resident on the device.  The column loop of each block is one kernel launch
-(amct_gptq_block); ordering, damping, the two Cholesky factorisations and the trailing update are library
-calls on the device, as they are library calls in the reference."""
+(amct_gptq_block) and the factorisations are one call (amct_gptq_factor); ordering, damping and the trailing update are
+library calls on the device."""
 import math
 
 import torch
@@ -64,6 +64,16 @@ def gptq_block(weight_sorted, i1, i2, hinv, scale_w, offset_w, gidx, qmin, qmax)
     return err
 
 
+def _read_later(flag):
+    """(host copy of a device flag, event behind the copy): read the copy after event.synchronize(), which waits for the
+    work up to here and not for what is enqueued behind it."""
+    host = torch.empty(flag.shape, dtype=flag.dtype, pin_memory=True)
+    host.copy_(flag, non_blocking=True)
+    event = torch.cuda.Event()
+    event.record()
+    return host, event
+
+
 @torch.no_grad()
 def get_opt_weight_and_quant_factor(weight, hessian, quant_config, block_size=128, perc_damp=0.01):
     """:91-155.  weight [N, K] (any float dtype), hessian [K, K] fp32 on the same device.  Returns
@@ -74,23 +84,20 @@ def get_opt_weight_and_quant_factor(weight, hessian, quant_config, block_size=12
     bits = int(wts_type.replace('int', ''))
     columns = weight.shape[1]
     out_dtype = weight.dtype
-    weight = weight.clone().float()
-    hessian = hessian.clone()
-    dead = torch.diag(hessian) == 0
-    hessian[dead, dead] = 1
-    weight[:, dead] = 0
-    perm = torch.argsort(torch.diag(hessian), descending=True)
+    hessian = hessian.float()
+    diag = torch.diag(hessian)
+    dead = diag == 0
+    diag = torch.where(dead, torch.ones_like(diag), diag)
+    weight = weight.float().masked_fill(dead, 0)
+    perm = torch.argsort(diag, descending=True)
     invperm = torch.argsort(perm)
     weight_min, weight_max = get_weight_min_max_by_granularity(weight, quant_config)
     scale_w, offset_w = calculate_scale_offset(weight_max, weight_min, cfg.get('symmetric'), wts_type)
     ws = weight[:, perm].contiguous()
-    hs = hessian[perm][:, perm]
-    damp = perc_damp * torch.mean(torch.diag(hs))
-    diag = torch.arange(columns, device=weight.device)
-    hs[diag, diag] += damp
-    hs = torch.linalg.cholesky(hs)
-    hs = torch.cholesky_inverse(hs)
-    hinv = torch.linalg.cholesky(hs, upper=True).contiguous()
+    # cholesky(cholesky_inverse(cholesky(hs)), upper=True) of the permuted, damped Hessian, as one factorisation
+    bad = torch.zeros(1, dtype=torch.int32, device=weight.device)
+    hinv = ops.gptq_factor(hessian, perm, perc_damp * torch.mean(diag), bad)
+    not_positive, factored = _read_later(bad)
     sc = scale_w.reshape(-1).float().contiguous()
     zc = None if offset_w is None else offset_w.reshape(-1).to(torch.int32).contiguous()
     if group_size:
@@ -103,4 +110,8 @@ def get_opt_weight_and_quant_factor(weight, hessian, quant_config, block_size=12
         err_block = gptq_block(ws, i1, i2, hinv, sc, zc, gidx_all[i1:i2].contiguous(), qmin, qmax)
         if i2 < columns:
             ws[:, i2:] -= err_block.matmul(hinv[i1:i2, i2:])
+    factored.synchronize()                          # of the copy only: long done when the last block is enqueued
+    if int(not_positive):
+        raise torch.linalg.LinAlgError("linalg.cholesky: the factorization could not be completed because the input is "
+                                       "not positive-definite.")
     return ws[:, invperm].to(out_dtype), scale_w, offset_w

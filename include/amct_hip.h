@@ -366,6 +366,18 @@ int amct_gptq_block(float* w, int64_t ld_w, float* err_out, int64_t ld_e, const 
                     const float* scale, const int32_t* offset, int64_t scale_stride, const int32_t* gidx,
                     int64_t rows, int count, int qmin, int qmax, amct_stream_t stream);
 
+/* ---- GPTQ factorisation -----------------------------------------------------------------------
+ * The three factorisations of amct_pytorch/quantize_op/gptq_module.py:108-121 as one: with Hp = hessian[perm][:, perm],
+ * zero diagonal entries replaced by 1 and *damp added to the diagonal, u [cols, cols] = the upper triangular factor with
+ * Hp^-1 = u^T u, zeros below the diagonal (the reference's cholesky(cholesky_inverse(cholesky(Hp)), upper=True), from one
+ * Cholesky factorisation in reversed order and one triangular inverse, all fp32).  hessian is read only; perm int64, a
+ * permutation of 0 .. cols - 1; damp one fp32 on the device.  *bad (int32 on the device, zeroed by the caller) becomes 1
+ * when a pivot is not positive (u is then meaningless).  workspace: amct_gptq_factor_workspace_bytes(cols), 16-byte
+ * aligned.  cols <= 65536. */
+size_t amct_gptq_factor_workspace_bytes(int64_t cols);
+int amct_gptq_factor(const float* hessian, const int64_t* perm, const float* damp, float* u, int32_t* bad, int64_t cols,
+                     void* workspace, size_t workspace_bytes, amct_stream_t stream);
+
 /* ---- GPTQ Hessian accumulation --------------------------------------------------------------
  * The update of amct_pytorch/quantize_op/gptq_module.py:176-181 for 16-bit calibration activations:
  *   hessian *= n / (n + b);  x = sqrt(2 / (n + b)) * x.float();  hessian += x.t() @ x      (x [tokens, cols])
