@@ -158,3 +158,42 @@ def test_update_hessian_on_16_bit_activations(dev):
     exact = exact * (1 / 4) + (2 / 4) * (xd[256:].t() @ xd[256:])    # second call: batch of 3, nsamples 1 -> 4
     mine, theirs = (dh.cpu().double() - exact).abs().max(), (hess.double() - exact).abs().max()
     assert float(mine) <= 1.5 * float(theirs) + 1e-6, (float(mine), float(theirs))
+
+
+@pytest.mark.parametrize("sym", [False, True])
+@pytest.mark.parametrize("n", [1, 4, 17, 63, 300, 8192, 8193])
+@pytest.mark.parametrize("special", ['none', 'tiny weights', 'huge weights', 'inf weight', 'tiny scale', 'tiny diagonal'])
+def test_gptq_full_block_is_the_general_kernel(dev, sym, n, special):
+    """Full blocks divide by reciprocals while everything stays in the range where that gives the quotient's bits, and
+    by the division itself in the waves that leave it: the bits of the general kernel, which an odd row stride selects."""
+    g = torch.Generator().manual_seed(n)
+    count = 128
+    w = (torch.randn(n, count, generator=g) * 0.05).float()
+    s, z = iq.weight_scale_offset(w, 'channel', sym, 'int4')
+    s, z = s.reshape(n, 1).repeat(1, 2), None if z is None else z.reshape(n, 1).repeat(1, 2)
+    s[:, 1] *= 1.25
+    hinv = _hinv(count, 5)
+    row = n // 2
+    w[row, 3] = -0.0
+    if special == 'tiny weights':
+        w[row, 40:44] = torch.tensor([1e-38, -1e-42, 1e-25, -1e-20])
+        hinv = hinv * torch.eye(count)                              # nothing is added to them on the way
+    elif special == 'huge weights':
+        w[row, 7], w[row, 100] = 1e30, -3e38
+    elif special == 'inf weight':
+        w[row, 64] = float('inf')
+    elif special == 'tiny scale':
+        s[row, 1] = 1e-30
+    elif special == 'tiny diagonal':
+        hinv[17, 17] = 1e-25
+    gidx = torch.randint(0, 2, (count,), generator=g, dtype=torch.int32)
+    factors = (s.contiguous().to(dev), None if z is None else z.to(torch.int32).contiguous().to(dev), gidx.to(dev))
+    padded = torch.full((n, count + 1), 7.0, device=dev)
+    padded[:, :count] = w.to(dev)
+    want_e = gptq.gptq_block(padded, 0, count, hinv.to(dev), *factors, -8, 7)
+    got = w.to(dev)
+    got_e = gptq.gptq_block(got, 0, count, hinv.to(dev), *factors, -8, 7)
+    assert_bits_equal(got_e.nan_to_num(1.5).cpu(), want_e.nan_to_num(1.5).cpu(), "err block")
+    assert torch.equal(got_e.isnan(), want_e.isnan())
+    assert_bits_equal(got.nan_to_num(1.5).cpu(), padded[:, :count].contiguous().nan_to_num(1.5).cpu(), "weight block")
+    assert torch.equal(got.isnan(), padded[:, :count].isnan())
