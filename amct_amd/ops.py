@@ -190,6 +190,45 @@ def hessian_update(hessian, x, beta, alpha):
     return hessian
 
 
+def gptq_trail(w, err, u, i1, i2):
+    """w[:, i2:] -= err @ u[i1:i2, i2:] in place; w fp32 [N,C], err fp32 [N, i2 - i1], u fp32 [C,C] (gptq_module.py:152-153)."""
+    dev = _dev(w, err, u)
+    rows, cols = w.shape
+    for name, t, shape in (("w", w, (rows, cols)), ("err", err, (rows, i2 - i1)), ("u", u, (cols, cols))):
+        _need(t.dtype == torch.float32 and tuple(t.shape) == shape and t.is_contiguous(),
+              "gptq_trail: {} must be a contiguous fp32 tensor of shape {}", name, shape)
+    _need(0 <= i1 < i2 <= cols, "gptq_trail: no columns {}:{} in {}", i1, i2, cols)
+    with _on(dev):
+        _lib.check(_lib.load().amct_gptq_trail(_p(w) + 4 * i2, cols, _p(err), i2 - i1, _p(u) + 4 * (i1 * cols + i2), cols, rows,
+                                               cols - i2, i2 - i1, _stream(dev)))
+
+
+def gptq_order(w, perm, dead):
+    """w[:, perm] as fp32, the columns of w marked in dead (bool [C]) as zeros."""
+    dev = _dev(w, perm, dead)
+    w = _c(w)
+    rows, cols = w.shape
+    _need(perm.dtype == torch.int64 and perm.numel() == cols and perm.is_contiguous(), "gptq_order: perm must hold {} int64 indices", cols)
+    _need(dead.dtype == torch.bool and dead.numel() == cols and dead.is_contiguous(), "gptq_order: dead must hold {} truth values", cols)
+    out = torch.empty(rows, cols, dtype=torch.float32, device=dev)
+    with _on(dev):
+        _lib.check(_lib.load().amct_gptq_order(_p(w), _p(out), _p(perm), _p(dead), rows, cols, 0, dtype_code(w.dtype), _stream(dev)))
+    return out
+
+
+def gptq_order_back(ws, perm, dtype):
+    """The inverse of gptq_order's column order: out[:, perm] = ws (fp32), in dtype."""
+    dev = _dev(ws, perm)
+    ws = _c(ws)
+    rows, cols = ws.shape
+    _need(ws.dtype == torch.float32, "gptq_order_back: ws must be fp32")
+    _need(perm.dtype == torch.int64 and perm.numel() == cols and perm.is_contiguous(), "gptq_order_back: perm must hold {} int64 indices", cols)
+    out = torch.empty(rows, cols, dtype=dtype, device=dev)
+    with _on(dev):
+        _lib.check(_lib.load().amct_gptq_order(_p(ws), _p(out), _p(perm), None, rows, cols, 1, dtype_code(dtype), _stream(dev)))
+    return out
+
+
 def gptq_factor(hessian, perm, damp, bad):
     """Upper triangular u with (hessian[perm][:, perm] (+ 1 on zero diagonal entries) + damp I)^-1 = u^T u, from one
     Cholesky factorisation and one triangular inverse on the matrix pipe.  hessian fp32 [C,C], perm int64 [C], damp fp32

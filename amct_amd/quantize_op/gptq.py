@@ -1,13 +1,12 @@
 """Host-side mirror of the weight optimisation of amct_pytorch/quantize_op/gptq_module.py (:91-155, :161-186)
-with the tensors resident on the device.  The column loop of each block is one kernel launch
-(amct_gptq_block) and the factorisations are one call (amct_gptq_factor); ordering, damping and the trailing update are
-library calls on the device."""
+with the tensors resident on the device.  The column loop of each block is one kernel launch (amct_gptq_block), the
+update of the columns behind it another (amct_gptq_trail), the factorisations one call (amct_gptq_factor)."""
 import math
 
 import torch
 
 from .. import _lib, ops
-from .utils import calculate_scale_offset, get_weight_min_max_by_granularity
+from .utils import check_scale_offset, get_weight_min_max_by_granularity
 
 
 @torch.no_grad()
@@ -84,20 +83,22 @@ def get_opt_weight_and_quant_factor(weight, hessian, quant_config, block_size=12
     bits = int(wts_type.replace('int', ''))
     columns = weight.shape[1]
     out_dtype = weight.dtype
+    if out_dtype not in (torch.float32, torch.float16, torch.bfloat16):
+        weight = weight.float()
     hessian = hessian.float()
     diag = torch.diag(hessian)
     dead = diag == 0
     diag = torch.where(dead, torch.ones_like(diag), diag)
-    weight = weight.float().masked_fill(dead, 0)
     perm = torch.argsort(diag, descending=True)
-    invperm = torch.argsort(perm)
-    weight_min, weight_max = get_weight_min_max_by_granularity(weight, quant_config)
-    scale_w, offset_w = calculate_scale_offset(weight_max, weight_min, cfg.get('symmetric'), wts_type)
-    ws = weight[:, perm].contiguous()
+    # the extrema of the weight with its dead columns at zero, in fp32 like the weight that the reference works on
+    weight_min, weight_max = get_weight_min_max_by_granularity(weight.masked_fill(dead, 0), quant_config)
+    # flags that the kernels raise, read when everything is enqueued: a factor not finite, a pivot not positive
+    bad = torch.zeros(2, dtype=torch.int32, device=weight.device)
+    scale_w, offset_w = ops.scale_offset(weight_max.float(), weight_min.float(), bits, bool(cfg.get('symmetric')), bad=bad[:1])
+    ws = ops.gptq_order(weight, perm, dead)
     # cholesky(cholesky_inverse(cholesky(hs)), upper=True) of the permuted, damped Hessian, as one factorisation
-    bad = torch.zeros(1, dtype=torch.int32, device=weight.device)
-    hinv = ops.gptq_factor(hessian, perm, perc_damp * torch.mean(diag), bad)
-    not_positive, factored = _read_later(bad)
+    hinv = ops.gptq_factor(hessian, perm, perc_damp * torch.mean(diag), bad[1:])
+    flags, factored = _read_later(bad)
     sc = scale_w.reshape(-1).float().contiguous()
     zc = None if offset_w is None else offset_w.reshape(-1).to(torch.int32).contiguous()
     if group_size:
@@ -109,9 +110,13 @@ def get_opt_weight_and_quant_factor(weight, hessian, quant_config, block_size=12
         i2 = min(i1 + block_size, columns)
         err_block = gptq_block(ws, i1, i2, hinv, sc, zc, gidx_all[i1:i2].contiguous(), qmin, qmax)
         if i2 < columns:
-            ws[:, i2:] -= err_block.matmul(hinv[i1:i2, i2:])
+            ops.gptq_trail(ws, err_block, hinv, i1, i2)
+    result = ops.gptq_order_back(ws, perm, weight.dtype).to(out_dtype)
     factored.synchronize()                          # of the copy only: long done when the last block is enqueued
-    if int(not_positive):
+    if int(flags[0]):
+        check_scale_offset(scale_w, None)
+        raise RuntimeError("Param offset has invalid value inf or nan!")
+    if int(flags[1]):
         raise torch.linalg.LinAlgError("linalg.cholesky: the factorization could not be completed because the input is "
                                        "not positive-definite.")
-    return ws[:, invperm].to(out_dtype), scale_w, offset_w
+    return result, scale_w, offset_w

@@ -361,10 +361,20 @@ int amct_gemm_w8a16_ws(const void* x, const void* smooth, const int8_t* wq, cons
  * (perm[i1 + i] / group_size for per-group factors, 0 otherwise).  w points at the block's first column inside
  * the column-sorted fp32 weight (row stride ld_w), hinv at the block's diagonal element (row stride ld_h);
  * err_out [rows, count] (row stride ld_e) feeds the reference's trailing update
- * weight[:, i2:] -= err_block @ hinv[i1:i2, i2:], which stays a library GEMM. */
+ * weight[:, i2:] -= err_block @ hinv[i1:i2, i2:] (amct_gptq_trail). */
 int amct_gptq_block(float* w, int64_t ld_w, float* err_out, int64_t ld_e, const float* hinv, int64_t ld_h,
                     const float* scale, const int32_t* offset, int64_t scale_stride, const int32_t* gidx,
                     int64_t rows, int count, int qmin, int qmax, amct_stream_t stream);
+
+/* w[rows, cols] -= err[rows, count] @ u[count, cols], all fp32: the products of an element are summed before the one
+ * subtraction.  Row strides ld_w, ld_e, ld_u in elements; w must not overlap err or u. */
+int amct_gptq_trail(float* w, int64_t ld_w, const float* err, int64_t ld_e, const float* u, int64_t ld_u, int64_t rows,
+                    int64_t cols, int count, amct_stream_t stream);
+/* Columns into the order of a permutation and back (amct_pytorch/quantize_op/gptq_module.py:122, :155), rows dense:
+ *   back = 0: out[r][c] (fp32) = dead[perm[c]] ? 0 : in[r][perm[c]] (dtype)       back = 1: out[r][perm[c]] (dtype) = in[r][c] (fp32)
+ * perm int64, a permutation of 0 .. cols - 1; dead one byte per column of `in` (read for back = 0 only). */
+int amct_gptq_order(const void* in, void* out, const int64_t* perm, const uint8_t* dead, int64_t rows, int64_t cols, int back,
+                    int dtype, amct_stream_t stream);
 
 /* ---- GPTQ factorisation -----------------------------------------------------------------------
  * The three factorisations of amct_pytorch/quantize_op/gptq_module.py:108-121 as one: with Hp = hessian[perm][:, perm],

@@ -42,3 +42,35 @@ def test_factor_of_an_indefinite_matrix_is_reported(dev):
     bad = torch.zeros(1, dtype=torch.int32, device=dev)
     ops.gptq_factor(h.to(dev), torch.arange(100, device=dev), torch.zeros((), device=dev), bad)
     assert int(bad) == 1
+
+
+# one tile, the edges of the 128 x 64 tiles and of the 32 steps, rows that are not 16-byte aligned, a short block
+@pytest.mark.parametrize("rows,cols,i1,i2", [(1, 132, 0, 128), (128, 192, 0, 128), (129, 320, 128, 256), (127, 193, 3, 128),
+                                             (260, 300, 0, 33), (64, 8, 0, 4), (1000, 1411, 1280, 1408), (3, 129, 0, 128)])
+def test_trailing_update(dev, rows, cols, i1, i2):
+    g = torch.Generator().manual_seed(rows + cols)
+    w, e, u = torch.randn(rows, cols, generator=g), torch.randn(rows, i2 - i1, generator=g), torch.randn(cols, cols, generator=g)
+    got = w.to(dev)
+    ops.gptq_trail(got, e.to(dev), u.to(dev), i1, i2)
+    got = got.cpu()
+    assert torch.equal(got[:, :i2], w[:, :i2]), "columns in front of the trailing part stay"
+    prod = e.double() @ u[i1:i2, i2:].double()
+    want = w[:, i2:].double() - prod
+    # a sum of n products in any order is within n u sum|e||u| (u = 2^-24), the subtraction adds half a unit of its result
+    bound = ((i2 - i1 + 1) * 2.0 ** -24) * (e.abs().double() @ u[i1:i2, i2:].abs().double()) + 2.0 ** -24 * want.abs() + 1e-30
+    assert bool(((got[:, i2:].double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (4, 100), (5, 4096), (7, 4097), (2, 9001)])
+def test_column_order_and_back(dev, dtype, rows, cols):
+    g = torch.Generator().manual_seed(cols)
+    w = torch.randn(rows, cols, generator=g).to(dtype)
+    perm, dead = torch.randperm(cols, generator=g), torch.rand(cols, generator=g) < 0.1
+    ws = ops.gptq_order(w.to(dev), perm.to(dev), dead.to(dev))
+    assert torch.equal(ws.cpu(), w.float().masked_fill(dead, 0)[:, perm])
+    back = ops.gptq_order_back(ws, perm.to(dev), dtype)
+    assert torch.equal(back.cpu(), w.masked_fill(dead, 0))
+    values = torch.randn(rows, cols, generator=g)                  # rounded on the way back
+    got = ops.gptq_order_back(values.to(dev), perm.to(dev), dtype).cpu()
+    assert torch.equal(got, values[:, torch.argsort(perm)].to(dtype))
