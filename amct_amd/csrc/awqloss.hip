@@ -5,6 +5,8 @@
 // d^4 is (d*d)*(d*d) in fp32.  The sum is deterministic: a fixed number of blocks, each a fixed partition of the
 // elements, per-block partials folded in a fixed order by one block (pass 2), which also divides by n.
 // The order of summation differs from torch's, so results agree to fp32 rounding of the sum, not bit for bit.
+#include <algorithm>
+
 #include "amct_common.h"
 
 namespace amct {
@@ -95,9 +97,124 @@ __global__ __launch_bounds__(kBlock) void awq_loss_final_k(const float* partial,
     }
 }
 
+// All candidate scales of a search in one launch, a thread block per grid point (amct_pytorch/algorithm/awq.py:85-88):
+// mean ** ratio rounded to the activations' dtype and clamped at 1e-4, divided in fp64 by the geometric mean of its extremes,
+// rounded to the dtype and clamped into [1e-4, largest finite].  As thirteen library launches per grid point these took
+// longer than the fake-quantised weight they are for.  The powers are kept in the output between the two passes.
+template <int DT> AMCT_DEV float dtype_max() { return DT == AMCT_F16 ? 65504.f : DT == AMCT_BF16 ? 3.38953138925153547590e38f : 3.40282346638528859812e38f; }
+// torch.clamp of a value of the dtype: NaN stays NaN, the bound is rounded to the dtype
+template <int DT> AMCT_DEV float clamp_low(float v) {
+    const float lo = round_to<DT>(1e-4f);
+    return v < lo ? lo : v;
+}
+
+template <int DT>
+__global__ __launch_bounds__(kBlock) void awq_candidates_k(const void* mean, const float* ratios, void* out, int64_t cols) {
+    __shared__ float smx[kBlock / 64], smn[kBlock / 64];
+    const int tid = threadIdx.x;
+    const float ratio = ratios[blockIdx.x];
+    const int64_t base = (int64_t)blockIdx.x * cols;
+    float mx = -__builtin_inff(), mn = __builtin_inff();
+    for (int64_t c = tid; c < cols; c += kBlock) {
+        const float x = load_scalar<DT>(mean, c);
+        // the square root and the zeroth power as such, as the library's power does
+        const float p = ratio == 0.5f ? sqrtf(x) : ratio == 0.f ? 1.f : powf(x, ratio);
+        const float v = clamp_low<DT>(round_to<DT>(p));
+        store_scalar<DT>(out, base + c, v);
+        mx = fmax_nan(mx, v);
+        mn = fmin_nan(mn, v);
+    }
+    team_minmax<64>(mn, mx);
+    if ((tid & 63) == 0) {
+        smx[tid >> 6] = mx;
+        smn[tid >> 6] = mn;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kBlock / 64; ++w) {
+        mx = fmax_nan(mx, smx[w]);
+        mn = fmin_nan(mn, smn[w]);
+    }
+    const double norm = sqrt((double)mx * (double)mn);
+    for (int64_t c = tid; c < cols; c += kBlock) {                 // a thread reads back what it wrote
+        const double q = (double)load_scalar<DT>(out, base + c) / norm;
+        const float v = clamp_low<DT>(round_to<DT>((float)q));
+        store_scalar<DT>(out, base + c, v > dtype_max<DT>() ? dtype_max<DT>() : v);
+    }
+}
+
+// The losses of a search from the partials of its grid points (kLossBlocks apart), folded as awq_loss_final_k folds them,
+// and the first grid point whose loss is below infinity and below every earlier one: -1 if there is none.
+__global__ __launch_bounds__(kBlock) void awq_pick_k(const float* partials, int nparts, int64_t n, int grids, float* losses, int32_t* winner) {
+    __shared__ float red[kBlock / 64];
+    const int tid = threadIdx.x;
+    float best = __builtin_inff();
+    int at = -1;
+    for (int g = 0; g < grids; ++g) {
+        float t = 0.f;
+        for (int i = tid; i < nparts; i += kBlock) t = t + partials[(int64_t)g * kLossBlocks + i];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) t = t + __shfl_xor(t, off, 64);
+        if (g) __syncthreads();
+        if ((tid & 63) == 0) red[tid >> 6] = t;
+        __syncthreads();
+        if (tid == 0) {
+            float b = red[0];
+#pragma unroll
+            for (int w = 1; w < kBlock / 64; ++w) b = b + red[w];
+            b = b / (float)n;
+            losses[g] = b;
+            if (b < best) {                          // false for NaN
+                best = b;
+                at = g;
+            }
+        }
+    }
+    if (tid == 0) *winner = at;
+}
+
+// *flag = 1 where x holds an infinity or a NaN: the check in front of a search, one pass where isfinite().all() makes five
+template <int DT>
+__global__ __launch_bounds__(kBlock) void nonfinite_k(const void* x, int64_t n, int vec_ok, int32_t* flag) {
+    constexpr int VEC = Tr<DT>::VEC;
+    bool bad = false;
+    const int64_t nvec = vec_ok ? n / VEC : 0, stride = (int64_t)gridDim.x * kBlock;
+    for (int64_t v0 = (int64_t)blockIdx.x * kBlock + threadIdx.x; v0 < nvec; v0 += stride * kLossUnroll) {
+        uint4 raw[kLossUnroll];
+#pragma unroll
+        for (int u = 0; u < kLossUnroll; ++u) {
+            const int64_t v = v0 + u * stride;
+            raw[u] = ldg16(reinterpret_cast<const char*>(x) + (v < nvec ? v : nvec - 1) * 16);
+        }
+#pragma unroll
+        for (int u = 0; u < kLossUnroll; ++u) {
+            float f[VEC];
+            unpack16<DT>(raw[u], f);
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) bad = bad || !finite_f(f[j]);
+        }
+    }
+    for (int64_t i = nvec * VEC + (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += stride) bad = bad || !finite_f(load_scalar<DT>(x, i));
+    if (bad) *flag = 1;
+}
+
 }  // namespace amct
 
 using namespace amct;
+
+static int loss_blocks(int64_t n, int dtype) {
+    const int vec = dtype == AMCT_F32 ? 4 : 8;
+    const int64_t blocks = (n / vec + (int64_t)kBlock * kLossUnroll - 1) / ((int64_t)kBlock * kLossUnroll);
+    return (int)std::min<int64_t>(std::max<int64_t>(blocks, 1), kLossBlocks);
+}
+
+// n == 0: the mean of nothing is 0 / 0 = NaN, as torch's; this pass then writes zeros
+static void loss_partials(const void* y, const void* yhat, int64_t n, int dtype, int blocks, float* partial, hipStream_t st) {
+    const dim3 grid((unsigned)blocks);
+    if (dtype == AMCT_F32) hipLaunchKernelGGL((awq_loss_partial_k<AMCT_F32>), grid, dim3(kBlock), 0, st, y, yhat, n, partial);
+    else if (dtype == AMCT_F16) hipLaunchKernelGGL((awq_loss_partial_k<AMCT_F16>), grid, dim3(kBlock), 0, st, y, yhat, n, partial);
+    else hipLaunchKernelGGL((awq_loss_partial_k<AMCT_BF16>), grid, dim3(kBlock), 0, st, y, yhat, n, partial);
+}
 
 extern "C" size_t amct_awq_loss_workspace_bytes(void) { return (size_t)kLossBlocks * sizeof(float); }
 
@@ -108,16 +225,58 @@ extern "C" int amct_awq_loss(const void* y, const void* yhat, int64_t n, int dty
     if (n != 0 && (!y || !yhat)) return AMCT_E_BADARG;
     if (!workspace || workspace_bytes < amct_awq_loss_workspace_bytes() || ((uintptr_t)workspace & 3)) return AMCT_E_BADARG;
     if (n != 0 && (!aligned16(y) || !aligned16(yhat))) return AMCT_E_ALIGN;
-    hipStream_t st = (hipStream_t)stream;
     float* partial = reinterpret_cast<float*>(workspace);
-    // n == 0: the mean of nothing is 0 / 0 = NaN, as torch's; the partial pass then writes zeros
+    const int blocks = loss_blocks(n, dtype);
+    loss_partials(y, yhat, n, dtype, blocks, partial, (hipStream_t)stream);
+    hipLaunchKernelGGL(awq_loss_final_k, dim3(1), dim3(kBlock), 0, (hipStream_t)stream, partial, blocks, n, loss);
+    return hip_status();
+}
+
+static bool loss_args_ok(int64_t n, int dtype) { return n >= 0 && (dtype == AMCT_F32 || dtype == AMCT_F16 || dtype == AMCT_BF16); }
+
+extern "C" int amct_awq_loss_partials(const void* y, const void* yhat, int64_t n, int dtype, float* partials, amct_stream_t stream) {
+    if (!loss_args_ok(n, dtype) || !partials || (n != 0 && (!y || !yhat))) return AMCT_E_BADARG;
+    if (n != 0 && (!aligned16(y) || !aligned16(yhat))) return AMCT_E_ALIGN;
+    loss_partials(y, yhat, n, dtype, loss_blocks(n, dtype), partials, (hipStream_t)stream);
+    return hip_status();
+}
+
+extern "C" int amct_awq_pick(const float* partials, int64_t n, int dtype, int grids, float* losses, int32_t* winner, amct_stream_t stream) {
+    if (!loss_args_ok(n, dtype) || grids <= 0 || !partials || !losses || !winner) return AMCT_E_BADARG;
+    hipLaunchKernelGGL(awq_pick_k, dim3(1), dim3(kBlock), 0, (hipStream_t)stream, partials, loss_blocks(n, dtype), n, grids, losses, winner);
+    return hip_status();
+}
+
+extern "C" int amct_awq_candidates(const void* mean, const float* ratios, void* out, int grids, int64_t cols, int dtype,
+                                   amct_stream_t stream) {
+    if (grids < 0 || cols < 0) return AMCT_E_BADARG;
+    if (grids == 0 || cols == 0) return AMCT_OK;
+    if (!mean || !ratios || !out) return AMCT_E_BADARG;
+    const dim3 grid((unsigned)grids);
+    hipStream_t st = (hipStream_t)stream;
+    switch (dtype) {
+        case AMCT_F32: hipLaunchKernelGGL((awq_candidates_k<AMCT_F32>), grid, dim3(kBlock), 0, st, mean, ratios, out, cols); break;
+        case AMCT_F16: hipLaunchKernelGGL((awq_candidates_k<AMCT_F16>), grid, dim3(kBlock), 0, st, mean, ratios, out, cols); break;
+        case AMCT_BF16: hipLaunchKernelGGL((awq_candidates_k<AMCT_BF16>), grid, dim3(kBlock), 0, st, mean, ratios, out, cols); break;
+        default: return AMCT_E_BADARG;
+    }
+    return hip_status();
+}
+
+extern "C" int amct_flag_nonfinite(const void* x, int64_t n, int dtype, int32_t* flag, amct_stream_t stream) {
+    if (n < 0 || !flag) return AMCT_E_BADARG;
+    if (n == 0) return AMCT_OK;
+    if (!x) return AMCT_E_BADARG;
     const int vec = dtype == AMCT_F32 ? 4 : 8;
-    int64_t blocks = (n / vec + (int64_t)kBlock * kLossUnroll - 1) / ((int64_t)kBlock * kLossUnroll);
-    if (blocks < 1) blocks = 1;
-    if (blocks > kLossBlocks) blocks = kLossBlocks;
-    if (dtype == AMCT_F32) hipLaunchKernelGGL((awq_loss_partial_k<AMCT_F32>), dim3((unsigned)blocks), dim3(kBlock), 0, st, y, yhat, n, partial);
-    else if (dtype == AMCT_F16) hipLaunchKernelGGL((awq_loss_partial_k<AMCT_F16>), dim3((unsigned)blocks), dim3(kBlock), 0, st, y, yhat, n, partial);
-    else hipLaunchKernelGGL((awq_loss_partial_k<AMCT_BF16>), dim3((unsigned)blocks), dim3(kBlock), 0, st, y, yhat, n, partial);
-    hipLaunchKernelGGL(awq_loss_final_k, dim3(1), dim3(kBlock), 0, st, partial, (int)blocks, n, loss);
+    const int64_t per = (int64_t)kBlock * kLossUnroll * vec;
+    const dim3 grid((unsigned)std::min<int64_t>((n + per - 1) / per, 2048));
+    const int vec_ok = aligned16(x);
+    hipStream_t st = (hipStream_t)stream;
+    switch (dtype) {
+        case AMCT_F32: hipLaunchKernelGGL((nonfinite_k<AMCT_F32>), grid, dim3(kBlock), 0, st, x, n, vec_ok, flag); break;
+        case AMCT_F16: hipLaunchKernelGGL((nonfinite_k<AMCT_F16>), grid, dim3(kBlock), 0, st, x, n, vec_ok, flag); break;
+        case AMCT_BF16: hipLaunchKernelGGL((nonfinite_k<AMCT_BF16>), grid, dim3(kBlock), 0, st, x, n, vec_ok, flag); break;
+        default: return AMCT_E_BADARG;
+    }
     return hip_status();
 }

@@ -48,6 +48,35 @@ template <int DT> AMCT_DEV void apply_col_pre(float* x, const float* c, int mode
     }
 }
 
+// d[j] <- round_to<DT>(d[j]) / c[j].  FAST: every |d[j]| is 0 or in [2^-60, 2^70).  Two 16-bit numbers have a quotient that is
+// either an fp32 number or further than 2^-36 (relative) from every rounding boundary of fp32, so the hardware reciprocal
+// (1 unit) with one correction by the exact remainder (relative error 2^-44 before its rounding) gives the bits of the IEEE
+// division in 5 instructions; column scales outside [2^-30, 2^30) and fp32 tensors divide.
+template <int DT, bool FAST> AMCT_DEV void divide_cols(float* d, const float* c) {
+    constexpr int VEC = Tr<DT>::VEC;
+    if constexpr (FAST && DT != AMCT_F32) {
+        uint32_t lo = __float_as_uint(c[0]), hi = lo;       // (a negative scale is large as an unsigned number)
+#pragma unroll
+        for (int j = 1; j < VEC; ++j) {
+            lo = min(lo, __float_as_uint(c[j]));
+            hi = max(hi, __float_as_uint(c[j]));
+        }
+        if (wave_all(lo >= (97u << 23) && hi < (157u << 23))) {
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) {
+                const float n = round_to<DT>(d[j]);
+                const float y = __builtin_amdgcn_rcpf(c[j]);
+                const float q0 = n * y;
+                const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, c[j], n), y, q0);
+                d[j] = __uint_as_float((__float_as_uint(q1) & 0x7FFFFFFFu) | (__float_as_uint(n) & 0x80000000u));
+            }
+            return;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) d[j] = round_to<DT>(d[j]) / c[j];
+}
+
 // Params path: the whole quantiser or one of the two halves the AWQ search calls separately.
 //   FULL    : q = clamp(rne(x/s + z)); d = (q - z) * s
 //   SCALE   : d = x/s + z                      (do_quant, amct_pytorch/algorithm/awq.py:129-149)
@@ -128,18 +157,40 @@ __global__ __launch_bounds__(kBlock) void fq_fused(FqArgs a) {
 #pragma unroll
             for (int i = 0; i < NV; ++i) unpack16<DT>(raw[u][i], x[u][i]);
     }
+    // first column of each segment: one remainder per team, in 32 bits where the segment count allows it.  All the column
+    // factors are asked for together and, where they fit (kKeepCol), stay in registers for the division at the end: fetched
+    // vector by vector, twice, they this kernel waited for each (W[4096,4096] bf16 in groups of 128: 25.9 us, now 21.8, bound by its instructions)
+    int64_t col0[U];
+    uint4 craw[COL ? U : 1][COL ? NV : 1];
+    constexpr bool kKeepCol = U * NV <= 8;
     if constexpr (COL) {
+        const uint32_t spr = (uint32_t)a.segs_per_row;
+        uint32_t sg = a.nseg <= 0xFFFFFFFFll ? (uint32_t)segc[0] % spr : (uint32_t)(segc[0] % spr);
+        col0[0] = (int64_t)sg * a.seg_len;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int64_t c0 = (segc[u] % a.segs_per_row) * (int64_t)a.seg_len;
+        for (int u = 1; u < U; ++u) {
+            if (segc[u] != segc[u - 1]) sg = sg + 1 == spr ? 0 : sg + 1;
+            col0[u] = (int64_t)sg * a.seg_len;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
 #pragma unroll
             for (int i = 0; i < NV; ++i) {
                 const int v = (i * T + lt < S) ? i * T + lt : S - 1;
-                float c[VEC];
-                unpack16<DT>(ldg16(reinterpret_cast<const char*>(a.col) + (c0 + (int64_t)v * VEC) * BYTES), c);
-                apply_col_pre<DT>(x[u][i], c, a.col_mode);
+                craw[u][i] = ldg16(reinterpret_cast<const char*>(a.col) + (col0[u] + (int64_t)v * VEC) * BYTES);
             }
-        }
+        auto pre = [&](int mode) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int i = 0; i < NV; ++i) {
+                    float c[VEC];
+                    unpack16<DT>(craw[u][i], c);
+                    apply_col_pre<DT>(x[u][i], c, mode);
+                }
+        };
+        if (a.col_mode == AMCT_COL_DIV) pre(AMCT_COL_DIV);
+        else pre(AMCT_COL_MUL);
     }
 
     float mx[U], mn[U];
@@ -224,7 +275,6 @@ __global__ __launch_bounds__(kBlock) void fq_fused(FqArgs a) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const bool ok = seg0 + u < a.nseg;
-            const int64_t c0 = (COL && a.col_mode == AMCT_COL_MUL_THEN_DIV) ? (segc[u] % a.segs_per_row) * (int64_t)a.seg_len : 0;
 #pragma unroll
             for (int i = 0; i < NV; ++i) {
                 const int v = i * T + lt;
@@ -241,9 +291,8 @@ __global__ __launch_bounds__(kBlock) void fq_fused(FqArgs a) {
                         if constexpr (COL) {
                             if (a.col_mode == AMCT_COL_MUL_THEN_DIV) {
                                 float c[VEC];
-                                unpack16<DT>(ldg16(reinterpret_cast<const char*>(a.col) + (c0 + (int64_t)v * VEC) * BYTES), c);
-#pragma unroll
-                                for (int j = 0; j < VEC; ++j) d[j] = round_to<DT>(d[j]) / c[j];
+                                unpack16<DT>(kKeepCol ? craw[u][i] : ldg16(reinterpret_cast<const char*>(a.col) + (col0[u] + (int64_t)v * VEC) * BYTES), c);
+                                divide_cols<DT, FAST>(d, c);
                             }
                         }
                         stg16_nt(reinterpret_cast<char*>(a.dq) + e0 * BYTES, pack16<DT>(d));

@@ -171,6 +171,62 @@ def awq_loss(y, yhat):
     return loss
 
 
+def awq_candidates(mean, ratios):
+    """The scales of all grid points of an AWQ search, [len(ratios), K] in mean's dtype (algorithm/awq.py:85-88)."""
+    dev = _dev(mean)
+    mean = _c(mean)
+    # a power with a Python exponent takes it in the tensor's dtype
+    exponents = torch.tensor(ratios, dtype=mean.dtype).float().to(dev)
+    out = torch.empty(len(ratios), mean.numel(), dtype=mean.dtype, device=dev)
+    with _on(dev):
+        _lib.check(_lib.load().amct_awq_candidates(_p(mean), _p(exponents), _p(out), len(ratios), mean.numel(),
+                                                   dtype_code(mean.dtype), _stream(dev)))
+    return out
+
+
+class AwqLosses:
+    """mean((y - yhat)^4) of every grid point of a search against one target, nothing read back until winner()."""
+
+    def __init__(self, target, grids):
+        self.target, self.grids = _c(target), grids
+        self._lib = _lib.load()
+        self._stride = self._lib.amct_awq_loss_workspace_bytes() // 4
+        self._partials = torch.empty(max(grids, 1), self._stride, dtype=torch.float32, device=_dev(target))
+
+    def add(self, grid, yhat):
+        y = self.target
+        dev = _dev(y, yhat)
+        if y.dtype != yhat.dtype or y.shape != yhat.shape:
+            raise RuntimeError("awq_loss: the two outputs must share dtype and shape")
+        yhat = _c(yhat)
+        with _on(dev):
+            _lib.check(self._lib.amct_awq_loss_partials(_p(y), _p(yhat), y.numel(), dtype_code(y.dtype),
+                                                        self._partials.data_ptr() + 4 * self._stride * grid, _stream(dev)))
+
+    def winner(self):
+        """Index of the first smallest loss below infinity, or -1 (waits for the device)."""
+        if self.grids == 0:
+            return -1
+        dev = self.target.device
+        losses = torch.empty(self.grids, dtype=torch.float32, device=dev)
+        at = torch.empty(1, dtype=torch.int32, device=dev)
+        with _on(dev):
+            _lib.check(self._lib.amct_awq_pick(_p(self._partials), self.target.numel(), dtype_code(self.target.dtype), self.grids,
+                                               _p(losses), _p(at), _stream(dev)))
+        return int(at)
+
+
+def nonfinite_flags(tensors):
+    """One truth value per tensor: whether it holds an infinity or a NaN (one read-back for all of them)."""
+    dev = _dev(*tensors)
+    flags = torch.zeros(len(tensors), dtype=torch.int32, device=dev)
+    with _on(dev):
+        for i, t in enumerate(tensors):
+            t = _c(t)
+            _lib.check(_lib.load().amct_flag_nonfinite(_p(t), t.numel(), dtype_code(t.dtype), flags.data_ptr() + 4 * i, _stream(dev)))
+    return [bool(f) for f in flags.tolist()]
+
+
 def hessian_update(hessian, x, beta, alpha):
     """hessian [C,C] fp32 <- beta * hessian + alpha * x^T x in place, x [tokens, C] bf16|f16 (gptq_module.py:176-181).
     beta == 0 does not read hessian."""

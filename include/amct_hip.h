@@ -125,6 +125,18 @@ int amct_col_minmax_noalloc(const void* x, float* col_max, float* col_min, int64
 size_t amct_awq_loss_workspace_bytes(void);
 int amct_awq_loss(const void* y, const void* yhat, int64_t n, int dtype, float* loss, void* workspace,
                   size_t workspace_bytes, amct_stream_t stream);
+/* The pieces of a whole AWQ scale search (amct_pytorch/algorithm/awq.py:84-103) with nothing read back between its grid points.
+ * amct_awq_candidates: out [grids, cols] = the scale of every ratio (fp32 [grids] on the device) from the mean magnitude per
+ *   channel; mean and out in dtype.
+ * amct_awq_loss_partials: the first pass of amct_awq_loss, into amct_awq_loss_workspace_bytes() bytes of partials; the next
+ *   grid point's follow directly behind.
+ * amct_awq_pick: from grids of those (same n and dtype) losses [grids] fp32 and *winner (int32), the first grid point with the
+ *   smallest loss below infinity, -1 if every loss is infinite or NaN.
+ * amct_flag_nonfinite: *flag (int32 on the device) becomes 1 if x [n] holds an infinity or a NaN, and stays as it is if not. */
+int amct_awq_candidates(const void* mean, const float* ratios, void* out, int grids, int64_t cols, int dtype, amct_stream_t stream);
+int amct_awq_loss_partials(const void* y, const void* yhat, int64_t n, int dtype, float* partials, amct_stream_t stream);
+int amct_awq_pick(const float* partials, int64_t n, int dtype, int grids, float* losses, int32_t* winner, amct_stream_t stream);
+int amct_flag_nonfinite(const void* x, int64_t n, int dtype, int32_t* flag, amct_stream_t stream);
 
 /* ---- A1: min / max per row (group = 0) or per group of `group` columns ----------------
  * Replaces get_weight_min_max_by_granularity (amct_pytorch/quantize_op/utils.py:111-136)

@@ -465,3 +465,39 @@ def test_calculate_scale_offset_without_the_synchronising_check(dev):
     assert z is None and s[0, 0].item() == torch.tensor(1.27).div(127).item() and torch.isinf(s[1, 0])
     with pytest.raises(RuntimeError, match="Param scale has invalid value"):
         qutils.check_scale_offset(s, None)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("k,grids", [(1, 1), (300, 8), (4096, 20)])
+def test_awq_candidates_are_the_scales_of_every_ratio(dev, dtype, k, grids):
+    g = torch.Generator().manual_seed(k)
+    mean = (torch.rand(k, generator=g) * 3).to(dtype).to(dev)
+    mean[k // 2] = 0
+    got = ops.awq_candidates(mean, [i / grids for i in range(grids)])
+    for i in range(grids):
+        want = awq.awq_scale_for_ratio(mean, i / grids, dtype)
+        # the same power, extremes and division; a unit of the dtype is what two powers may differ by
+        unit = torch.finfo(dtype).eps
+        assert float(((got[i:i + 1] - want).float().abs() / want.float()).max()) <= unit
+
+
+def test_awq_pick_and_nonfinite_flags(dev):
+    n = 5000
+    y = torch.randn(n, device=dev)
+    outs = [y + 1, y + 0.5, y * float('nan'), y + 0.25, y.clone().fill_(float('inf')), y + 0.25]
+    losses = ops.AwqLosses(y, len(outs))
+    for i, o in enumerate(outs):
+        losses.add(i, o)
+    assert losses.winner() == 3, "the first of the smallest, NaN and infinity never"
+    only = ops.AwqLosses(y, 2)
+    for i in range(2):
+        only.add(i, outs[2])
+    assert only.winner() == -1
+    for dtype in (torch.float32, torch.float16, torch.bfloat16):
+        for size in (1, 7, 4099, 100001):
+            x = torch.ones(size, device=dev, dtype=dtype)
+            z = x.clone()
+            z[size - 1] = float('-inf')
+            a = x.clone()
+            a[0] = float('nan')
+            assert ops.nonfinite_flags([x, z, a, torch.ones(size + 1, device=dev, dtype=dtype)[1:]]) == [False, True, True, False]

@@ -287,3 +287,22 @@ def test_fakequant_matches_exact_arithmetic_fixture(dev):
             assert int(got_z.cpu().reshape(())) == offset
         assert torch.equal(got_codes.cpu(), codes)
         assert_bits_equal(got_dq.cpu(), dq, "dq int%d sym=%s" % (bits, sym))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,cols,group", [(1, 32, 32), (3, 96, 32), (5, 640, 128), (67, 384, 64), (9, 1536, 0), (2, 8200, 0)])
+@pytest.mark.parametrize("wide", [False, True])
+def test_column_scaled_fake_quant_of_any_shape(dev, dtype, rows, cols, group, wide):
+    """W * c -> fake-quant -> / c: every segment meets its own columns' factors (segments of a team across the ends of
+    rows), and factors beyond the range of the reciprocal division are divided by."""
+    g = torch.Generator().manual_seed(rows * cols)
+    w = (torch.randn(rows, cols, generator=g) * 0.05).to(dtype)
+    w[0, 0] = -0.0
+    c = (0.5 + torch.rand(1, cols, generator=g))
+    if wide:
+        c = c * torch.where(torch.rand(1, cols, generator=g) < 0.01, 2.0 ** 35 if dtype != torch.float16 else 2.0 ** 9, 1.0)
+    c = c.to(dtype)
+    strategy = 'group' if group else 'channel'
+    want = iq.awq_grid_step(w, c, 'int4', strategy, False, group or None)[0]
+    got, _, _, _ = ops.fakequant_int(w.to(dev), 4, False, group=group, col_scale=c.to(dev), col_mode=ops.COL_MUL_THEN_DIV, via_src=True)
+    assert_bits_equal(got, want, "awq grid step")
