@@ -12,7 +12,8 @@
 // swizzled by the row so that fragment reads spread over the banks; the next step waits in registers), two barriers
 // per step.  The epilogue reads the
 // tile of H, applies beta and alpha, writes the tile and -- through LDS, as whole 256-byte rows -- its mirror image, so H
-// stays exactly symmetric and only its lower triangle is ever read.
+// stays exactly symmetric and only its lower triangle is ever read.  It also notes whether everything it wrote is finite:
+// as five library passes over H that check took as long as the update itself (75 us at 4096 columns).
 #include "amct_common.h"
 
 namespace amct {
@@ -25,10 +26,11 @@ constexpr int kHsTile = 128;                         // rows / columns of H per 
 constexpr int kHsK = 64;                             // tokens per step (128 bytes of a row of X^T)
 
 // X [T, C] -> Xt [Cp, Tp], zeros beyond T and C.  64 x 64 tiles through LDS.
-__global__ __launch_bounds__(kBlock) void hess_transpose_k(const uint16_t* x, uint16_t* xt, int64_t T, int64_t C, int64_t Tp) {
+__global__ __launch_bounds__(kBlock) void hess_transpose_k(const uint16_t* x, uint16_t* xt, int64_t T, int64_t C, int64_t Tp, int32_t* bad) {
     __shared__ uint16_t tile[64][66];
     const int tid = threadIdx.x;
     const int64_t c0 = (int64_t)blockIdx.x * 64, t0 = (int64_t)blockIdx.y * 64;
+    if (bad && blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) *bad = 0;      // before the kernel that may set it
     {
         const int c = tid & 63;
 #pragma unroll
@@ -53,10 +55,11 @@ __global__ __launch_bounds__(kBlock) void hess_transpose_k(const uint16_t* x, ui
 // The same for C % 8 == 0 and a 16-byte aligned x: 16-byte loads (8 columns of one token) and 16-byte stores (8
 // tokens of one column); the tile is held column-major, a column 72 tokens apart (144 bytes: 16-byte aligned rows whose
 // 16-byte reads by 8 lanes of consecutive columns fall into different banks).
-__global__ __launch_bounds__(kBlock) void hess_transpose_vec_k(const uint16_t* x, uint16_t* xt, int64_t T, int64_t C, int64_t Tp) {
+__global__ __launch_bounds__(kBlock) void hess_transpose_vec_k(const uint16_t* x, uint16_t* xt, int64_t T, int64_t C, int64_t Tp, int32_t* bad) {
     __shared__ __align__(16) uint16_t tile[64][72];                           // [column][token]
     const int tid = threadIdx.x;
     const int64_t c0 = (int64_t)blockIdx.x * 64, t0 = (int64_t)blockIdx.y * 64;
+    if (bad && blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) *bad = 0;      // before the kernel that may set it
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int v = tid + 256 * i;                                          // 512 vectors: token v / 8, columns 8 (v % 8) ..
@@ -88,6 +91,7 @@ struct SyrkArgs {
     int per_die;                                     // tiles of the lower triangle per die (rounded up)
     int64_t ntiles;                                  // nb (nb + 1) / 2
     float beta, alpha;
+    int32_t* bad;                                    // set where an element of the new H is not finite, or null
 };
 
 template <bool F16>
@@ -230,6 +234,7 @@ __global__ __launch_bounds__(kBlock, 3) void hess_syrk_k(SyrkArgs a) {
     float* hm = a.h + wj0 * a.C + wi0;                                        // its mirror image H[wj0][wi0]
     const int rows_left = (int)min((int64_t)64, a.C - wi0), cols_left = (int)min((int64_t)64, a.C - wj0);   // may be <= 0
     const uint32_t lane_off = (uint32_t)(4 * fh) * C32 + (uint32_t)fr;
+    bool finite = true;                              // of everything this lane writes (the mirror image repeats it)
 #pragma unroll
     for (int n = 0; n < 2; ++n) {                    // the wave's columns 32 n .. 32 n + 31
         const bool col_ok = n * 32 + fr < cols_left;
@@ -253,7 +258,10 @@ __global__ __launch_bounds__(kBlock, 3) void hess_syrk_k(SyrkArgs a) {
                 const uint32_t idx = lane_off + (uint32_t)row * C32 + (uint32_t)(n * 32);
                 float v = a.alpha * acc[m][n][r];
                 if (have) v = old[m][r] * a.beta + v;
-                if (col_ok && lr < rows_left) hw[idx] = v;
+                if (col_ok && lr < rows_left) {
+                    hw[idx] = v;
+                    finite = finite && finite_f(v);
+                }
                 patch[lr * 32 + (fr ^ (lr & 31))] = v;
             }
         }
@@ -267,6 +275,7 @@ __global__ __launch_bounds__(kBlock, 3) void hess_syrk_k(SyrkArgs a) {
             if (lr < rows_left && n * 32 + lc < cols_left) hm[(uint32_t)(n * 32 + lc) * C32 + (uint32_t)lr] = v;
         }
     }
+    if (a.bad && !finite) *a.bad = 1;
 }
 
 }  // namespace amct
@@ -282,6 +291,11 @@ extern "C" size_t amct_hessian_update_workspace_bytes(int64_t tokens, int64_t co
 
 extern "C" int amct_hessian_update(float* hessian, const void* x, int64_t tokens, int64_t cols, float beta, float alpha,
                                    int dtype, void* workspace, size_t workspace_bytes, amct_stream_t stream) {
+    return amct_hessian_update_checked(hessian, x, tokens, cols, beta, alpha, dtype, nullptr, workspace, workspace_bytes, stream);
+}
+
+extern "C" int amct_hessian_update_checked(float* hessian, const void* x, int64_t tokens, int64_t cols, float beta, float alpha,
+                                           int dtype, int32_t* bad, void* workspace, size_t workspace_bytes, amct_stream_t stream) {
     if (tokens < 0 || cols <= 0 || !hessian) return AMCT_E_BADARG;
     if (dtype != AMCT_BF16 && dtype != AMCT_F16) return AMCT_E_UNSUPPORTED;
     if (tokens != 0 && !x) return AMCT_E_BADARG;
@@ -294,12 +308,12 @@ extern "C" int amct_hessian_update(float* hessian, const void* x, int64_t tokens
     hipStream_t st = (hipStream_t)stream;
     if (cols % 8 == 0 && aligned16(x))
         hipLaunchKernelGGL(hess_transpose_vec_k, dim3((unsigned)(Cp / 64), (unsigned)(Tp / 64)), dim3(kBlock), 0, st,
-                           reinterpret_cast<const uint16_t*>(x), reinterpret_cast<uint16_t*>(workspace), tokens, cols, Tp);
+                           reinterpret_cast<const uint16_t*>(x), reinterpret_cast<uint16_t*>(workspace), tokens, cols, Tp, bad);
     else
         hipLaunchKernelGGL(hess_transpose_k, dim3((unsigned)(Cp / 64), (unsigned)(Tp / 64)), dim3(kBlock), 0, st,
-                           reinterpret_cast<const uint16_t*>(x), reinterpret_cast<uint16_t*>(workspace), tokens, cols, Tp);
+                           reinterpret_cast<const uint16_t*>(x), reinterpret_cast<uint16_t*>(workspace), tokens, cols, Tp, bad);
     const int64_t ntiles = nb * (nb + 1) / 2, per_die = (ntiles + 7) / 8;
-    SyrkArgs a{reinterpret_cast<const uint16_t*>(workspace), hessian, cols, Tp, (int)nb, (int)per_die, ntiles, beta, alpha};
+    SyrkArgs a{reinterpret_cast<const uint16_t*>(workspace), hessian, cols, Tp, (int)nb, (int)per_die, ntiles, beta, alpha, bad};
     constexpr size_t lds_bytes = 2 * kHsTile * 128;                           // 32 KB
     const dim3 grid((unsigned)(8 * per_die));
     if (dtype == AMCT_F16) hipLaunchKernelGGL((hess_syrk_k<true>), grid, dim3(kBlock), lds_bytes, st, a);

@@ -227,10 +227,11 @@ def nonfinite_flags(tensors):
     return [bool(f) for f in flags.tolist()]
 
 
-def hessian_update(hessian, x, beta, alpha):
+def hessian_update(hessian, x, beta, alpha, bad=None):
     """hessian [C,C] fp32 <- beta * hessian + alpha * x^T x in place, x [tokens, C] bf16|f16 (gptq_module.py:176-181).
-    beta == 0 does not read hessian."""
-    dev = _dev(hessian, x)
+    beta == 0 does not read hessian.  bad (int32, one element) becomes 1 if the new hessian is not finite, 0 if it is."""
+    dev = _dev(hessian, x, bad)
+    _need(bad is None or (bad.dtype == torch.int32 and bad.numel() == 1), "hessian_update: bad must be one int32 value")
     _need(hessian.dim() == 2 and hessian.shape[0] == hessian.shape[1] and hessian.dtype == torch.float32 and
           hessian.is_contiguous(), "hessian_update: the Hessian must be a contiguous square fp32 matrix")
     _need(x.dim() == 2 and x.shape[1] == hessian.shape[0], "hessian_update: x must be [tokens, {}]".format(hessian.shape[0]))
@@ -241,8 +242,8 @@ def hessian_update(hessian, x, beta, alpha):
     nbytes = lib.amct_hessian_update_workspace_bytes(tokens, cols)
     ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev)
     with _on(dev):
-        _lib.check(lib.amct_hessian_update(_p(hessian), _p(x), tokens, cols, float(beta), float(alpha), dtype_code(x.dtype),
-                                           _p(ws), ws.numel(), _stream(dev)))
+        _lib.check(lib.amct_hessian_update_checked(_p(hessian), _p(x), tokens, cols, float(beta), float(alpha),
+                                                   dtype_code(x.dtype), _p(bad), _p(ws), ws.numel(), _stream(dev)))
     return hessian
 
 

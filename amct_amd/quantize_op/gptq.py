@@ -28,7 +28,9 @@ def update_hessian(hessian, nsamples, input_data, columns):
         else:
             beta = nsamples / (nsamples + batch_size)
         nsamples += batch_size
-        hessian = ops.hessian_update(hessian, rows, beta, 2 / nsamples)
+        bad = torch.empty(1, dtype=torch.int32, device=rows.device)
+        hessian = ops.hessian_update(hessian, rows, beta, 2 / nsamples, bad)
+        finite = not int(bad)
     else:
         # fp32 activations keep the fp32 product
         x = rows.t()
@@ -38,7 +40,8 @@ def update_hessian(hessian, nsamples, input_data, columns):
         nsamples += batch_size
         x = math.sqrt(2 / nsamples) * x.float()
         hessian = hessian + x.matmul(x.t())
-    if not torch.isfinite(hessian).all():
+        finite = bool(torch.isfinite(hessian).all())
+    if not finite:
         raise RuntimeError("hessian matrix has invalid value, inf or nan.")
     return hessian, nsamples
 

@@ -413,6 +413,9 @@ int amct_gptq_factor(const float* hessian, const int64_t* perm, const float* dam
 size_t amct_hessian_update_workspace_bytes(int64_t tokens, int64_t cols);
 int amct_hessian_update(float* hessian, const void* x, int64_t tokens, int64_t cols, float beta, float alpha,
                         int dtype, void* workspace, size_t workspace_bytes, amct_stream_t stream);
+/* The same, and *bad (int32 on the device) = 1 if an element of the new hessian is not finite, 0 if all are. */
+int amct_hessian_update_checked(float* hessian, const void* x, int64_t tokens, int64_t cols, float beta, float alpha, int dtype,
+                                int32_t* bad, void* workspace, size_t workspace_bytes, amct_stream_t stream);
 
 /* ---- interchange formats of the checkpoint converter ---------------------------------------
  * (amct_pytorch/experimental/quantization/DeepSeekV3.2/deploy.py)

@@ -4,6 +4,7 @@ factorisations and GEMMs are library calls on both sides)."""
 import pytest
 import torch
 
+from amct_amd import ops
 from amct_amd.quantize_op import gptq
 from oracle import gptq as og
 from oracle import int_quant as iq
@@ -197,3 +198,22 @@ def test_gptq_full_block_is_the_general_kernel(dev, sym, n, special):
     assert torch.equal(got_e.isnan(), want_e.isnan())
     assert_bits_equal(got.nan_to_num(1.5).cpu(), padded[:, :count].contiguous().nan_to_num(1.5).cpu(), "weight block")
     assert torch.equal(got.isnan(), padded[:, :count].isnan())
+
+
+@pytest.mark.parametrize("cols", [8, 130, 300])
+@pytest.mark.parametrize("where", [None, 'first', 'last', 'overflow', 'old'])
+def test_hessian_update_reports_what_is_not_finite(dev, cols, where):
+    x = torch.ones(5, cols, dtype=torch.bfloat16, device=dev)
+    h = torch.ones(cols, cols, device=dev)
+    if where == 'first':
+        x[0, 0] = float('nan')
+    elif where == 'last':
+        x[4, cols - 1] = float('inf')
+    elif where == 'overflow':
+        x[2, cols // 2] = 3e38
+    elif where == 'old':
+        h[cols - 1, 0] = h[0, cols - 1] = float('-inf')
+    bad = torch.full((1,), 7, dtype=torch.int32, device=dev)
+    for _ in range(2):
+        ops.hessian_update(h, x, 0.5, 0.5, bad)
+        assert int(bad) == int(where is not None) == int(not bool(torch.isfinite(h).all()))
