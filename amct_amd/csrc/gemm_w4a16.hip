@@ -1967,11 +1967,24 @@ static SpecPlan spec_plan(int64_t M, int64_t N, int64_t K, int group, int64_t cu
         }
         return true;
     };
-    int64_t S = cus / blocks;
-    if (S > 8) S = 8;
-    while (S > 1 && K / S < 2048) --S;
-    if (S < 1) S = 1;
-    while (S <= 16 && S <= units && !fits(S)) ++S;
+    auto slices = [&](int64_t nblocks) {
+        int64_t S = cus / nblocks;
+        if (S > 8) S = 8;
+        while (S > 1 && K / S < 2048) --S;
+        if (S < 1) S = 1;
+        while (S <= 16 && S <= units && !fits(S)) ++S;
+        return S;
+    };
+    int64_t S = slices(blocks);
+    // Where K is split anyway and the slices stay long, 128x128 blocks over twice the slices: a step of theirs takes 1.5
+    // times a step of the 128x64 block (each weight is dequantised for the same 128 rows, each row of the activations is read
+    // by half as many blocks) and there are half as many steps; the partial sums double.  K = 11008 / 14336, 128x64 -> 128x128:
+    // int8 W[4096, K] at 200 rows 43.3 -> 39.6 / 54.1 -> 47.2 us, int4 48.4 -> 39.3 us, W[2048, K] at 300 rows 40.5 -> 36.7 /
+    // 50.9 -> 39.9 us (slices of 5504 / 7168); with slices of 2752 and 3584 the other way round (80 rows: 28.6 -> 30.8 us).
+    if (p.shape == 4 && S > 1 && K / S > 4096) {
+        const int64_t S1 = slices(mt * nt128);
+        if (S1 > S && S1 <= 8) p.shape = 1, S = S1;
+    }
     if (S > 16 || S > units || mt > 65535) return SpecPlan{0, 1};
     p.splits = (int)S;
     return p;

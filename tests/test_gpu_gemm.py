@@ -510,3 +510,33 @@ def test_gemm_random_shapes(dev, seed):
         o4 = ops.gemm_w4a16(x.to(dev), workloads.pack_nibbles(codes).to(dev), scales.to(dev), zeros.to(dev), group,
                             None if sm is None else sm.to(dev), bias.to(dev)).cpu()
         w4a16_check(o4, x, codes, scales, zeros, group, sm, bias, what=(M, N, K, group, sdt, sm is not None))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bits", [4, 8])
+# the edges of the rule that moves long K slices onto 128x128 blocks: rows 129 (two row tiles), 200, 256; columns that end
+# inside a 128-column tile; K whose units of 256 do not divide by the slices; slices of 4096 (not moved) and just above
+@pytest.mark.parametrize("M,N,K", [(129, 4040, 11008), (200, 2056, 14336), (256, 4096, 8448), (200, 4096, 8192), (80, 8200, 11008)])
+def test_long_slices_on_square_blocks(dev, dtype, bits, M, N, K):
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    group = 128 if bits == 4 else K
+    x = torch.randn(M, K, generator=g, device=dev).to(dtype)
+    scales = (1e-3 + 9e-3 * torch.rand(N, K // group, generator=g, device=dev)).to(dtype)
+    bias = torch.randn(N, generator=g, device=dev)
+    if bits == 4:
+        packed = torch.randint(0, 256, (N, K // 2), generator=g, device=dev, dtype=torch.uint8)
+        zeros = torch.randint(0, 16, (N, K // group), generator=g, device=dev, dtype=torch.uint8)
+        got = ops.gemm_w4a16(x, packed, scales, zeros, group, None, bias)
+        u = torch.stack([packed & 15, packed >> 4], dim=-1).reshape(N, K).float()
+        w = (u.reshape(N, -1, group) - zeros.float().unsqueeze(-1)) * scales.float().unsqueeze(-1)
+    else:
+        codes = torch.randint(-127, 128, (N, K), generator=g, device=dev, dtype=torch.int8)
+        got = ops.gemm_w8a16(x, codes, scales, None, group, None, bias)
+        w = codes.float().reshape(N, -1, group) * scales.float().unsqueeze(-1)
+    w = w.reshape(N, K).to(dtype).double()                          # these kernels round the weight to the activations' type
+    want = x.double() @ w.t() + bias.double()
+    # a sum of K products of random sign stays within four standard deviations, and each of its K fp32 additions rounds
+    # by at most 2^-24 of that; then the result's own rounding
+    norm = ((x.double() ** 2) @ (w ** 2).t() + bias.double() ** 2).sqrt()
+    bound = (K + 2) * 2.0 ** -24 * 4 * norm + torch.finfo(dtype).eps * want.abs()
+    assert bool(((got.double() - want).abs() <= bound).all())
