@@ -30,6 +30,7 @@ SIGNATURES = {
     "amct_mfma_yardstick": (_I, [_I, _I, _I, _P, _P, _P]),
     "amct_minmax": (_I, [_P, _P, _P, _L, _L, _I, _I, _P]),
     "amct_gptq_block": (_I, [_P, _L, _P, _L, _P, _L, _P, _P, _L, _P, _L, _I, _I, _I, _P]),
+    "amct_col_minmax_update": (_I, [_P, _L, _L, _I, _P, _P, _I, _P, _P, _I, _P, ctypes.c_size_t, _P]),
     "amct_awq_candidates": (_I, [_P, _P, _P, _I, _L, _I, _P]),
     "amct_awq_loss_partials": (_I, [_P, _P, _L, _I, _P, _P]),
     "amct_awq_pick": (_I, [_P, _L, _I, _I, _P, _P, _P]),

@@ -155,6 +155,27 @@ def col_minmax(x, col_max=None, col_min=None, absolute=False):
     return col_max if absolute else (col_max, col_min)
 
 
+def col_minmax_update(x, old_max, old_min, out_dtype):
+    """(new_max, new_min) [cols] in out_dtype: the running update of col_minmax with old_max / old_min ([cols], one dtype) read
+    where they are and left alone.  x [rows > 0, cols]."""
+    rows, cols = x.shape
+    for name, t in (("old_max", old_max), ("old_min", old_min)):
+        _need(t.numel() == cols and t.is_contiguous() and t.dtype == old_max.dtype,
+              "col_minmax_update: {} must be a contiguous tensor of {} elements", name, cols)
+    dev = _dev(x, old_max, old_min)
+    x = _c(x)
+    new_max = torch.empty(cols, dtype=out_dtype, device=dev)
+    new_min = torch.empty(cols, dtype=out_dtype, device=dev)
+    lib = _lib.load()
+    nbytes = lib.amct_col_minmax_workspace_bytes(rows, cols)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    with _on(dev):
+        _lib.check(lib.amct_col_minmax_update(_p(x), rows, cols, dtype_code(x.dtype), _p(old_max), _p(old_min),
+                                              dtype_code(old_max.dtype), _p(new_max), _p(new_min), dtype_code(out_dtype), _p(ws),
+                                              nbytes, _stream(dev)))
+    return new_max, new_min
+
+
 def awq_loss(y, yhat):
     """mean((y - yhat)^4) as a 0-d fp32 tensor on the device, the difference rounded to the tensors' dtype
     (algorithm/awq.py:96); one pass over both tensors."""

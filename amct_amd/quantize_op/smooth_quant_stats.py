@@ -7,6 +7,8 @@ import torch
 from .. import ops
 from .utils import calculate_scale_offset
 
+_KERNEL_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
+
 
 def new_channel_stats(weight):
     """(data_max, data_min) as the module initialises them (:58-61): [1, K] of the weight's dtype, -inf / +inf."""
@@ -23,6 +25,9 @@ def update_channel_min_max(inputs, data_max, data_min):
     (data_max, data_min), [1, K], in the promoted dtype of inputs and the running tensors like torch.where."""
     x2 = inputs.reshape(-1, inputs.shape[-1])
     out_dtype = torch.promote_types(x2.dtype, data_max.dtype)
+    if x2.shape[0] > 0 and data_max.dtype == data_min.dtype and data_max.dtype in _KERNEL_DTYPES and out_dtype in _KERNEL_DTYPES:
+        new_max, new_min = ops.col_minmax_update(x2, data_max.reshape(-1).contiguous(), data_min.reshape(-1).contiguous(), out_dtype)
+        return new_max.reshape(1, -1), new_min.reshape(1, -1)
     cmax = data_max.reshape(-1).to(torch.float32).contiguous()
     cmin = data_min.reshape(-1).to(torch.float32).contiguous()
     ops.col_minmax(x2, cmax, cmin)

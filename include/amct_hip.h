@@ -98,6 +98,12 @@ int amct_mfma_yardstick(int bf16, int random_operands, int iters, void* sink, in
 size_t amct_col_minmax_workspace_bytes(int64_t rows, int64_t cols);
 int amct_col_minmax(const void* x, float* col_max, float* col_min, int64_t rows, int64_t cols, int absolute,
                     int accumulate, int dtype, void* workspace, size_t workspace_bytes, amct_stream_t stream);
+/* The running update with the values in dtypes of their own: new_max = batch > old_max ? batch : old_max and the mirror image for
+ * the minimum, [cols] each, the old values in old_dtype, the new ones in new_dtype (new_ may be old_ where the dtypes agree);
+ * rows > 0.  Workspace as for amct_col_minmax. */
+int amct_col_minmax_update(const void* x, int64_t rows, int64_t cols, int dtype, const void* old_max, const void* old_min,
+                           int old_dtype, void* new_max, void* new_min, int new_dtype, void* workspace, size_t workspace_bytes,
+                           amct_stream_t stream);
 
 /* amct_col_minmax without a workspace argument.  No counterpart in the reference: it is for callers that cannot
  * allocate device memory around the call (code under HIP graph capture, tight serving loops, harnesses that forbid

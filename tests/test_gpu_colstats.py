@@ -90,3 +90,27 @@ def test_col_minmax_errors(dev):
     assert lib.amct_col_minmax(x.data_ptr(), None, None, 4, 8, 0, 0, 0, ws.data_ptr(), need, st) == -1
     assert lib.amct_col_minmax(x.data_ptr(), out.data_ptr(), None, 4, 8, 0, 0, 9, ws.data_ptr(), need, st) == -1
     assert lib.amct_col_minmax(None, None, None, 0, 8, 0, 0, 0, None, 0, st) == 0
+
+
+@pytest.mark.parametrize("xdt", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("odt", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 7), (257, 72), (16500, 40)])
+def test_running_update_of_any_dtypes(dev, xdt, odt, rows, cols):
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, cols, generator=g).to(xdt)
+    x[0, cols // 2] = float('nan')
+    dmax, dmin = torch.randn(1, cols, generator=g).abs().to(odt), -torch.randn(1, cols, generator=g).abs().to(odt)
+    dmax[0, 0] = float('-inf')
+    want_max = torch.where(x.amax(0, keepdim=True) > dmax, x.amax(0, keepdim=True), dmax)
+    want_min = torch.where(x.amin(0, keepdim=True) < dmin, x.amin(0, keepdim=True), dmin)
+    for strided in (False, True):
+        old = [t.to(dev) for t in (dmax, dmin)]
+        if strided:
+            old = [torch.stack([t, t], dim=-1)[..., 0] for t in old]
+        kept = [t.clone() for t in old]
+        got_max, got_min = sqs.update_channel_min_max(x.to(dev), *old)
+        assert got_max.shape == want_max.shape and got_max.dtype == want_max.dtype
+        assert torch.equal(got_max.cpu(), want_max) and torch.equal(got_min.cpu(), want_min)
+        assert all(torch.equal(a, b) for a, b in zip(old, kept)), "the values before stay as they are"
+    got = sqs.update_channel_min_max(x[:0].to(dev), dmax.to(dev), dmin.to(dev))
+    assert got[0].dtype == want_max.dtype and torch.equal(got[0].cpu(), dmax.to(want_max.dtype))
