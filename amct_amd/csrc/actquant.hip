@@ -65,16 +65,7 @@ __global__ __launch_bounds__(kBlock) void act_quant_token(const void* x, const v
         mn = fmin_nan(mn, sm[0][wv]);
         mx = fmax_nan(mx, sm[1][wv]);
     }
-    float s;
-    if (mode == 0) {
-        s = make_factors<AMCT_F32>(mx, mn, 8, true, AMCT_SCOPE_AMCT).s;
-    } else {
-        // node.py:181-204: xmax = max(|min(amin,0)|, max(amax,0)); s = xmax / 127; s = 1 where xmax == 0
-        const float hi = fmax_nan(mx, 0.f), lo = fmin_nan(mn, 0.f);
-        const float amax = fmax_nan(__builtin_fabsf(lo), hi);
-        s = amax / 127.0f;
-        s = (amax == 0.f) ? 1.0f : s;
-    }
+    const float s = token_scale(mx, mn, mode);
     if (tid == 0) scale[row] = s;
     const Divisor dv = make_divisor(s);
     const uint32_t big = max(__float_as_uint(mx) & 0x7FFFFFFFu, __float_as_uint(mn) & 0x7FFFFFFFu);
@@ -124,15 +115,7 @@ __global__ __launch_bounds__(kBlock) void act_quant_token_general(const void* x,
         mn = fmin_nan(mn, sm[0][wv]);
         mx = fmax_nan(mx, sm[1][wv]);
     }
-    float s;
-    if (mode == 0) {
-        s = make_factors<AMCT_F32>(mx, mn, 8, true, AMCT_SCOPE_AMCT).s;
-    } else {
-        const float hi = fmax_nan(mx, 0.f), lo = fmin_nan(mn, 0.f);
-        const float amax = fmax_nan(__builtin_fabsf(lo), hi);
-        s = amax / 127.0f;
-        s = (amax == 0.f) ? 1.0f : s;
-    }
+    const float s = token_scale(mx, mn, mode);
     if (tid == 0) scale[row] = s;
     for (int64_t c = tid; c < K; c += kBlock) {
         float v = load_scalar<DT>(x, row * K + c);

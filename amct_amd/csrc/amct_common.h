@@ -295,6 +295,15 @@ AMCT_DEV Factors make_factors(float vmax, float vmin, int bits, bool symmetric, 
     return r;
 }
 
+// The live scale of one token from its extrema: mode 0 as weights get theirs (symmetric, int8), mode 1 as
+// experimental node.py:181-204: xmax = max(|min(amin,0)|, max(amax,0)); s = xmax / 127; s = 1 where xmax == 0
+AMCT_DEV float token_scale(float mx, float mn, int mode) {
+    if (mode == 0) return make_factors<AMCT_F32>(mx, mn, 8, true, AMCT_SCOPE_AMCT).s;
+    const float hi = fmax_nan(mx, 0.f), lo = fmin_nan(mn, 0.f);
+    const float amax = fmax_nan(__builtin_fabsf(lo), hi);
+    return amax == 0.f ? 1.0f : amax / 127.0f;
+}
+
 // the element divisor of a segment from its factors (no second reciprocal)
 AMCT_DEV Divisor divisor_of(const Factors& f) {
     Divisor d;

@@ -1288,7 +1288,10 @@ extern "C" size_t amct_gemm_w8a8_workspace_bytes(int64_t M, int64_t N, int64_t K
 namespace amct {
 int w8a8_stream_quant_dispatch(const void* x, int x_dtype, const void* smooth, const void* act_scale, const void* act_zp,
                                int per_token, const int8_t* wq, const float* s_tok, const float* s_ch, const void* bias,
-                               int bias_kind, void* out, int64_t M, int64_t N, int64_t K, int out_dtype, hipStream_t st);   // gemm_w8a8_stream.hip
+                               int bias_kind, void* out, int64_t M, int64_t N, int64_t K, int out_dtype, hipStream_t st);
+int w8a8_stream_dynamic_dispatch(const void* x, int x_dtype, const void* smooth, int mode, const int8_t* wq, const float* s_ch,
+                                 const void* bias, int bias_kind, void* out, int64_t M, int64_t N, int64_t K, int out_dtype,
+                                 hipStream_t st);                   // gemm_w8a8_stream.hip   // gemm_w8a8_stream.hip
 }
 
 // the int8 activations of the two-kernel form (rounded up to 16 bytes), then what the GEMM asks for
@@ -1319,6 +1322,36 @@ extern "C" int amct_linear_w8a8(const void* x, int x_dtype, const void* smooth, 
     if (rc != AMCT_OK) return rc;
     return amct_gemm_w8a8_ws(xq, wq, s_tok, s_ch, bias, bias_kind, out, nullptr, M, N, K, out_dtype,
                              reinterpret_cast<char*>(workspace) + xq_bytes, workspace_bytes - xq_bytes, stream);
+}
+
+static size_t dynamic_rows_bytes(int64_t M, int64_t K) {           // the int8 activations and their scales
+    return (((size_t)M * (size_t)K + 15) & ~(size_t)15) + (((size_t)M * 4 + 15) & ~(size_t)15);
+}
+
+extern "C" size_t amct_linear_w8a8_dynamic_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    return dynamic_rows_bytes(M, K) + amct_gemm_w8a8_workspace_bytes(M, N, K);
+}
+
+extern "C" int amct_linear_w8a8_dynamic(const void* x, int x_dtype, const void* smooth, int mode, const int8_t* wq, const float* s_ch,
+                                        const void* bias, int bias_kind, void* out, int64_t M, int64_t N, int64_t K, int out_dtype,
+                                        void* workspace, size_t workspace_bytes, amct_stream_t stream) {
+    if (M < 0 || N <= 0 || K <= 0 || bias_kind < 0 || bias_kind > 2 || (mode != 0 && mode != 1)) return AMCT_E_BADARG;
+    if (x_dtype != AMCT_F32 && x_dtype != AMCT_F16 && x_dtype != AMCT_BF16) return AMCT_E_BADARG;
+    if (out_dtype != AMCT_F32 && out_dtype != AMCT_F16 && out_dtype != AMCT_BF16) return AMCT_E_BADARG;
+    if (M == 0) return AMCT_OK;
+    if (!x || !wq || !s_ch || !out || (bias_kind != 0 && !bias)) return AMCT_E_BADARG;
+    const int rc = w8a8_stream_dynamic_dispatch(x, x_dtype, smooth, mode, wq, s_ch, bias, bias_kind, out, M, N, K, out_dtype,
+                                                (hipStream_t)stream);
+    if (rc != AMCT_E_UNSUPPORTED) return rc;
+    const size_t rows_bytes = dynamic_rows_bytes(M, K);
+    if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0 || workspace_bytes < rows_bytes) return AMCT_E_BADARG;
+    int8_t* xq = reinterpret_cast<int8_t*>(workspace);
+    float* s_tok = reinterpret_cast<float*>(xq + (((size_t)M * (size_t)K + 15) & ~(size_t)15));
+    const int rq = amct_act_quant_per_token_int8(x, smooth, xq, s_tok, M, K, mode, x_dtype, stream);
+    if (rq != AMCT_OK) return rq;
+    return amct_gemm_w8a8_ws(xq, wq, s_tok, s_ch, bias, bias_kind, out, nullptr, M, N, K, out_dtype,
+                             reinterpret_cast<char*>(workspace) + rows_bytes, workspace_bytes - rows_bytes, stream);
 }
 
 extern "C" int amct_gemm_w8a8(const int8_t* xq, const int8_t* wq, const float* s_tok, const float* s_ch,

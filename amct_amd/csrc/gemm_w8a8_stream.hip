@@ -37,10 +37,15 @@ struct StreamArgs8 {
     const void* act_scale;                           // [1] or [M] (per_token)
     const void* act_zp;                              // the same shape, or null
     int per_token;
+    // DYN: act_scale and act_zp are not read; every row is quantised with its own live scale (mode as for
+    // amct_act_quant_per_token_int8, whose arithmetic this repeats element for element) and leaves with it
+    int mode;
 };
 
 // XJ: 16-byte activation vectors a thread stages (clamped duplicates beyond the tensor)
-template <int ODT, int KS, int CG, int NL, int XJ, int XDT = 0>
+// DYN: the 64 vectors of a wave belong to one row (K / 8 is a multiple of 64), so a row's extrema are the reduced ones of
+// K / 512 waves, met in LDS; the row's factors are computed once per block.
+template <int ODT, int KS, int CG, int NL, int XJ, int XDT = 0, bool DYN = false>
 __global__ __launch_bounds__(KS * CG * 64) void w8a8_stream(StreamArgs8 a) {
     static_assert(NL % 2 == 0, "the weight loads come in pairs");
     extern __shared__ __align__(16) uint8_t lds[];
@@ -59,7 +64,9 @@ __global__ __launch_bounds__(KS * CG * 64) void w8a8_stream(StreamArgs8 a) {
     const uint32_t KV = K / XE, n_xv = M * KV;
     uint4 xv[XJ];
     uint32_t xoff[XJ];
-    float qs[XDT ? XJ : 1], qz[XDT ? XJ : 1];
+    float qs[XDT && !DYN ? XJ : 1], qz[XDT && !DYN ? XJ : 1];
+    __shared__ __align__(16) float slot_mn[DYN ? XJ * KS * CG * 4 : 1], slot_mx[DYN ? XJ * KS * CG * 4 : 1];   // per 16 vectors
+    __shared__ float row_s[DYN ? 16 : 1], row_y[DYN ? 16 : 1];                          // y = 0: divide
     uint4 cvec = make_uint4(0u, 0u, 0u, 0u);
 #pragma unroll
     for (int j = 0; j < XJ; ++j) {
@@ -69,9 +76,11 @@ __global__ __launch_bounds__(KS * CG * 64) void w8a8_stream(StreamArgs8 a) {
         xoff[j] = row * xstride + (vc - row * KV) * XE;
         if constexpr (XDT != 0) {
             xv[j] = ldg16(reinterpret_cast<const char*>(a.x16) + (size_t)vc * 16);
-            const int64_t si = a.per_token ? row : 0;
-            qs[j] = load_scalar<XDT>(a.act_scale, si);
-            qz[j] = a.act_zp ? load_scalar<XDT>(a.act_zp, si) : 0.f;
+            if constexpr (!DYN) {
+                const int64_t si = a.per_token ? row : 0;
+                qs[j] = load_scalar<XDT>(a.act_scale, si);
+                qz[j] = a.act_zp ? load_scalar<XDT>(a.act_zp, si) : 0.f;
+            }
             // NT is a multiple of K / 8: every vector of a thread lies in the same columns
             if (j == 0 && a.smooth) cvec = ldg16(reinterpret_cast<const char*>(a.smooth) + (size_t)(vc - row * KV) * 16);
         } else {
@@ -108,12 +117,83 @@ __global__ __launch_bounds__(KS * CG * 64) void w8a8_stream(StreamArgs8 a) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int m = 4 * g + r;
-        tok[r] = a.s_tok ? a.s_tok[m < (int)M ? m : (int)M - 1] : 1.0f;
+        tok[r] = !DYN && a.s_tok ? a.s_tok[m < (int)M ? m : (int)M - 1] : 1.0f;
     }
     __builtin_amdgcn_sched_barrier(0);
 
     // ---- stage the activations (waits are in issue order: the weights stay in flight) ---------------------------
-    if constexpr (XDT != 0) {
+    if constexpr (DYN) {
+        float c[8];
+        if (a.smooth) unpack16<XDT>(cvec, c);
+        auto smoothed = [&](int j, float (&f)[8]) {
+            unpack16<XDT>(xv[j], f);
+            if (a.smooth) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) f[e] = round_to<XDT>(f[e] * c[e]);
+            }
+        };
+#pragma unroll
+        for (int j = 0; j < XJ; ++j) {
+            float f[8];
+            smoothed(j, f);
+            float mx = f[0], mn = f[0];
+#pragma unroll
+            for (int e = 1; e < 8; ++e) {
+                mx = fmax_nan(mx, f[e]);
+                mn = fmin_nan(mn, f[e]);
+            }
+            team_minmax<16>(mn, mx);                 // the exchanges beyond 16 lanes go through LDS: left to the row's thread
+            if (r16 == 0) {
+                slot_mn[(j * (KS * CG) + wave) * 4 + g] = mn;
+                slot_mx[(j * (KS * CG) + wave) * 4 + g] = mx;
+            }
+            __builtin_amdgcn_sched_barrier(0);       // one vector unpacked at a time: the weights hold half the registers
+        }
+        __syncthreads();
+        if (tid < (int)M) {
+            const int per = (int)(KV / 64);          // slots of a row, by fours; slot of vector v: v / 16
+            const float4* px = reinterpret_cast<const float4*>(slot_mx) + tid * per;
+            const float4* pn = reinterpret_cast<const float4*>(slot_mn) + tid * per;
+            float mx = px[0].x, mn = pn[0].x;
+#pragma unroll 2
+            for (int i = 0; i < per; ++i) {
+                const float4 vx = px[i], vn = pn[i];
+                mx = fmax_nan(fmax_nan(fmax_nan(mx, vx.x), fmax_nan(vx.y, vx.z)), vx.w);
+                mn = fmin_nan(fmin_nan(fmin_nan(mn, vn.x), fmin_nan(vn.y, vn.z)), vn.w);
+            }
+            const float s = token_scale(mx, mn, a.mode);
+            const Divisor dv = make_divisor(s);
+            const uint32_t big = max(__float_as_uint(mx) & 0x7FFFFFFFu, __float_as_uint(mn) & 0x7FFFFFFFu);
+            row_s[tid] = s;
+            row_y[tid] = dv.fast && big < 0x5D800000u ? dv.y : 0.f;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < XJ; ++j) {
+            const uint32_t v = tid + NT * j;
+            const uint32_t row = __umulhi(v < n_xv ? v : n_xv - 1, a.kv_magic);
+            // (unpacked again: kept from the first pass the values take twice the registers)
+            asm volatile("" : "+v"(xv[j].x), "+v"(xv[j].y), "+v"(xv[j].z), "+v"(xv[j].w));
+            float f[8], q[8];
+            smoothed(j, f);
+            Divisor dv;
+            dv.s = row_s[row];
+            dv.y = row_y[row];
+            dv.fast = dv.y != 0.f;
+            if (wave_all(dv.fast)) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) q[e] = quant_elem<XDT, false, true, false>(f[e], dv, 0.f, false, -128.f, 127.f);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) q[e] = quant_elem<XDT, false, false>(f[e], dv, 0.f, false, -128.f, 127.f);
+            }
+            uint32_t o[2] = {0u, 0u};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e >> 2] |= ((uint32_t)(int)q[e] & 0xFFu) << (8 * (e & 3));
+            if (v < n_xv) *reinterpret_cast<uint2*>(lds + xoff[j]) = make_uint2(o[0], o[1]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    } else if constexpr (XDT != 0) {
         float c[8];
         if (a.smooth) unpack16<XDT>(cvec, c);
 #pragma unroll
@@ -192,7 +272,8 @@ __global__ __launch_bounds__(KS * CG * 64) void w8a8_stream(StreamArgs8 a) {
             const size_t o = (size_t)m * a.N + ncol;
             if (a.acc_out) a.acc_out[o] = t;
             float f = (float)t * sc;
-            if (a.s_tok) f = f * tok[r];
+            if constexpr (DYN) f = f * row_s[m];
+            else if (a.s_tok) f = f * tok[r];
             if (a.bias_kind == 2) f = f + fb;
             if constexpr (ODT == AMCT_F32) reinterpret_cast<float*>(a.out)[o] = f;
             else if constexpr (ODT == AMCT_BF16) reinterpret_cast<uint16_t*>(a.out)[o] = (uint16_t)f32_to_bf16_bits(f);
@@ -201,7 +282,7 @@ __global__ __launch_bounds__(KS * CG * 64) void w8a8_stream(StreamArgs8 a) {
     }
 }
 
-template <int ODT, int KS, int CG, int NL, int XDT = 0>
+template <int ODT, int KS, int CG, int NL, int XDT = 0, bool DYN = false>
 static int stream8_launch_x(const StreamArgs8& a, size_t lds_bytes, hipStream_t st) {
     constexpr int NT = KS * CG * 64;
     const int n_xv = a.M * (a.K / (XDT ? 8 : 16));
@@ -209,9 +290,9 @@ static int stream8_launch_x(const StreamArgs8& a, size_t lds_bytes, hipStream_t 
     const dim3 grid((unsigned)((a.N + CG * 16 - 1) / (CG * 16)));
 #define AMCT_STREAM8_GO(XJ)                                                                                         \
     {                                                                                                               \
-        auto kern = &w8a8_stream<ODT, KS, CG, NL, XJ, XDT>;                                                         \
+        auto kern = &w8a8_stream<ODT, KS, CG, NL, XJ, XDT, DYN>;                                                    \
         if (lds_bytes > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern),                       \
-                                                         hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess) { \
+                                                         hipFuncAttributeMaxDynamicSharedMemorySize, 152 * 1024) != hipSuccess) { \
             (void)hipGetLastError();                                                                                \
             return AMCT_E_HIP;                                                                                      \
         }                                                                                                           \
@@ -223,15 +304,18 @@ static int stream8_launch_x(const StreamArgs8& a, size_t lds_bytes, hipStream_t 
     }
     if (xj <= 2) AMCT_STREAM8_GO(2)
     if (xj <= 4) AMCT_STREAM8_GO(4)
-    if (xj <= 8) AMCT_STREAM8_GO(8)
+    if constexpr (!DYN) {
+        if (xj <= 8) AMCT_STREAM8_GO(8)
+    }
 #undef AMCT_STREAM8_GO
     return AMCT_E_UNSUPPORTED;
 }
 
-template <int ODT, int XDT = 0>
+template <int ODT, int XDT = 0, bool DYN = false>
 static int stream8_shape(const StreamArgs8& a, int cg, int nl, size_t lds_bytes, hipStream_t st) {
 #define AMCT_STREAM8_SHAPE(CG_, NL_) \
-    if (cg == CG_ && nl == NL_) return stream8_launch_x<ODT, 4, CG_, NL_, XDT>(a, lds_bytes, st);
+    if constexpr (!DYN || CG_ == 2)                                 \
+        if (cg == CG_ && nl == NL_) return stream8_launch_x<ODT, 4, CG_, NL_, XDT, DYN>(a, lds_bytes, st);
     AMCT_STREAM8_SHAPE(4, 16)
     AMCT_STREAM8_SHAPE(2, 16)
     AMCT_STREAM8_SHAPE(4, 8)
@@ -250,7 +334,7 @@ int w8a8_stream_dispatch(const int8_t* xq, const int8_t* wq, const float* s_tok,
     if (M < 1 || M > 16 || (K != 1024 && K != 2048 && K != 4096) || N > (int64_t(1) << 30)) return AMCT_E_UNSUPPORTED;
     if (!aligned16(xq) || !aligned16(wq)) return AMCT_E_UNSUPPORTED;
     StreamArgs8 a{xq, wq, s_tok, s_ch, bias_kind ? bias : nullptr, out, acc_out, (int)M, (int)N, (int)K, bias_kind,
-                  (uint32_t)(0x100000000ull / (uint64_t)(K / 16)) + 1u, nullptr, nullptr, nullptr, nullptr, 0};
+                  (uint32_t)(0x100000000ull / (uint64_t)(K / 16)) + 1u, nullptr, nullptr, nullptr, nullptr, 0, 0};
     // Large activation blocks are staged by few, wide blocks (16 waves share one copy in LDS), small ones by blocks of
     // 8 waves.  Measured on W[14336,4096] (58.7 MB, us per call back to back): M = 1 10.8, M = 4 11.4, M = 16 12.4,
     // against 13.5 / 14.4 / 14.4 for the kernels this one replaced (blocks of 4 waves at M = 1: 11.3; blocks of 8 waves at
@@ -274,7 +358,7 @@ int w8a8_stream_quant_dispatch(const void* x, int x_dtype, const void* smooth, c
     if (x_dtype != AMCT_BF16 && x_dtype != AMCT_F16) return AMCT_E_UNSUPPORTED;
     if (!aligned16(x) || !aligned16(wq) || (smooth && !aligned16(smooth))) return AMCT_E_UNSUPPORTED;
     StreamArgs8 a{nullptr, wq, s_tok, s_ch, bias_kind ? bias : nullptr, out, nullptr, (int)M, (int)N, (int)K, bias_kind,
-                  (uint32_t)(0x100000000ull / (uint64_t)(K / 8)) + 1u, x, smooth, act_scale, act_zp, per_token};
+                  (uint32_t)(0x100000000ull / (uint64_t)(K / 8)) + 1u, x, smooth, act_scale, act_zp, per_token, 0};
     // the quantised image in LDS is what the int8 launch stages; block widths from the 16-bit source (twice the vectors)
     const size_t xbytes = (size_t)M * ((size_t)K + 16);
     const int cg = xbytes > 20 * 1024 ? 4 : 2;
@@ -288,6 +372,28 @@ int w8a8_stream_quant_dispatch(const void* x, int x_dtype, const void* smooth, c
     if (out_dtype == AMCT_F16) { AMCT_STREAM8_Q(AMCT_F16) }
     AMCT_STREAM8_Q(AMCT_F32)
 #undef AMCT_STREAM8_Q
+}
+
+// The same launch with a live scale per row (out of x's dtype only: what the deploy module writes), up to 16384 activations.
+// Every block quantises all of them, about 20 instructions each: below that line this hides behind the arriving weights and
+// saves a launch (two launches / one: M = 4, K = 4096 8.9 / 8.3 us for N = 512, 15.5 / 15.0 for N = 14336; M = 1 14.6 / 12.3;
+// M = 16, K = 1024 6.2 / 5.1), beyond it the block is busy quantising (M = 8, K = 4096: 9.1 / 10.0 and 16.1 / 16.4; M = 16,
+// N = 14336: 16.6 / 17.0, more in blocks of 8 waves).
+int w8a8_stream_dynamic_dispatch(const void* x, int x_dtype, const void* smooth, int mode, const int8_t* wq, const float* s_ch,
+                                 const void* bias, int bias_kind, void* out, int64_t M, int64_t N, int64_t K, int out_dtype,
+                                 hipStream_t st) {
+    if (M < 1 || M > 16 || (K != 1024 && K != 2048 && K != 4096) || M * K > 16384 || N > (int64_t(1) << 30)) return AMCT_E_UNSUPPORTED;
+    if ((x_dtype != AMCT_BF16 && x_dtype != AMCT_F16) || out_dtype != x_dtype) return AMCT_E_UNSUPPORTED;
+    if (!aligned16(x) || !aligned16(wq) || (smooth && !aligned16(smooth))) return AMCT_E_UNSUPPORTED;
+    StreamArgs8 a{nullptr, wq, nullptr, s_ch, bias_kind ? bias : nullptr, out, nullptr, (int)M, (int)N, (int)K, bias_kind,
+                  (uint32_t)(0x100000000ull / (uint64_t)(K / 8)) + 1u, x, smooth, nullptr, nullptr, 0, mode};
+    const size_t xbytes = (size_t)M * ((size_t)K + 16);
+    const int cg = 2;
+    const int nl = (int)(K / 256);
+    const size_t red = (size_t)3 * cg * 64 * 16;
+    const size_t lds_bytes = xbytes > red ? xbytes : red;
+    return x_dtype == AMCT_BF16 ? stream8_shape<AMCT_BF16, AMCT_BF16, true>(a, cg, nl, lds_bytes, st)
+                                : stream8_shape<AMCT_F16, AMCT_F16, true>(a, cg, nl, lds_bytes, st);
 }
 
 }  // namespace amct

@@ -78,10 +78,9 @@ class HipQuantizationLinear(torch.nn.Module):
         smooth = self.scale_factor if hasattr(self, 'scale_factor') else None
         lead = x.shape[:-1]
         if self.dynamic_act:
-            xq, s_tok = ops.act_quant_per_token_int8(x, smooth)
             s_ch = self.deq_scale if self.act_granularity == 'PER_TOKEN' else self._scale_w()
-            out = ops.gemm_w8a8(xq.reshape(-1, x.shape[-1]), self.quantized_weight.t(), s_ch, s_tok,
-                                self._float_bias(), self.output_dtype)
+            out = ops.linear_w8a8_dynamic(x.reshape(-1, x.shape[-1]), self.quantized_weight.t(), s_ch, self._float_bias(),
+                                          self.output_dtype, smooth)
             return out.reshape(*lead, -1)
         per_token = self.act_granularity == 'PER_TOKEN'
         x2 = x.reshape(-1, x.shape[-1])

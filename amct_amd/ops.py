@@ -701,6 +701,47 @@ def linear_w8a8(x, act_scale, act_offset, per_token, wq_nk, s_ch, s_tok=None, bi
     return out
 
 
+def linear_w8a8_dynamic(x, wq_nk, s_ch, bias=None, out_dtype=torch.bfloat16, smooth=None, mode=0):
+    """act_quant_per_token_int8 followed by gemm_w8a8 with the tokens' scales, in one library call (the W8A8 Linear with live
+    activation scales); x [M,K], the other operands as for those two.  A few tokens are quantised inside the weight-streaming
+    kernel."""
+    _need(x.dim() == 2 and wq_nk.dim() == 2 and wq_nk.dtype == torch.int8, "W8A8 Linear expects x [M,K] and an int8 weight [N,K]")
+    M, K = x.shape
+    N = wq_nk.shape[0]
+    if wq_nk.shape[1] != K:
+        raise RuntimeError("int8 GEMM: K mismatch ({} vs {})".format(K, wq_nk.shape[1]))
+    _need(s_ch.numel() in (1, N), "int8 GEMM: {} channel scales for {} output channels", s_ch.numel(), N)
+    _need(bias is None or bias.numel() == N, "int8 GEMM: bias has {} entries, {} output channels",
+          0 if bias is None else bias.numel(), N)
+    dev = _dev(x, wq_nk, s_ch, bias, smooth)
+    lib = _lib.load()
+    nbytes = lib.amct_linear_w8a8_dynamic_workspace_bytes(M, N, K)
+    ws = lent_workspace(dev, nbytes)
+    if M > 0 and (ws is None or ws.numel() < nbytes):  # less than the activations may need: the two calls
+        xq, s_tok = act_quant_per_token_int8(x, smooth, mode)
+        return gemm_w8a8(xq, wq_nk, s_ch, s_tok, bias, out_dtype)
+    x, wq_nk = _c(x), _c(wq_nk)
+    if smooth is not None:
+        smooth = _c(smooth.reshape(-1).to(x.dtype))
+        if smooth.numel() != K:
+            raise RuntimeError("smooth factor must have K elements")
+    s_ch = _c(s_ch.reshape(-1).to(torch.float32))
+    if s_ch.numel() == 1:
+        s_ch = s_ch.expand(N).contiguous()
+    kind = 0
+    if bias is not None:
+        if bias.dtype == torch.int32:
+            kind, bias = 1, _c(bias)
+        else:
+            kind, bias = 2, _c(bias.to(torch.float32))
+    out = torch.empty(M, N, dtype=out_dtype, device=dev)
+    with _on(dev):
+        _lib.check(lib.amct_linear_w8a8_dynamic(_p(x), dtype_code(x.dtype), _p(smooth), mode, _p(wq_nk), _p(s_ch), _p(bias), kind,
+                                                _p(out), M, N, K, dtype_code(out_dtype), _p(ws), 0 if ws is None else ws.numel(),
+                                                _stream(dev)))
+    return out
+
+
 def _check_weight_only(x, N, K, scales, zeros, group, smooth, bias, zeros_dtype, what):
     _need(x.dim() == 2 and x.shape[1] == K, "{}: activations must be [M, {}], got {}", what, K, tuple(x.shape))
     _need(x.dtype in (torch.bfloat16, torch.float16), "Not support tensor dtype {}, support dtypes {}.", x.dtype,

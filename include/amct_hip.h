@@ -290,6 +290,15 @@ int amct_linear_w8a8(const void* x, int x_dtype, const void* smooth, const void*
                      int64_t n_scales, int per_token, const int8_t* wq, const float* s_tok, const float* s_ch,
                      const void* bias, int bias_kind, void* out, int64_t M, int64_t N, int64_t K, int out_dtype,
                      void* workspace, size_t workspace_bytes, amct_stream_t stream);
+/* The W8A8 Linear with a live scale per token in one call: amct_act_quant_per_token_int8(x, smooth, mode) followed by
+ * amct_gemm_w8a8_ws with those scales, the bits of the two calls.  Up to 16 rows and 16384 16-bit activations of K = 1024, 2048
+ * or 4096 with out_dtype = x_dtype are quantised inside the weight-streaming kernel (no workspace is read then); other calls need
+ * amct_linear_w8a8_dynamic_workspace_bytes, 16-byte aligned, of which the part behind the int8 activations and their scales
+ * (M * K and 4 * M bytes, each rounded up to 16) may be missing. */
+size_t amct_linear_w8a8_dynamic_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int amct_linear_w8a8_dynamic(const void* x, int x_dtype, const void* smooth, int mode, const int8_t* wq, const float* s_ch,
+                             const void* bias, int bias_kind, void* out, int64_t M, int64_t N, int64_t K, int out_dtype,
+                             void* workspace, size_t workspace_bytes, amct_stream_t stream);
 
 /* ---- K7: W4A16 Linear -------------------------------------------------------------------------------------
  * Replaces torch_npu.npu_weight_quant_batchmatmul as called at

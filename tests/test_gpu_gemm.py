@@ -540,3 +540,41 @@ def test_long_slices_on_square_blocks(dev, dtype, bits, M, N, K):
     norm = ((x.double() ** 2) @ (w ** 2).t() + bias.double() ** 2).sqrt()
     bound = (K + 2) * 2.0 ** -24 * 4 * norm + torch.finfo(dtype).eps * want.abs()
     assert bool(((got.double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 64, 1024), (16, 200, 2048), (9, 72, 4096), (16, 14336, 4096), (5, 33, 2048), (3, 4104, 4096),
+                                   (16, 1000, 1024), (8, 520, 2048), (4, 1000, 4096), (17, 200, 1024), (7, 136, 8192), (300, 520, 4096), (2, 40, 100)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_linear_w8a8_with_live_scales_is_the_two_calls(dev, M, N, K, dtype):
+    """Per-token quantisation inside the weight-streaming kernel (up to 16 rows and 16384
+    activations, K of 1024 / 2048 / 4096, output in their type) and through the workspace: the bits of the two separate calls, for ordinary rows, rows of zeros,
+    rows whose scale leaves the range of the reciprocal division, infinities and NaN."""
+    g = torch.Generator().manual_seed(400 + M)
+    x = torch.randn(M, K, generator=g) * 3
+    x[M // 2, K // 3] = -0.0
+    rows = [x.clone() for _ in range(3)]
+    rows[1][0] = 0
+    rows[1][M - 1] *= 1e-30 if dtype != torch.float16 else 1e-7
+    rows[2][0, K - 1] = float('inf')
+    rows[2][M - 1, 0] = float('nan')
+    smooth = (0.5 + torch.rand(K, generator=g)).to(dtype).to(dev)
+    _, wq, s_ch, _, b = w8a8_case(M, N, K, 410 + M, True, 'float')
+    for x in rows:
+        x = x.to(dtype).to(dev)
+        for mode in (0, 1):
+            for sm, bias, odt in ((None, None, dtype), (smooth, b.to(dev), dtype), (smooth, None, torch.float32)):
+                got = ops.linear_w8a8_dynamic(x, wq.to(dev), s_ch.to(dev), bias, odt, sm, mode)
+                xq, s_tok = ops.act_quant_per_token_int8(x, sm, mode)
+                want = ops.gemm_w8a8(xq, wq.to(dev), s_ch.to(dev), s_tok, bias, odt)
+                assert torch.equal(got.isnan(), want.isnan())
+                assert_bits_equal(got.nan_to_num(7).cpu(), want.nan_to_num(7).cpu(), "one call against two, mode %d" % mode)
+    old = ops.workspace_limit_bytes
+    try:
+        ops.release_workspaces()
+        ops.workspace_limit_bytes = 64
+        assert torch.equal(ops.linear_w8a8_dynamic(rows[0].to(dtype).to(dev), wq.to(dev), s_ch.to(dev), None, dtype),
+                           ops.gemm_w8a8(*(lambda q: (q[0], wq.to(dev), s_ch.to(dev), q[1]))(
+                               ops.act_quant_per_token_int8(rows[0].to(dtype).to(dev))), out_dtype=dtype))
+    finally:
+        ops.workspace_limit_bytes = old
+        ops.release_workspaces()
