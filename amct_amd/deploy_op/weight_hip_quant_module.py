@@ -87,17 +87,15 @@ class HipWeightQuantizedLinear(nn.Module):
             self.bias = None
 
     def forward(self, inputs):
-        ori_shape = inputs.shape
         if inputs.dim() < 2 or inputs.dim() > 6:
             raise RuntimeError("Linear quant only support dim from 2 to 6")
-        inputs = inputs.to(self.quantized_weight.device).reshape(-1, ori_shape[-1])
-        if self.wts_type == 'int4':
-            out = ops.gemm_w4a16(inputs, self.quantized_weight, self.scale_w, self.offset_w, self._gemm_group,
-                                 self.scale_factor, self.bias)
-        else:
-            out = ops.gemm_w8a16(inputs, self.quantized_weight, self.scale_w, self.offset_w, self._gemm_group,
-                                 self.scale_factor, self.bias)
-        return out.reshape(*ori_shape[:-1], -1)
+        weight = self.quantized_weight
+        x = inputs if inputs.device == weight.device else inputs.to(weight.device)
+        flat = x.dim() == 2
+        gemm = ops.gemm_w4a16 if self.wts_type == 'int4' else ops.gemm_w8a16
+        out = gemm(x if flat else x.reshape(-1, inputs.shape[-1]), weight, self.scale_w, self.offset_w, self._gemm_group,
+                   self.scale_factor, self.bias)
+        return out if flat and out.shape[0] else out.reshape(*inputs.shape[:-1], -1)
 
     def reference_layout(self):
         """(quantized_weight, scale_w [K/g, N], offset_w [K/g, N] = -offset | None) as the reference registers them

@@ -24,17 +24,18 @@ def dtype_code(dt):
 
 def _dev(*tensors):
     """All tensors must live on one HIP device; there is no CPU path."""
-    dev = None
+    first, index = None, -1
     for t in tensors:
         if t is None:
             continue
-        if not t.is_cuda:
+        i = t.get_device()                             # an int per tensor: comparing device objects costs a call 2 us
+        if i < 0 or not t.is_cuda:
             raise RuntimeError("amct_amd kernels run on the GPU only: got a tensor on '{}'".format(t.device))
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise RuntimeError("amct_amd: tensors on different devices ({} vs {})".format(dev, t.device))
-    return dev
+        if first is None:
+            first, index = t, i
+        elif i != index:
+            raise RuntimeError("amct_amd: tensors on different devices ({} vs {})".format(first.device, t.device))
+    return None if first is None else first.device
 
 
 def _p(t):
@@ -56,6 +57,7 @@ def _segments(rows, cols, group):
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
 _SAME_DEVICE = contextlib.nullcontext()
 
 
@@ -68,13 +70,18 @@ def _stream(dev):
 
 def _on(dev):
     """Device guard for a launch: nothing to switch (the common case) when dev is already current."""
-    if dev.index is None or dev.index == torch.cuda.current_device():
+    if dev.index is None or dev.index == _current_device():
         return _SAME_DEVICE
     return torch.cuda.device(dev)
 
 
 def _c(t):
     return t if t.is_contiguous() else t.contiguous()
+
+
+def _flat(t, dtype):
+    """The elements of t in order in dtype, dense (t itself where it is that already: only its pointer is used)."""
+    return t if t.dtype == dtype and t.is_contiguous() else _c(t.reshape(-1).to(dtype))
 
 
 # Scratch memory the GEMM wrappers lend to the library (it never allocates): ONE grow-only byte tensor per device and
@@ -743,20 +750,25 @@ def linear_w8a8_dynamic(x, wq_nk, s_ch, bias=None, out_dtype=torch.bfloat16, smo
 
 
 def _check_weight_only(x, N, K, scales, zeros, group, smooth, bias, zeros_dtype, what):
-    _need(x.dim() == 2 and x.shape[1] == K, "{}: activations must be [M, {}], got {}", what, K, tuple(x.shape))
-    _need(x.dtype in (torch.bfloat16, torch.float16), "Not support tensor dtype {}, support dtypes {}.", x.dtype,
-          [torch.bfloat16, torch.float16])
-    _need(group > 0 and K % group == 0, "{}: K = {} is not a multiple of the group size {}", what, K, group)
+    # (plain conditions: the arguments of the messages are only worth building for a message)
+    if x.dim() != 2 or x.shape[1] != K:
+        raise RuntimeError("{}: activations must be [M, {}], got {}".format(what, K, tuple(x.shape)))
+    if x.dtype != torch.bfloat16 and x.dtype != torch.float16:
+        raise RuntimeError("Not support tensor dtype {}, support dtypes {}.".format(x.dtype, [torch.bfloat16, torch.float16]))
+    if group <= 0 or K % group != 0:
+        raise RuntimeError("{}: K = {} is not a multiple of the group size {}".format(what, K, group))
     want = (N, K // group)
-    _need(scales.dtype in (torch.float16, torch.bfloat16), "{}: scales must be fp16 or bf16, got {}", what, scales.dtype)
-    _need(tuple(scales.shape) == want, "{}: scales have shape {}, expected {}", what, tuple(scales.shape), want)
-    _need(zeros is None or (zeros.dtype == zeros_dtype and tuple(zeros.shape) == want),
-          "{}: zero-points have shape {} / dtype {}, expected {} / {}", what,
-          None if zeros is None else tuple(zeros.shape), None if zeros is None else zeros.dtype, want, zeros_dtype)
-    _need(smooth is None or smooth.numel() == K, "{}: smooth factor has {} entries, K = {}", what,
-          0 if smooth is None else smooth.numel(), K)
-    _need(bias is None or bias.numel() == N, "{}: bias has {} entries, {} output channels", what,
-          0 if bias is None else bias.numel(), N)
+    if scales.dtype != torch.float16 and scales.dtype != torch.bfloat16:
+        raise RuntimeError("{}: scales must be fp16 or bf16, got {}".format(what, scales.dtype))
+    if scales.shape != want:
+        raise RuntimeError("{}: scales have shape {}, expected {}".format(what, tuple(scales.shape), want))
+    if zeros is not None and (zeros.dtype != zeros_dtype or zeros.shape != want):
+        raise RuntimeError("{}: zero-points have shape {} / dtype {}, expected {} / {}".format(
+            what, tuple(zeros.shape), zeros.dtype, want, zeros_dtype))
+    if smooth is not None and smooth.numel() != K:
+        raise RuntimeError("{}: smooth factor has {} entries, K = {}".format(what, smooth.numel(), K))
+    if bias is not None and bias.numel() != N:
+        raise RuntimeError("{}: bias has {} entries, {} output channels".format(what, bias.numel(), N))
 
 
 def gemm_w4a16_weight_rounded(M, N, K, group, dtype, workspace_bytes=None):
@@ -798,15 +810,16 @@ def gemm_w4a16(x, wq_packed, scales, zeros, group, smooth=None, bias=None):
     x, wq_packed, scales, zeros = _c(x), _c(wq_packed), _c(scales), _c(zeros)
     M = x.shape[0]
     if smooth is not None:
-        smooth = _c(smooth.reshape(-1).to(x.dtype))
+        smooth = _flat(smooth, x.dtype)
     if bias is not None:
-        bias = _c(bias.reshape(-1).to(torch.float32))
+        bias = _flat(bias, torch.float32)
     out = torch.empty(M, N, dtype=x.dtype, device=dev)
     # the workspace the library asks for: the smoothed activations for the tile kernels, or the activation image the
     # weight-streaming kernel for a few rows fetches
-    ws = lent_workspace(dev, _lib.load().amct_gemm_w4a16_workspace_bytes(M, N, K, group, int(smooth is not None)))
+    lib = _lib.load()
+    ws = lent_workspace(dev, lib.amct_gemm_w4a16_workspace_bytes(M, N, K, group, int(smooth is not None)))
     with _on(dev):
-        _lib.check(_lib.load().amct_gemm_w4a16(_p(x), _p(smooth), _p(wq_packed), _p(scales), dtype_code(scales.dtype),
+        _lib.check(lib.amct_gemm_w4a16(_p(x), _p(smooth), _p(wq_packed), _p(scales), dtype_code(scales.dtype),
                                                _p(zeros), _p(bias), _p(out), M, N, K, group, dtype_code(x.dtype),
                                                _p(ws), 0 if ws is None else ws.numel(), _stream(dev)))
     return out
@@ -822,9 +835,9 @@ def gemm_w8a16(x, wq_nk, scales, offsets, group, smooth=None, bias=None):
     offsets = None if offsets is None else _c(offsets)
     M = x.shape[0]
     if smooth is not None:
-        smooth = _c(smooth.reshape(-1).to(x.dtype))
+        smooth = _flat(smooth, x.dtype)
     if bias is not None:
-        bias = _c(bias.reshape(-1).to(torch.float32))
+        bias = _flat(bias, torch.float32)
     out = torch.empty(M, N, dtype=x.dtype, device=dev)
     # the workspace the library asks for: from 256 rows on, the dequantised weight (and the smoothed activations)
     ws = lent_workspace(dev, _lib.load().amct_gemm_w8a16_workspace_bytes(M, N, K, group, int(smooth is not None)))
