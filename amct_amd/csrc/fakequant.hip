@@ -48,30 +48,35 @@ template <int DT> AMCT_DEV void apply_col_pre(float* x, const float* c, int mode
     }
 }
 
-// d[j] <- round_to<DT>(d[j]) / c[j].  FAST: every |d[j]| is 0 or in [2^-60, 2^70).  Two 16-bit numbers have a quotient that is
+// d[j] <- round_to<DT>(d[j]) / c[j], every |d[j]| 0 or in [2^-60, 2^70) where FAST.  Two 16-bit numbers have a quotient that is
 // either an fp32 number or further than 2^-36 (relative) from every rounding boundary of fp32, so the hardware reciprocal
 // (1 unit) with one correction by the exact remainder (relative error 2^-44 before its rounding) gives the bits of the IEEE
-// division in 5 instructions; column scales outside [2^-30, 2^30) and fp32 tensors divide.
-template <int DT, bool FAST> AMCT_DEV void divide_cols(float* d, const float* c) {
-    constexpr int VEC = Tr<DT>::VEC;
+// division; waves with a column factor outside [2^-30, 2^30) and fp32 tensors divide.
+template <int DT, bool FAST> AMCT_DEV bool col_reciprocals(const float* c, float* yc) {
     if constexpr (FAST && DT != AMCT_F32) {
-        uint32_t lo = __float_as_uint(c[0]), hi = lo;       // (a negative scale is large as an unsigned number)
+        constexpr int VEC = Tr<DT>::VEC;
+        uint32_t lo = __float_as_uint(c[0]), hi = lo;       // (a negative factor is large as an unsigned number)
 #pragma unroll
-        for (int j = 1; j < VEC; ++j) {
+        for (int j = 0; j < VEC; ++j) {
             lo = min(lo, __float_as_uint(c[j]));
             hi = max(hi, __float_as_uint(c[j]));
+            yc[j] = __builtin_amdgcn_rcpf(c[j]);
         }
-        if (wave_all(lo >= (97u << 23) && hi < (157u << 23))) {
+        return wave_all(lo >= (97u << 23) && hi < (157u << 23));
+    }
+    return false;
+}
+template <int DT> AMCT_DEV void divide_cols(float* d, const float* c, const float* yc, bool by_reciprocal) {
+    constexpr int VEC = Tr<DT>::VEC;
+    if (by_reciprocal) {
 #pragma unroll
-            for (int j = 0; j < VEC; ++j) {
-                const float n = round_to<DT>(d[j]);
-                const float y = __builtin_amdgcn_rcpf(c[j]);
-                const float q0 = n * y;
-                const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, c[j], n), y, q0);
-                d[j] = __uint_as_float((__float_as_uint(q1) & 0x7FFFFFFFu) | (__float_as_uint(n) & 0x80000000u));
-            }
-            return;
+        for (int j = 0; j < VEC; ++j) {
+            const float n = round_to<DT>(d[j]);
+            const float q0 = n * yc[j];
+            const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, c[j], n), yc[j], q0);
+            d[j] = __uint_as_float((__float_as_uint(q1) & 0x7FFFFFFFu) | (__float_as_uint(n) & 0x80000000u));
         }
+        return;
     }
 #pragma unroll
     for (int j = 0; j < VEC; ++j) d[j] = round_to<DT>(d[j]) / c[j];
@@ -137,7 +142,20 @@ __global__ __launch_bounds__(kBlock) void fq_fused(FqArgs a) {
     const int team = tid / T, lt = tid % T;
     const int S = a.seg_len / VEC;
     const bool asym = !a.symmetric;
-    const int64_t seg0 = ((int64_t)blockIdx.x * TEAMS + team) * U;
+    // The U segments of a team: consecutive ones, or with column factors (COL) the same columns of U consecutive rows, so
+    // that a team fetches, unpacks and inverts the factors of its columns once for all of them.
+    const int64_t tm = (int64_t)blockIdx.x * TEAMS + team;
+    int64_t seg0 = tm * U, sstep = 1, last_u = a.nseg - seg0;       // segment u < last_u exists: seg0 + u * sstep
+    int64_t col0 = 0;                                               // COL: first column of the team's segments
+    if constexpr (COL) {
+        const int64_t spr = a.segs_per_row, teams = (a.rows + U - 1) / U * spr, t = tm < teams ? tm : teams - 1;
+        // (64-bit divisions only where the number of segments needs them)
+        const int64_t rq = a.nseg <= 0x7FFFFFFF ? (int64_t)((uint32_t)t / (uint32_t)spr) : t / spr;
+        seg0 = rq * U * spr + (t - rq * spr);
+        sstep = spr;
+        last_u = tm < teams ? a.rows - rq * U : 0;
+        col0 = (t - rq * spr) * a.seg_len;
+    }
 
     float x[U][NV][VEC];
     int64_t segc[U];
@@ -145,7 +163,8 @@ __global__ __launch_bounds__(kBlock) void fq_fused(FqArgs a) {
         uint4 raw[U][NV];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            segc[u] = (seg0 + u < a.nseg) ? seg0 + u : a.nseg - 1;
+            if constexpr (COL) segc[u] = seg0 + (u == 0 || u < last_u ? u : 0) * sstep;
+            else segc[u] = u < last_u ? seg0 + u : a.nseg - 1;
 #pragma unroll
             for (int i = 0; i < NV; ++i) {
                 const int v = (i * T + lt < S) ? i * T + lt : S - 1;
@@ -157,40 +176,37 @@ __global__ __launch_bounds__(kBlock) void fq_fused(FqArgs a) {
 #pragma unroll
             for (int i = 0; i < NV; ++i) unpack16<DT>(raw[u][i], x[u][i]);
     }
-    // first column of each segment: one remainder per team, in 32 bits where the segment count allows it.  All the column
-    // factors are asked for together and, where they fit (kKeepCol), stay in registers for the division at the end: fetched
-    // vector by vector, twice, they this kernel waited for each (W[4096,4096] bf16 in groups of 128: 25.9 us, now 21.8, bound by its instructions)
-    int64_t col0[U];
-    uint4 craw[COL ? U : 1][COL ? NV : 1];
-    constexpr bool kKeepCol = U * NV <= 8;
-    if constexpr (COL) {
-        const uint32_t spr = (uint32_t)a.segs_per_row;
-        uint32_t sg = a.nseg <= 0xFFFFFFFFll ? (uint32_t)segc[0] % spr : (uint32_t)(segc[0] % spr);
-        col0[0] = (int64_t)sg * a.seg_len;
+    // Fetched vector by vector and segment by segment, before and behind the quantiser, this kernel waited for each of its
+    // column factors, and inverted every one four times: W[4096,4096] bf16 in groups of 128 22.8 us back to back, now 18.0;
+    // groups of 32 26.9, now 18.6; W[2048,14336] 37.3, now 28.9.  Bound by its instructions: without column factors 13.8.
+    // (Rows that a team has one of at a time share nothing, and fill the registers by themselves: vector by vector as before.)
+    constexpr bool kKeepCol = COL && U > 1;
+    uint4 craw[kKeepCol ? NV : 1];
+    auto col_vec = [&](int i) {
+        const int v = (i * T + lt < S) ? i * T + lt : S - 1;
+        return ldg16(reinterpret_cast<const char*>(a.col) + (col0 + (int64_t)v * VEC) * BYTES);
+    };
+    if constexpr (kKeepCol) {
 #pragma unroll
-        for (int u = 1; u < U; ++u) {
-            if (segc[u] != segc[u - 1]) sg = sg + 1 == spr ? 0 : sg + 1;
-            col0[u] = (int64_t)sg * a.seg_len;
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int i = 0; i < NV; ++i) {
-                const int v = (i * T + lt < S) ? i * T + lt : S - 1;
-                craw[u][i] = ldg16(reinterpret_cast<const char*>(a.col) + (col0[u] + (int64_t)v * VEC) * BYTES);
-            }
+        for (int i = 0; i < NV; ++i) craw[i] = col_vec(i);
         auto pre = [&](int mode) {
 #pragma unroll
-            for (int u = 0; u < U; ++u)
+            for (int i = 0; i < NV; ++i) {
+                float c[VEC];
+                unpack16<DT>(craw[i], c);
 #pragma unroll
-                for (int i = 0; i < NV; ++i) {
-                    float c[VEC];
-                    unpack16<DT>(craw[u][i], c);
-                    apply_col_pre<DT>(x[u][i], c, mode);
-                }
+                for (int u = 0; u < U; ++u) apply_col_pre<DT>(x[u][i], c, mode);
+            }
         };
         if (a.col_mode == AMCT_COL_DIV) pre(AMCT_COL_DIV);
         else pre(AMCT_COL_MUL);
+    } else if constexpr (COL) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            float c[VEC];
+            unpack16<DT>(col_vec(i), c);
+            apply_col_pre<DT>(x[0][i], c, a.col_mode);
+        }
     }
 
     float mx[U], mn[U];
@@ -243,9 +259,10 @@ __global__ __launch_bounds__(kBlock) void fq_fused(FqArgs a) {
         const Divisor dmy = divisor_of(f);
         const uint32_t big = max(__float_as_uint(mx_my) & 0x7FFFFFFFu, __float_as_uint(mn_my) & 0x7FFFFFFFu);
         fast = wave_all(dmy.fast && big < 0x5D800000u);
-        if (lt < 4 && seg0 + my < a.nseg) {
-            a.scale[seg0 + my] = f.s;
-            if (a.offset) a.offset[seg0 + my] = (int32_t)f.z;
+        if (lt < 4 && my < last_u) {
+            const int64_t at = seg0 + my * sstep;
+            a.scale[at] = f.s;
+            if (a.offset) a.offset[at] = (int32_t)f.z;
             if (f.bad && a.bad) atomicAdd(a.bad, 1);
         }
         dv[0].s = quad_bcast<0>(f.s); dv[0].y = quad_bcast<0>(dmy.y); z[0] = quad_bcast<0>(f.z);
@@ -261,9 +278,10 @@ __global__ __launch_bounds__(kBlock) void fq_fused(FqArgs a) {
             z[u] = f.z;
             const uint32_t big = max(__float_as_uint(mx[u]) & 0x7FFFFFFFu, __float_as_uint(mn[u]) & 0x7FFFFFFFu);
             ok = ok && dv[u].fast && big < 0x5D800000u;
-            if (lt == 0 && seg0 + u < a.nseg) {
-                a.scale[seg0 + u] = f.s;
-                if (a.offset) a.offset[seg0 + u] = (int32_t)f.z;
+            if (lt == 0 && u < last_u) {
+                const int64_t at = seg0 + u * sstep;
+                a.scale[at] = f.s;
+                if (a.offset) a.offset[at] = (int32_t)f.z;
                 if (f.bad && a.bad) atomicAdd(a.bad, 1);
             }
         }
@@ -273,26 +291,36 @@ __global__ __launch_bounds__(kBlock) void fq_fused(FqArgs a) {
     auto emit = [&](auto fast_tag) {
         constexpr bool FAST = decltype(fast_tag)::value;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const bool ok = seg0 + u < a.nseg;
+        for (int i = 0; i < NV; ++i) {
+            const int v = i * T + lt;
+            float c[VEC], yc[VEC];
+            bool by_reciprocal = false;
+            const bool then_div = COL && a.col_mode == AMCT_COL_MUL_THEN_DIV;
+            if constexpr (kKeepCol) {
+                if (then_div) {
+                    unpack16<DT>(craw[i], c);
+                    by_reciprocal = col_reciprocals<DT, FAST>(c, yc);
+                }
+            }
 #pragma unroll
-            for (int i = 0; i < NV; ++i) {
-                const int v = i * T + lt;
+            for (int u = 0; u < U; ++u) {
                 float q[VEC], d[VEC];
 #pragma unroll
                 for (int j = 0; j < VEC; ++j) {
                     q[j] = quant_elem<DT, VIA_SRC, FAST>(x[u][i][j], dv[u], z[u], asym, a.qmin, a.qmax);
                     d[j] = dequant_elem(q[j], dv[u].s, z[u], asym);
                 }
-                if (ok && v < S) {
-                    const int64_t e0 = (seg0 + u) * a.seg_len + (int64_t)v * VEC;
+                if (u < last_u && v < S) {
+                    const int64_t e0 = (seg0 + u * sstep) * a.seg_len + (int64_t)v * VEC;
                     if (a.codes) store_codes<DT>(a.codes, a.codes_kind, e0, q);
                     if (a.dq) {
                         if constexpr (COL) {
-                            if (a.col_mode == AMCT_COL_MUL_THEN_DIV) {
-                                float c[VEC];
-                                unpack16<DT>(kKeepCol ? craw[u][i] : ldg16(reinterpret_cast<const char*>(a.col) + (col0[u] + (int64_t)v * VEC) * BYTES), c);
-                                divide_cols<DT, FAST>(d, c);
+                            if (then_div) {
+                                if constexpr (!kKeepCol) {
+                                    unpack16<DT>(col_vec(i), c);
+                                    by_reciprocal = col_reciprocals<DT, FAST>(c, yc);
+                                }
+                                divide_cols<DT>(d, c, yc, by_reciprocal);
                             }
                         }
                         stg16_nt(reinterpret_cast<char*>(a.dq) + e0 * BYTES, pack16<DT>(d));
@@ -544,11 +572,11 @@ __global__ __launch_bounds__(kBlock) void scale_offset_k(const void* mx, const v
 template <int DT, int T, int NV, int U>
 static void launch_fused(const FqArgs& a, hipStream_t st) {
     constexpr int TEAMS = kBlock / T;
-    const int64_t per_block = (int64_t)TEAMS * U;
-    const int64_t nb = (a.nseg + per_block - 1) / per_block;
-    const dim3 grid((unsigned)nb), block(kBlock);
     const bool via = a.via_src && DT != AMCT_F32;
     const bool col = a.col_mode != AMCT_COL_NONE;
+    const int64_t teams = col ? (a.rows + U - 1) / U * a.segs_per_row : (a.nseg + U - 1) / U;
+    const int64_t nb = (teams + TEAMS - 1) / TEAMS;
+    const dim3 grid((unsigned)nb), block(kBlock);
     if (via && col) hipLaunchKernelGGL((fq_fused<DT, T, NV, U, true, true>), grid, block, 0, st, a);
     else if (via) hipLaunchKernelGGL((fq_fused<DT, T, NV, U, true, false>), grid, block, 0, st, a);
     else if (col) hipLaunchKernelGGL((fq_fused<DT, T, NV, U, false, true>), grid, block, 0, st, a);
