@@ -723,10 +723,11 @@ def linear_w8a8_dynamic(x, wq_nk, s_ch, bias=None, out_dtype=torch.bfloat16, smo
     dev = _dev(x, wq_nk, s_ch, bias, smooth)
     lib = _lib.load()
     nbytes = lib.amct_linear_w8a8_dynamic_workspace_bytes(M, N, K)
-    ws = lent_workspace(dev, nbytes)
-    if M > 0 and (ws is None or ws.numel() < nbytes):  # less than the activations may need: the two calls
-        xq, s_tok = act_quant_per_token_int8(x, smooth, mode)
-        return gemm_w8a8(xq, wq_nk, s_ch, s_tok, bias, out_dtype)
+    if workspace_limit_bytes is not None:              # the cap is on the GEMM's part, behind the activations and their scales
+        rows_bytes = (M * K + 15) // 16 * 16 + (4 * M + 15) // 16 * 16
+        nbytes = min(nbytes, rows_bytes + int(workspace_limit_bytes))
+    # of the call, not lent: the quantised activations of two captured graphs must not share memory
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
     x, wq_nk = _c(x), _c(wq_nk)
     if smooth is not None:
         smooth = _c(smooth.reshape(-1).to(x.dtype))
@@ -744,8 +745,7 @@ def linear_w8a8_dynamic(x, wq_nk, s_ch, bias=None, out_dtype=torch.bfloat16, smo
     out = torch.empty(M, N, dtype=out_dtype, device=dev)
     with _on(dev):
         _lib.check(lib.amct_linear_w8a8_dynamic(_p(x), dtype_code(x.dtype), _p(smooth), mode, _p(wq_nk), _p(s_ch), _p(bias), kind,
-                                                _p(out), M, N, K, dtype_code(out_dtype), _p(ws), 0 if ws is None else ws.numel(),
-                                                _stream(dev)))
+                                                _p(out), M, N, K, dtype_code(out_dtype), _p(ws), nbytes, _stream(dev)))
     return out
 
 
