@@ -48,10 +48,13 @@ template <int DT> AMCT_DEV void apply_col_pre(float* x, const float* c, int mode
     }
 }
 
-// d[j] <- round_to<DT>(d[j]) / c[j], every |d[j]| 0 or in [2^-60, 2^70) where FAST.  Two 16-bit numbers have a quotient that is
+// d[j] <- n / c[j] with n = round_to<DT>(d[j]); where FAST (inputs below 2^60, every scale from 2^-60) a bf16 n is 0 or in
+// [2^-60, 2^96), an fp16 n is 0, from 2^-24 on, or infinite: an asymmetric zero-point takes the extremum of a segment up to half
+// a step past itself, next to 65504 past the largest fp16 number.  Two finite 16-bit numbers have a quotient that is
 // either an fp32 number or further than 2^-36 (relative) from every rounding boundary of fp32, so the hardware reciprocal
 // (1 unit) with one correction by the exact remainder (relative error 2^-44 before its rounding) gives the bits of the IEEE
-// division; waves with a column factor outside [2^-30, 2^30) and fp32 tensors divide.
+// division; an infinite n has no remainder (inf - inf) and is its own quotient; waves with a column factor outside
+// [2^-30, 2^30) and fp32 tensors divide.
 template <int DT, bool FAST> AMCT_DEV bool col_reciprocals(const float* c, float* yc) {
     if constexpr (FAST && DT != AMCT_F32) {
         constexpr int VEC = Tr<DT>::VEC;
@@ -73,7 +76,8 @@ template <int DT> AMCT_DEV void divide_cols(float* d, const float* c, const floa
         for (int j = 0; j < VEC; ++j) {
             const float n = round_to<DT>(d[j]);
             const float q0 = n * yc[j];
-            const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, c[j], n), yc[j], q0);
+            float q1 = __builtin_fmaf(__builtin_fmaf(-q0, c[j], n), yc[j], q0);
+            if constexpr (DT == AMCT_F16) q1 = finite_f(n) ? q1 : n;
             d[j] = __uint_as_float((__float_as_uint(q1) & 0x7FFFFFFFu) | (__float_as_uint(n) & 0x80000000u));
         }
         return;

@@ -306,3 +306,25 @@ def test_column_scaled_fake_quant_of_any_shape(dev, dtype, rows, cols, group, wi
     want = iq.awq_grid_step(w, c, 'int4', strategy, False, group or None)[0]
     got, _, _, _ = ops.fakequant_int(w.to(dev), 4, False, group=group, col_scale=c.to(dev), col_mode=ops.COL_MUL_THEN_DIV, via_src=True)
     assert_bits_equal(got, want, "awq grid step")
+
+
+@pytest.mark.parametrize("sym", [False, True])
+@pytest.mark.parametrize("rows,cols,group", [(1, 32, 32), (5, 640, 128), (67, 384, 64), (9, 1536, 0), (2, 8200, 0), (3, 100, 20)])
+def test_column_scaled_fake_quant_beyond_the_largest_fp16(dev, rows, cols, group, sym):
+    """An asymmetric zero-point puts the extremum of a segment up to half a step beyond itself: next to 65504 the dequantised
+    product rounds to infinity in fp16, which the division by the column factor keeps (in the vector kernels and, for groups
+    of 20 columns, in the general one)."""
+    g = torch.Generator().manual_seed(rows + cols)
+    c = 0.5 + 199 * torch.rand(1, cols, generator=g)
+    w = (torch.randn(rows, cols, generator=g) * 50).clamp(-200, 200)
+    step = group or cols
+    for i, at in enumerate(range(0, cols, step)):
+        far, near = (0, 1) if i % 2 else (1, step - 1)
+        c[0, at + far] = c[0, at + near] = 200.
+        sign = 1. if i % 3 else -1.
+        w[:, at + far], w[:, at + near] = sign * 327.5, sign * -310.   # products 65504 and -62000: 8500 a step at 4 bits
+    w, c = w.half(), c.half()
+    want = iq.awq_grid_step(w, c, 'int4', 'group' if group else 'channel', sym, group or None)[0]
+    assert sym or bool(want.isinf().any()) and not bool(want.isnan().any())
+    got, _, _, _ = ops.fakequant_int(w.to(dev), 4, sym, group=group, col_scale=c.to(dev), col_mode=ops.COL_MUL_THEN_DIV, via_src=True)
+    assert_bits_equal(got, want, "awq grid step")
