@@ -68,11 +68,12 @@ def gptq_block(weight_sorted, i1, i2, hinv, scale_w, offset_w, gidx, qmin, qmax)
 
 def _read_later(flag):
     """(host copy of a device flag, event behind the copy): read the copy after event.synchronize(), which waits for the
-    work up to here and not for what is enqueued behind it."""
+    work up to here and not for what is enqueued behind it.  The copy runs on the current stream of the flag's device, which
+    need not be the current device: the event is recorded there."""
     host = torch.empty(flag.shape, dtype=flag.dtype, pin_memory=True)
     host.copy_(flag, non_blocking=True)
     event = torch.cuda.Event()
-    event.record()
+    event.record(torch.cuda.current_stream(flag.device))
     return host, event
 
 

@@ -187,3 +187,22 @@ def test_weight_rounding_queries_answer_without_a_gpu():
     # what the GEMM entry points reject, the queries reject
     assert q4(16, 0, 4096, 128, _lib.BF16, 0) < 0 and q4(16, 64, 4096, 0, _lib.BF16, 0) < 0
     assert q4(16, 64, 4096, 128, _lib.F32, 0) < 0 and q8(16, 64, 4096, 128, _lib.F32, 0) < 0
+
+
+def test_event_behind_a_flag_copy_is_recorded_on_the_stream_of_the_copy(monkeypatch):
+    """A layer may live on another device than the current one: an event on the current device's stream would be done
+    before the copy that it is meant to follow."""
+    from types import SimpleNamespace
+    from amct_amd.quantize_op import gptq
+    done = []
+
+    class Event:
+        def record(self, stream='the stream of the current device'):
+            done.append(stream)
+
+    host = SimpleNamespace(copy_=lambda flag, non_blocking: done.append('copy'))
+    monkeypatch.setattr(gptq, 'torch', SimpleNamespace(
+        empty=lambda shape, dtype, pin_memory: host,
+        cuda=SimpleNamespace(Event=Event, current_stream=lambda device=None: ('stream of', device))))
+    got, _ = gptq._read_later(SimpleNamespace(shape=(2,), dtype=torch.int32, device='cuda:1'))
+    assert got is host and done == ['copy', ('stream of', 'cuda:1')]

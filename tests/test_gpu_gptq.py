@@ -217,3 +217,33 @@ def test_hessian_update_reports_what_is_not_finite(dev, cols, where):
     for _ in range(2):
         ops.hessian_update(h, x, 0.5, 0.5, bad)
         assert int(bad) == int(where is not None) == int(not bool(torch.isfinite(h).all()))
+
+
+@pytest.mark.parametrize("columns", [64, 300])
+@pytest.mark.parametrize("sym", [False, True])
+def test_gptq_whole_routine_raises_what_the_kernels_report(dev, columns, sym):
+    """The flags of the factors and of the factorisation are read behind everything that is enqueued (several blocks of
+    columns at 300): each raises the error of its own, the factors' first, and a valid layer raises none."""
+    g = torch.Generator().manual_seed(columns)
+    w = torch.randn(24, columns, generator=g) * 0.05
+    x = torch.randn(3 * columns, columns, generator=g)
+    hess = (x.t() @ x).div(x.shape[0]).to(dev)
+    cfg = {'weights_cfg': {'quant_type': 'int4', 'symmetric': sym, 'strategy': 'channel'}}
+    spoilt = []
+    for value in (float('inf'), float('nan')):
+        spoilt.append(w.clone())
+        spoilt[-1][7, columns - 1] = value
+    indefinite = hess.clone()
+    indefinite[3, columns - 2] = indefinite[columns - 2, 3] = 50.
+    with_nan = hess.clone()
+    with_nan[columns // 2, columns // 2] = float('nan')
+    for _ in range(2):
+        for bad in spoilt:
+            for h in (hess, indefinite):
+                with pytest.raises(RuntimeError, match="Param scale has invalid value inf, nan or zeros!"):
+                    gptq.get_opt_weight_and_quant_factor(bad.to(dev), h, cfg)
+        for h in (indefinite, with_nan):
+            with pytest.raises(torch.linalg.LinAlgError, match="not positive-definite"):
+                gptq.get_opt_weight_and_quant_factor(w.to(dev), h, cfg)
+        got = gptq.get_opt_weight_and_quant_factor(w.to(dev), hess, cfg)[0]
+        assert bool(torch.isfinite(got).all())
