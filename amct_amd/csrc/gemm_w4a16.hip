@@ -1942,11 +1942,12 @@ static int two_pass(const void* x, const void* smooth, const uint8_t* wq, const 
 // of K slices of the launch.  K is split over blocks when the tiles alone would leave CUs idle (few output columns, long
 // rows: the down projection of an MLP) or when a row has more groups than the kernel's factor table holds; a slice is
 // at least 2048 elements.  max_rounds: 1 = only launches whose 128x128 blocks run at once; 2 = the rule for int8 weights below.
+// square: long slices may move onto 128x128 blocks, which want twice the partial sums.
 struct SpecPlan {
     int shape;
     int splits;
 };
-static SpecPlan spec_plan(int64_t M, int64_t N, int64_t K, int group, int64_t cus, int max_rounds) {
+static SpecPlan spec_plan(int64_t M, int64_t N, int64_t K, int group, int64_t cus, int max_rounds, bool square = true) {
     SpecPlan p{0, 1};
     if (M <= 0 || cus <= 0 || K % 256 != 0 || K >= 65536 || group % 64 != 0 || group <= 0 || K % group != 0) return p;
     const int64_t mt = (M + 127) / 128, nt64 = (N + 63) / 64, nt128 = (N + 127) / 128;
@@ -1981,7 +1982,7 @@ static SpecPlan spec_plan(int64_t M, int64_t N, int64_t K, int group, int64_t cu
     // by half as many blocks) and there are half as many steps; the partial sums double.  K = 11008 / 14336, 128x64 -> 128x128:
     // int8 W[4096, K] at 200 rows 43.3 -> 39.6 / 54.1 -> 47.2 us, int4 48.4 -> 39.3 us, W[2048, K] at 300 rows 40.5 -> 36.7 /
     // 50.9 -> 39.9 us (slices of 5504 / 7168); with slices of 2752 and 3584 the other way round (80 rows: 28.6 -> 30.8 us).
-    if (p.shape == 4 && S > 1 && K / S > 4096) {
+    if (square && p.shape == 4 && S > 1 && K / S > 4096) {
         const int64_t S1 = slices(mt * nt128);
         if (S1 > S && S1 <= 8) p.shape = 1, S = S1;
     }
@@ -2009,8 +2010,14 @@ static int spec_launch(const void* x, const void* smooth, const uint8_t* wq, con
     const size_t xs_bytes = smooth ? (size_t)(M * K * 2) : 0;
     const bool ws_ok = workspace && aligned16(workspace);
     if (smooth && !(ws_ok && workspace_bytes >= xs_bytes && aligned16(smooth))) return AMCT_E_UNSUPPORTED;
-    if (p.splits > 1 && !(ws_ok && workspace_bytes >= xs_bytes + spec_part_bytes(p, M, N) && (!bias || aligned16(bias)))) {
-        // no room for the partial sums: the unsplit launch, if the factor table allows it
+    const auto fits = [&](const SpecPlan& q) {
+        return q.splits == 1 || (ws_ok && workspace_bytes >= xs_bytes + spec_part_bytes(q, M, N) && (!bias || aligned16(bias)));
+    };
+    // no room for the partial sums of the square blocks: the 128x64 blocks, which want half of them (W[4096,11008] at 200
+    // rows with room for those: int8 42.1 us, int4 38.6, unsplit on the square blocks 85.5 and 82.4)
+    if (!fits(p)) p = spec_plan(M, N, K, group, cus, max_rounds, false);
+    if (!fits(p)) {
+        // not for those either: the unsplit launch, if the factor table allows it
         if (G > kSpecMaxG) return AMCT_E_UNSUPPORTED;
         p.splits = 1;
     }

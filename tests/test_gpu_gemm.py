@@ -578,3 +578,39 @@ def test_linear_w8a8_with_live_scales_is_the_two_calls(dev, M, N, K, dtype):
     finally:
         ops.workspace_limit_bytes = old
         ops.release_workspaces()
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("scaled", [False, True])
+def test_split_launch_takes_the_plan_its_workspace_holds(dev, bits, scaled):
+    """K = 11008 at 200 rows of W[4096, K]: four slices on 128x128 blocks, two on 128x64 blocks where the workspace holds
+    only theirs, none below.  Which one ran shows in sums that lose 2048 small terms behind 2^20 where one slice adds both
+    (2^-12 each, 2^-5 at most at a time, against half a unit of 2^-4) and keep them where a slice ends in between."""
+    M, N, K = 200, 4096, 11008
+    big, small, total = 2.0 ** 20, 2.0 ** -12, 0.5
+    x = torch.zeros(M, K)
+    x[0::2, 0], x[0::2, 2560:4608], x[0::2, 5376] = big, small, -big       # kept by slices that end at 2560 (of four)
+    x[1::2, 2560], x[1::2, 5376:7424], x[1::2, 8192] = big, small, -big    # and at 5376 (of two or four)
+    x = x.to(torch.bfloat16).to(dev)
+    group = 256 if bits == 4 else K
+    ones = torch.ones(N, K // group, dtype=torch.bfloat16, device=dev)
+    smooth = torch.ones(K, dtype=torch.bfloat16, device=dev) if scaled else None
+    bias = torch.zeros(N + 1, device=dev)
+    if bits == 4:
+        w, z = torch.full((N, K // 2), 0x11, dtype=torch.uint8, device=dev), torch.zeros(N, K // group, dtype=torch.uint8, device=dev)
+    else:
+        w, z = torch.ones(N, K, dtype=torch.int8, device=dev), None
+    gemm = ops.gemm_w4a16 if bits == 4 else ops.gemm_w8a16
+    part, rows = M * N * 4, M * K * 2 if scaled else 0
+    old = ops.workspace_limit_bytes
+    try:
+        for limit, b, even, odd in ((None, None, total, total), (rows + 4 * part, bias[:N], total, total),
+                                    (rows + 4 * part - 16, None, 0, total), (rows + 2 * part, bias[:N], 0, total),
+                                    (rows + 2 * part - 16, None, 0, 0), (rows, None, 0, 0), (None, bias[1:], 0, 0)):
+            ops.release_workspaces()
+            ops.workspace_limit_bytes = limit
+            got = gemm(x, w, ones, z, group, smooth, b)
+            assert bool((got[0::2] == even).all()) and bool((got[1::2] == odd).all()), (limit, float(got[0, 0]), float(got[1, 0]))
+    finally:
+        ops.workspace_limit_bytes = old
+        ops.release_workspaces()
