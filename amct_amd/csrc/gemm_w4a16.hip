@@ -1947,7 +1947,7 @@ struct SpecPlan {
     int shape;
     int splits;
 };
-static SpecPlan spec_plan(int64_t M, int64_t N, int64_t K, int group, int64_t cus, int max_rounds, bool square = true) {
+static SpecPlan spec_plan(int64_t M, int64_t N, int64_t K, int group, int bits, int64_t cus, int max_rounds, bool square = true) {
     SpecPlan p{0, 1};
     if (M <= 0 || cus <= 0 || K % 256 != 0 || K >= 65536 || group % 64 != 0 || group <= 0 || K % group != 0) return p;
     const int64_t mt = (M + 127) / 128, nt64 = (N + 63) / 64, nt128 = (N + 127) / 128;
@@ -1979,10 +1979,14 @@ static SpecPlan spec_plan(int64_t M, int64_t N, int64_t K, int group, int64_t cu
     int64_t S = slices(blocks);
     // Where K is split anyway and the slices stay long, 128x128 blocks over twice the slices: a step of theirs takes 1.5
     // times a step of the 128x64 block (each weight is dequantised for the same 128 rows, each row of the activations is read
-    // by half as many blocks) and there are half as many steps; the partial sums double.  K = 11008 / 14336, 128x64 -> 128x128:
-    // int8 W[4096, K] at 200 rows 43.3 -> 39.6 / 54.1 -> 47.2 us, int4 48.4 -> 39.3 us, W[2048, K] at 300 rows 40.5 -> 36.7 /
-    // 50.9 -> 39.9 us (slices of 5504 / 7168); with slices of 2752 and 3584 the other way round (80 rows: 28.6 -> 30.8 us).
-    if (square && p.shape == 4 && S > 1 && K / S > 4096) {
+    // by half as many blocks) and there are half as many steps; the partial sums double.  The line lies where every cell
+    // measured is as fast, to the 2 % between runs, or faster (slices of the 128x64 plan; cold weights; W[8192, K] at 72 and
+    // 128 rows, W[4096, K] at 136, 200 and 256, W[2048, K] at 300, 384 and 500; 128x64 / 128x128 time of the least and the best):
+    //   int8: slices of 4224 0.99 - 1.18, 4608 1.04 - 1.21, 5504 1.02 - 1.26, 7168 1.12 - 1.32, 8192 1.17 - 1.42
+    //         (W[4096,11008] at 200 rows 41.3 -> 36.4 us); slices of 2752 and 3584 the other way round (80 rows: 28.6 -> 30.8)
+    //   int4: slices of 4224 0.93 - 1.03, 4352 0.95 - 1.04, 4608 0.97 - 1.07, 4864 0.98 - 1.06, 5120 1.02 - 1.18,
+    //         5504 1.02 - 1.15, 7168 1.05 - 1.15, 8192 1.04 - 1.20 (W[4096,11008] at 200 rows in groups of 256 37.5 -> 35.9 us)
+    if (square && p.shape == 4 && S > 1 && K / S > (bits == 8 ? 4096 : 4608)) {
         const int64_t S1 = slices(mt * nt128);
         if (S1 > S && S1 <= 8) p.shape = 1, S = S1;
     }
@@ -2003,7 +2007,7 @@ static int spec_launch(const void* x, const void* smooth, const uint8_t* wq, con
                        const float* bias, void* out, int64_t M, int64_t N, int64_t K, int group, int dtype, void* workspace,
                        size_t workspace_bytes, hipStream_t st, int max_rounds, bool only_split) {
     const int64_t G = group > 0 ? K / group : 0, cus = current_cu_count();
-    SpecPlan p = spec_plan(M, N, K, group, cus, max_rounds);
+    SpecPlan p = spec_plan(M, N, K, group, WB, cus, max_rounds);
     if (!p.shape || N % 8 != 0 || !aligned16(x) || !aligned16(wq) || !aligned16(out) || (reinterpret_cast<uintptr_t>(scales) & 1u) != 0 ||
         M * K * 2 >= (int64_t(1) << 32) || N * K * WB / 8 >= (int64_t(1) << 32) || N * G * 2 >= (int64_t(1) << 32))
         return AMCT_E_UNSUPPORTED;
@@ -2015,7 +2019,7 @@ static int spec_launch(const void* x, const void* smooth, const uint8_t* wq, con
     };
     // no room for the partial sums of the square blocks: the 128x64 blocks, which want half of them (W[4096,11008] at 200
     // rows with room for those: int8 42.1 us, int4 38.6, unsplit on the square blocks 85.5 and 82.4)
-    if (!fits(p)) p = spec_plan(M, N, K, group, cus, max_rounds, false);
+    if (!fits(p)) p = spec_plan(M, N, K, group, WB, cus, max_rounds, false);
     if (!fits(p)) {
         // not for those either: the unsplit launch, if the factor table allows it
         if (G > kSpecMaxG) return AMCT_E_UNSUPPORTED;
@@ -2076,7 +2080,7 @@ int w8a16_spec_dispatch(const void* x, const void* smooth, const uint8_t* wq, co
 }
 // what that path wants lent beyond the smoothed activations: the partial sums of a split launch
 size_t w8a16_spec_part_bytes(int64_t M, int64_t N, int64_t K, int group) {
-    return spec_part_bytes(spec_plan(M, N, K, group, current_cu_count(), 2), M, N);
+    return spec_part_bytes(spec_plan(M, N, K, group, 8, current_cu_count(), 2), M, N);
 }
 
 }  // namespace amct
@@ -2088,7 +2092,7 @@ extern "C" size_t amct_gemm_w4a16_workspace_bytes(int64_t M, int64_t N, int64_t 
     const size_t two = two_pass_workspace(M, N, K, group, has_smooth);    // many rows: the dequantised weight as well
     if (two) return two;
     // tile kernels: x * smooth done once; long rows on few column blocks: the partial sums of the K slices behind it
-    const size_t part = spec_part_bytes(spec_plan(M, N, K, group, current_cu_count(), 1), M, N);
+    const size_t part = spec_part_bytes(spec_plan(M, N, K, group, 4, current_cu_count(), 1), M, N);
     const size_t tiles = (has_smooth && (M > 16 || part) ? (size_t)M * (size_t)K * 2 : 0) + part;
     const size_t stream = w4a16_stream_part_bytes(M, N, K, group);     // a few rows, K in slices: its partial sums only
     return tiles > stream ? tiles : stream;

@@ -614,3 +614,19 @@ def test_split_launch_takes_the_plan_its_workspace_holds(dev, bits, scaled):
     finally:
         ops.workspace_limit_bytes = old
         ops.release_workspaces()
+
+
+@pytest.mark.parametrize("bits,K,four", [(8, 9216, True), (4, 9216, False), (4, 9728, True)])
+def test_line_of_the_square_blocks(dev, bits, K, four):
+    """Two slices of 128x64 blocks become four of 128x128 blocks above 4096 columns a slice for int8 weights, above 4608 for
+    int4 ones: seen as in the test above, by a slice that ends at 2304 (of four) in front of the small terms."""
+    M, N, group = 256, 4096, K if bits == 8 else 256
+    x = torch.zeros(M, K)
+    x[:, 0], x[:, 2304:4352], x[:, K // 2] = 2.0 ** 20, 2.0 ** -12, -2.0 ** 20
+    x, ones = x.to(torch.bfloat16).to(dev), torch.ones(N, K // group, dtype=torch.bfloat16, device=dev)
+    if bits == 4:
+        got = ops.gemm_w4a16(x, torch.full((N, K // 2), 0x11, dtype=torch.uint8, device=dev), ones,
+                             torch.zeros(N, K // group, dtype=torch.uint8, device=dev), group)
+    else:
+        got = ops.gemm_w8a16(x, torch.ones(N, K, dtype=torch.int8, device=dev), ones, None, group)
+    assert bool((got == (0.5 if four else 0.)).all())
