@@ -15,7 +15,9 @@
 // goes on to factor it while the other blocks update the rest.  What bounds it is the chain of dependent pivots: 64 columns
 // take 6.8 us at 2.4 GHz, with the launch, the tile's update and the way to memory and back 12.5 us, which hide the
 // matrix products (fp32 MFMA) of the same launch once fewer than about 1000 tiles are left (20 us at 2000 tiles).
-// 4096 columns: 1.5 ms, where the library's three factorisations take 28.6 ms.
+// 4096 columns: 1.5 ms, where the library's three factorisations take 28.6 ms.  From about 8000 columns on the matrix leaves the
+// last-level cache and the sweeps over it bound the call instead (one per 64 columns, 535 MB read and written on average at
+// 14336): 8192 columns 6.9 ms, 11008 16.3, 14336 35.3 (3.4 TB/s, 56 TFLOP/s), 65600 3.1 s; the library 81, 154 and 262 ms.
 #include <algorithm>
 
 #include "amct_common.h"
@@ -32,6 +34,9 @@ constexpr int kFld = kFb + 4;                        // row stride of a tile in 
 // per thread block, up to the end of its diagonal tile.  The row of H comes in whole, in pieces of kFgRow floats through
 // LDS, and is picked apart there: picked straight from memory every element costs a 64-byte sector.
 constexpr int kFgRow = 16384;
+// Threads of a launch over half of (kFgMax / 64)^2 tiles stay below 2^32.  (A Hessian of that many columns is 256 GiB, the
+// factor and the workspace as much again each.)
+constexpr int64_t kFgMax = 262144;
 
 __global__ __launch_bounds__(kBlock) void gqf_gather_k(const float* h, const int64_t* perm, const float* damp, float* w, int64_t C,
                                                        int64_t Cp) {
@@ -301,7 +306,7 @@ extern "C" size_t amct_gptq_factor_workspace_bytes(int64_t cols) {
 extern "C" int amct_gptq_factor(const float* hessian, const int64_t* perm, const float* damp, float* u, int32_t* bad, int64_t cols,
                                 void* workspace, size_t workspace_bytes, amct_stream_t stream) {
     if (cols <= 0 || !hessian || !perm || !damp || !u || !bad || !workspace) return AMCT_E_BADARG;
-    if (cols > 65536) return AMCT_E_TOO_LARGE;       // tile counts and block ids in 32 bits
+    if (cols > kFgMax) return AMCT_E_TOO_LARGE;
     if (workspace_bytes < amct_gptq_factor_workspace_bytes(cols)) return AMCT_E_BADARG;
     if (!aligned16(workspace)) return AMCT_E_ALIGN;
     hipStream_t st = (hipStream_t)stream;

@@ -410,7 +410,7 @@ int amct_gptq_order(const void* in, void* out, const int64_t* perm, const uint8_
  * Cholesky factorisation in reversed order and one triangular inverse, all fp32).  hessian is read only; perm int64, a
  * permutation of 0 .. cols - 1; damp one fp32 on the device.  *bad (int32 on the device, zeroed by the caller) becomes 1
  * when a pivot is not positive (u is then meaningless).  workspace: amct_gptq_factor_workspace_bytes(cols), 16-byte
- * aligned.  cols <= 65536. */
+ * aligned.  cols <= 262144. */
 size_t amct_gptq_factor_workspace_bytes(int64_t cols);
 int amct_gptq_factor(const float* hessian, const int64_t* perm, const float* damp, float* u, int32_t* bad, int64_t cols,
                      void* workspace, size_t workspace_bytes, amct_stream_t stream);

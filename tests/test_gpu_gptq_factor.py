@@ -45,6 +45,39 @@ def test_factor(dev, cols):
     assert float((got @ hp @ got.t() - eye).abs().max()) <= 8 * float((theirs @ hp @ theirs.t() - eye).abs().max()) + 2.0 ** -22
 
 
+# rows of the Hessian that come in two pieces (from 16385 columns on) and in five, tile numbers beyond 2^18
+@pytest.mark.parametrize("cols", [4160, 16500, 65600])
+def test_factor_of_many_columns(dev, cols):
+    """The factor of I + V V^T in a random order, without a factorisation to compare with: u is upper triangular and u hp lower
+    triangular with the reciprocals of u's diagonal on its own, which only the factor is.  In fp64, some rows at a time."""
+    rank, step = 32, 4096
+    g = torch.Generator(device=dev).manual_seed(cols)
+    v = torch.randn(cols, rank, generator=g, device=dev) / rank ** 0.5
+    h = torch.empty(cols, cols, device=dev)
+    for i in range(0, cols, step):
+        h[i:i + step] = v[i:i + step] @ v.t()
+        h[i:i + step, i:i + step].diagonal().add_(1.)
+    perm = torch.randperm(cols, generator=g, device=dev)
+    bad = torch.zeros(1, dtype=torch.int32, device=dev)
+    u = ops.gptq_factor(h, perm, torch.full((), 0.0078125, device=dev), bad)
+    assert int(bad) == 0
+    del h
+    v = v[perm].double()
+    col = torch.arange(cols, device=dev)
+    for i in range(0, cols, step):
+        rows = u[i:i + step].double()
+        prod = (rows @ v) @ v.t() + 1.0078125 * rows
+        at = col[i:i + step, None]
+        assert not bool((rows.masked_fill(col >= at, 0) != 0).any()), "zeros below the diagonal"
+        # entries of the order of 1 in fp32: 64 units of its rounding, eight times what it measures at each of the sizes; an
+        # entry of u far from the diagonal is 5e-5 or more on average, so a lost tile is beyond it
+        assert float(prod.masked_fill(col <= at, 0).abs().max()) <= 2.0 ** -18
+        diag = rows.gather(1, at) * prod.gather(1, at)
+        assert float((diag - 1).abs().max()) <= 2.0 ** -15             # (measured: 4.6e-6 at 65600 columns)
+    del u, rows, prod
+    torch.cuda.empty_cache()
+
+
 def test_factor_of_an_indefinite_matrix_is_reported(dev):
     h = torch.eye(100)
     h[40, 41] = h[41, 40] = 3.0
