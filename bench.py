@@ -347,30 +347,28 @@ def build_cases(dev, only):
                               "static activation quantisation + W8A8 Linear M=16 in one launch (decode, config 4): bf16 x "
                               "quantised while the weight-streaming kernel stages it"))
 
-        # config 4 as the deployed module runs it with dynamic activation quantisation: K3 (per-token scales and codes
-        # of the bf16 activations) and K6 back to back on one stream, two launches per step.  (Quantising inside the
-        # GEMM would repeat K3's arithmetic in every one of the 56 / 224 blocks that share a row.)
+        # config 4 as the deployed module runs it with dynamic activation quantisation: one library call, at these sizes K3
+        # (per-token scales and codes of the bf16 activations) and K6 back to back, two launches per step.  (Quantising
+        # inside the GEMM would repeat K3's arithmetic in every one of the 56 / 224 blocks that share a row: up to 16384
+        # activations that hides behind the arriving weights and the call takes one launch.)
         for name, M6 in chain.items():
             if not want(name):
                 continue
             xb6 = x6[:M6].contiguous().to(dev)
-            xq6 = torch.empty(M6, K6, dtype=torch.int8, device=dev)
-            st6 = torch.empty(M6, dtype=torch.float32, device=dev)
+            ws6 = torch.empty(lib.amct_linear_w8a8_dynamic_workspace_bytes(M6, N6, K6), dtype=torch.uint8, device=dev)
             outs = [torch.empty(M6, N6, dtype=torch.bfloat16, device=dev) for _ in range(nw)]
 
-            def launch(i, xb6=xb6, xq6=xq6, st6=st6, outs=outs, M6=M6, wqs=wqs, swd=swd, N6=N6, K6=K6):
+            def launch(i, xb6=xb6, ws6=ws6, outs=outs, M6=M6, wqs=wqs, swd=swd, N6=N6, K6=K6):
                 j = i % len(wqs)
-                rc = lib.amct_act_quant_per_token_int8(xb6.data_ptr(), None, xq6.data_ptr(), st6.data_ptr(), M6, K6, 0, _lib.BF16, st)
-                assert rc == 0, rc
-                rc = lib.amct_gemm_w8a8(xq6.data_ptr(), wqs[j].data_ptr(), st6.data_ptr(), swd.data_ptr(), None, 0,
-                                        outs[j].data_ptr(), None, M6, N6, K6, _lib.BF16, st)
+                rc = lib.amct_linear_w8a8_dynamic(xb6.data_ptr(), _lib.BF16, None, 0, wqs[j].data_ptr(), swd.data_ptr(), None, 0,
+                                                  outs[j].data_ptr(), M6, N6, K6, _lib.BF16, ws6.data_ptr(), ws6.numel(), st)
                 assert rc == 0, rc
             if M6 >= 256:
                 cases.append(Case(name, "mfma_i8", 2 * M6 * N6 * K6, "op", launch, nw, "int8",
-                                  "dynamic per-token quantise + W8A8 Linear, M=%d, two launches (config 4 as deployed)" % M6))
+                                  "dynamic per-token quantise + W8A8 Linear, M=%d, one call of two launches (config 4 as deployed)" % M6))
             else:
                 cases.append(Case(name, "hbm", N6 * K6 + M6 * K6 * 2 + M6 * N6 * 2 + N6 * 4, "B", launch, nw, "int8",
-                                  "dynamic per-token quantise + W8A8 Linear, M=%d (decode), two launches" % M6))
+                                  "dynamic per-token quantise + W8A8 Linear, M=%d (decode), one call of two launches" % M6))
 
     # ---- K7: W4A16 Linear, W[14336,4096] int4 g128 ------------------------------------------------------
     if want("w4a16_m2048") or want("w4a16_m2048_fused") or want("w4a16_m16") or want("w4a16_m1"):
