@@ -1291,7 +1291,7 @@ int w8a8_stream_quant_dispatch(const void* x, int x_dtype, const void* smooth, c
                                int bias_kind, void* out, int64_t M, int64_t N, int64_t K, int out_dtype, hipStream_t st);
 int w8a8_stream_dynamic_dispatch(const void* x, int x_dtype, const void* smooth, int mode, const int8_t* wq, const float* s_ch,
                                  const void* bias, int bias_kind, void* out, int64_t M, int64_t N, int64_t K, int out_dtype,
-                                 hipStream_t st);                   // gemm_w8a8_stream.hip   // gemm_w8a8_stream.hip
+                                 hipStream_t st);                   // both: gemm_w8a8_stream.hip
 }
 
 // the int8 activations of the two-kernel form (rounded up to 16 bytes), then what the GEMM asks for

@@ -30,7 +30,8 @@ typedef float f4v __attribute__((ext_vector_type(4)));
 constexpr int kFb = 64;                              // columns eliminated per step
 constexpr int kFld = kFb + 4;                        // row stride of a tile in LDS, in floats: 16 rows apart meet no bank
 
-// W = J (H with zero diagonal entries set to 1, rows and columns in the order perm, + damp I) J, identity beyond C; one row
+// W = J (H with zero diagonal entries set to 1, rows and columns in the order perm, + damp I) J, identity beyond C (of each
+// pair H[a][b] = H[b][a] the row of the one that comes later in the reversed order is read); one row
 // per thread block, up to the end of its diagonal tile.  The row of H comes in whole, in pieces of kFgRow floats through
 // LDS, and is picked apart there: picked straight from memory every element costs a 64-byte sector.
 constexpr int kFgRow = 16384;

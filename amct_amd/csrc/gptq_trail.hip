@@ -10,7 +10,7 @@
 // (71 TFLOP/s; the register-only loop reaches 150), 32.0 for 2048, 9.4 for 256; the library's product and subtraction
 // 87, 42, 28.  128 x 64 because the trailing part shrinks to nothing over the blocks of a layer: 64-row tiles read half as
 // much again from L2, 128-column tiles leave CUs idle earlier.
-// gptq_order_k: W[4096,4096] bf16, 19 us there and 23 back (indexing with the conversions around it 150 and 130).
+// gptq_order_k: W[4096,4096] bf16, 21 us there and 22 back (indexing with the conversions around it 150 and 130).
 #include "amct_common.h"
 
 namespace amct {

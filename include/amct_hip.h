@@ -371,7 +371,8 @@ int amct_gemm_w8a16(const void* x, const void* smooth, const int8_t* wq, const v
  * the query asks for M * K * 2 bytes: the multiply is then done once up front and the fast tile kernels apply (K a
  * multiple of 256, groups a multiple of 64; they take precedence up to 384 rows, and up to 512 rows unless a last round
  * of 128x128 blocks would run half empty; for long rows on few column blocks with K split over blocks, whose fp32 partial sums follow the
- * activations in the workspace: S * M * N * 4 bytes more).  0 bytes are asked for otherwise; a null or smaller workspace
+ * activations in the workspace: S * M * N * 4 bytes more, or a workspace for half of them where slices are long: S / 2 slices on
+ * smaller blocks).  0 bytes are asked for otherwise; a null or smaller workspace
  * is never an error. */
 size_t amct_gemm_w8a16_workspace_bytes(int64_t M, int64_t N, int64_t K, int group, int has_smooth);
 int amct_gemm_w8a16_ws(const void* x, const void* smooth, const int8_t* wq, const void* scales, int scale_dtype,
@@ -407,7 +408,8 @@ int amct_gptq_order(const void* in, void* out, const int64_t* perm, const uint8_
  * The three factorisations of amct_pytorch/quantize_op/gptq_module.py:108-121 as one: with Hp = hessian[perm][:, perm],
  * zero diagonal entries replaced by 1 and *damp added to the diagonal, u [cols, cols] = the upper triangular factor with
  * Hp^-1 = u^T u, zeros below the diagonal (the reference's cholesky(cholesky_inverse(cholesky(Hp)), upper=True), from one
- * Cholesky factorisation in reversed order and one triangular inverse, all fp32).  hessian is read only; perm int64, a
+ * Cholesky factorisation in reversed order and one triangular inverse, all fp32).  hessian is read only and taken to be
+ * symmetric: one entry of every pair is read; perm int64, a
  * permutation of 0 .. cols - 1; damp one fp32 on the device.  *bad (int32 on the device, zeroed by the caller) becomes 1
  * when a pivot is not positive (u is then meaningless).  workspace: amct_gptq_factor_workspace_bytes(cols), 16-byte
  * aligned.  cols <= 262144. */
