@@ -6,111 +6,105 @@
 // product of the 16-bit inputs is the reference's fp32 product up to the order of the sum; the factor 2 / n is
 // applied once to the sum instead of sqrt(2 / n) to every element.
 //
-// Two kernels.  hess_transpose_k writes X^T, zero-padded to whole tiles, into the caller's workspace ([Cp, Tp], K
-// contiguous), so that both MFMA operands are rows of one matrix.  hess_syrk_k owns one 128 x 128 tile of the lower
-// triangle: 4 waves of 64 x 64 (2 x 2 MFMA 32x32x16), 64 tokens per step, one LDS stage (16-byte chunks of a row
-// swizzled by the row so that fragment reads spread over the banks; the next step waits in registers), two barriers
-// per step.  The epilogue reads the
-// tile of H, applies beta and alpha, writes the tile and -- through LDS, as whole 256-byte rows -- its mirror image, so H
-// stays exactly symmetric and only its lower triangle is ever read.  It also notes whether everything it wrote is finite:
-// as five library passes over H that check took as long as the update itself (75 us at 4096 columns).
+// hess_syrk_k owns one square tile of the lower triangle and reads X as it lies in memory, tokens by columns: a step of 64
+// tokens of the tile's two column ranges goes to LDS by direct-to-LDS loads, and the transposing LDS read
+// (ds_read_b64_tr_b16: of a block of 4 tokens x 16 columns, lane i gets the 4 tokens of column i) makes MFMA operands of it.
+// Two or three stages of LDS, one barrier per step; the fragments of the second half of a step are read under the products of
+// the first half, those of the next step under the products of the second.
+// A tile is 64, 128 or 192 columns wide, 2 x 2 waves of half that: see hs_width.  The epilogue
+// applies beta and alpha, writes the tile and its mirror image, so H stays exactly symmetric, and notes whether everything
+// it wrote is finite: as library passes over H that check took as long as the update itself (75 us at 4096 columns).
+// X[2048,4096] bf16 into an empty / a running H[4096,4096]: 50 / 54 us (1 PFLOP/s on the 253 tiles), where 128-column tiles fed by a
+// kernel that transposed X first took 75 / 82; 512 columns 12.9 / 13.2 (39 / 40), 2816 30 / 31 (50 / 53), 11008 293 / 348 (350 / 404).
+// At 4096 columns the products take 33 us (21 at the rate of a register-only loop, 8 more are the loads' and LDS's), the
+// rest is the launch and H itself, 64 MB written and half of it read, all tiles at the same time.
+#include <type_traits>
+
 #include "amct_common.h"
 
 namespace amct {
 
-typedef float h16f __attribute__((ext_vector_type(16)));
+typedef float h4f __attribute__((ext_vector_type(4)));
 typedef __bf16 h8bf __attribute__((ext_vector_type(8)));
 typedef _Float16 h8h __attribute__((ext_vector_type(8)));
+typedef short h4s __attribute__((ext_vector_type(4)));
+typedef short h8s __attribute__((ext_vector_type(8)));
 
-constexpr int kHsTile = 128;                         // rows / columns of H per block
-constexpr int kHsK = 64;                             // tokens per step (128 bytes of a row of X^T)
+constexpr int kHsK = 64;                             // tokens per step
 
-// X [T, C] -> Xt [Cp, Tp], zeros beyond T and C.  64 x 64 tiles through LDS.
-__global__ __launch_bounds__(kBlock) void hess_transpose_k(const uint16_t* x, uint16_t* xt, int64_t T, int64_t C, int64_t Tp, int32_t* bad) {
-    __shared__ uint16_t tile[64][66];
-    const int tid = threadIdx.x;
-    const int64_t c0 = (int64_t)blockIdx.x * 64, t0 = (int64_t)blockIdx.y * 64;
-    if (bad && blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) *bad = 0;      // before the kernel that may set it
-    {
-        const int c = tid & 63;
+// X [T, C] -> [T, ld], columns beyond C zero: rows that start 16-byte aligned, where those of X do not.
+__global__ __launch_bounds__(kBlock) void hess_align_k(const uint16_t* x, uint16_t* xa, int64_t T, int64_t C, int64_t ld) {
+    const int64_t c = ((int64_t)blockIdx.x * kBlock + threadIdx.x) * 8;
+    if (c >= ld) return;
+    for (int64_t t = blockIdx.y; t < T; t += gridDim.y) {
+        uint16_t v[8];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int t = (tid >> 6) + 4 * i;
-            uint16_t v = 0;
-            if (t0 + t < T && c0 + c < C) v = x[(t0 + t) * C + c0 + c];
-            tile[t][c] = v;
-        }
-    }
-    __syncthreads();
-    {
-        const int t = tid & 63;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int c = (tid >> 6) + 4 * i;
-            xt[(c0 + c) * Tp + t0 + t] = tile[t][c];      // c0 + c < Cp and t0 + t < Tp by the grid
-        }
+        for (int j = 0; j < 8; ++j) v[j] = c + j < C ? x[t * C + c + j] : (uint16_t)0;
+        uint4 q;
+        q.x = v[0] | (uint32_t)v[1] << 16;
+        q.y = v[2] | (uint32_t)v[3] << 16;
+        q.z = v[4] | (uint32_t)v[5] << 16;
+        q.w = v[6] | (uint32_t)v[7] << 16;
+        stg16(xa + t * ld + c, q);
     }
 }
 
-// The same for C % 8 == 0 and a 16-byte aligned x: 16-byte loads (8 columns of one token) and 16-byte stores (8
-// tokens of one column); the tile is held column-major, a column 72 tokens apart (144 bytes: 16-byte aligned rows whose
-// 16-byte reads by 8 lanes of consecutive columns fall into different banks).
-__global__ __launch_bounds__(kBlock) void hess_transpose_vec_k(const uint16_t* x, uint16_t* xt, int64_t T, int64_t C, int64_t Tp, int32_t* bad) {
-    __shared__ __align__(16) uint16_t tile[64][72];                           // [column][token]
-    const int tid = threadIdx.x;
-    const int64_t c0 = (int64_t)blockIdx.x * 64, t0 = (int64_t)blockIdx.y * 64;
-    if (bad && blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) *bad = 0;      // before the kernel that may set it
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int v = tid + 256 * i;                                          // 512 vectors: token v / 8, columns 8 (v % 8) ..
-        const int t = v >> 3, cv = (v & 7) * 8;
-        uint4 q = make_uint4(0, 0, 0, 0);
-        if (t0 + t < T && c0 + cv < C) q = ldg16_nt(x + (t0 + t) * C + c0 + cv);
-        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            tile[cv + 2 * j][t] = (uint16_t)(w[j] & 0xFFFFu);
-            tile[cv + 2 * j + 1][t] = (uint16_t)(w[j] >> 16);
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int v = tid + 256 * i;                                          // column v / 8, tokens 8 (v % 8) ..
-        const int c = v >> 3, tv = (v & 7) * 8;
-        const uint4 q = *reinterpret_cast<const uint4*>(&tile[c][tv]);
-        stg16(xt + (c0 + c) * Tp + t0 + tv, q);                               // inside [Cp, Tp] by the grid
-    }
-}
+__global__ void hess_clear_k(int32_t* bad) { *bad = 0; }
 
 struct SyrkArgs {
-    const uint16_t* xt;                              // [Cp, Tp]
+    const uint16_t* x;                               // [T, ld], rows 16-byte aligned
     float* h;                                        // [C, C]
-    int64_t C, Tp;
+    int64_t T, C, ld;
     int nb;                                          // tiles per side
     int per_die;                                     // tiles of the lower triangle per die (rounded up)
     int64_t ntiles;                                  // nb (nb + 1) / 2
     float beta, alpha;
+    int vec;                                         // rows of H are 16-byte aligned
     int32_t* bad;                                    // set where an element of the new H is not finite, or null
 };
 
 template <bool F16>
-AMCT_DEV h16f hs_mfma(const uint4& a, const uint4& b, const h16f& c) {
-    if constexpr (F16) return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8h, a), __builtin_bit_cast(h8h, b), c, 0, 0, 0);
-    else return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(h8bf, a), __builtin_bit_cast(h8bf, b), c, 0, 0, 0);
+AMCT_DEV h4f hs_mfma(const h8s& a, const h8s& b, const h4f& c) {
+    if constexpr (F16) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8h, a), __builtin_bit_cast(h8h, b), c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(h8bf, a), __builtin_bit_cast(h8bf, b), c, 0, 0, 0);
 }
 
-template <bool F16>
-__global__ __launch_bounds__(kBlock, 3) void hess_syrk_k(SyrkArgs a) {
-    // one stage: two operands x 128 rows x 128 bytes = 32 KB (the next step waits in registers); the epilogue reuses it as
-    // four 64 x 32 fp32 patches.  Three blocks fit a CU.
+// A direct-to-LDS load: wave-uniform 64-bit base, a byte offset per lane, lane l's 16 bytes land at lds + 16 l.  (Inline, with
+// hand-counted waits: the compiler would wait for all of them before every LDS read.)
+AMCT_DEV void hs_dma(uint32_t lds, const void* base, uint32_t off) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(off), "s"(base) : "memory");
+}
+template <int N> AMCT_DEV void hs_wait() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory"); }
+AMCT_DEV void hs_meet() {
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// W: 16-column tiles per side of a wave (2, 4 or 6); the block's tile is 32 W columns wide.  128-column tiles take two stages so
+// that two blocks fit a CU, and one's epilogue runs under the other's products: X[2048,11008] 293 us, with three stages and
+// one block 381.
+template <int W> struct SyrkShape {
+    static constexpr int kTile = 32 * W;
+    static constexpr int kRow = 2 * kTile;           // bytes of a token in LDS
+    static constexpr int kOperand = kHsK * kRow;
+    static constexpr int kStage = 2 * kOperand;
+    static constexpr int kStages = W == 4 ? 2 : 3;
+    static constexpr int kLds = kStages * kStage;
+    static constexpr int kPerCu = 160 * 1024 / kLds;
+    static_assert(W == 2 || W == 4 || W == 6, "the swaps of LDS units below are for these");
+    static_assert(kLds >= 4 * (16 * W) * (16 * W) * 4, "the epilogue's patches");
+};
+
+template <bool F16, int W>
+__global__ __launch_bounds__(kBlock, SyrkShape<W>::kPerCu) void hess_syrk_k(SyrkArgs a) {
+    using S = SyrkShape<W>;
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // block -> tile (bi, bj) of the lower triangle, bi >= bj.  The chip hands consecutive blocks to its eight dies in
     // turn, and each die has an L2 of its own: block id works on tile (id % 8) * per + id / 8 of an order in which
-    // consecutive tiles form compact patches (bands of 8 rows of tiles, inside a band column after column), so the 64
-    // blocks that a die runs at a time share 8 + 8 operand tiles instead of fetching 64 + 64.
+    // consecutive tiles form compact patches (bands of 8 rows of tiles, inside a band column after column), so the blocks
+    // that a die runs at a time share their operand tiles.
     const int per = a.per_die;
     const int64_t logical = (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if ((int)(blockIdx.x >> 3) >= per || logical >= a.ntiles) return;         // whole block (before any barrier)
@@ -133,147 +127,222 @@ __global__ __launch_bounds__(kBlock, 3) void hess_syrk_k(SyrkArgs a) {
             bi = bj + o;
         }
     }
+    bi = __builtin_amdgcn_readfirstlane(bi);         // (a square root is not scalar arithmetic)
+    bj = __builtin_amdgcn_readfirstlane(bj);
     const bool diag = bi == bj;
-    const int64_t i0 = (int64_t)bi * kHsTile, j0 = (int64_t)bj * kHsTile;
-    const int wi = wave >> 1, wj = wave & 1;         // 2 x 2 waves of 64 x 64
+    const int64_t i0 = (int64_t)bi * S::kTile, j0 = (int64_t)bj * S::kTile;
+    const int wi = wave >> 1, wj = wave & 1;         // 2 x 2 waves of 16 W x 16 W
 
-    // global -> LDS: a tile is 128 rows x 8 chunks of 16 bytes; thread t moves chunks t, t + 256, t + 512, t + 768
-    const int ld_row = tid >> 3, ld_chunk = tid & 7; // + 32 rows per repeat
-    const uint8_t* ga = reinterpret_cast<const uint8_t*>(a.xt) + ((i0 + ld_row) * a.Tp) * 2 + ld_chunk * 16;
-    const uint8_t* gb = reinterpret_cast<const uint8_t*>(a.xt) + ((j0 + ld_row) * a.Tp) * 2 + ld_chunk * 16;
-    const int64_t row_step = 32 * a.Tp * 2;          // bytes between the repeats
-    // chunk c of row r sits at c ^ ((r >> 1) & 7): LDS has 64 banks of 4 bytes, two 128-byte rows cover them once, so 16
-    // lanes reading the same logical chunk of 16 consecutive rows meet in no bank
-    const uint32_t st_off = (uint32_t)ld_row * 128u + (uint32_t)((ld_chunk ^ ((ld_row >> 1) & 7)) * 16);   // rows 32 apart: same swizzle
-    constexpr uint32_t kTileBytes = kHsTile * 128;
-
-    // fragments: lane l holds row l % 32 of a 32-row tile, chunk 2 * slice + l / 32 of the step's 128 bytes
-    const int fr = lane & 31, fh = lane >> 5;
-    uint32_t fa_off[2], fb_off[2];
+    // Memory -> LDS: per operand and step 64 tokens x 4 W chunks of 16 bytes, token after token; a wave moves W pieces of 1 KB.
+    // A fragment read takes 16 tokens x 32 bytes at a time: inside a token the 32-byte units are swapped by the token (swap), so
+    // that eight consecutive tokens' units lie in different banks (a token is 128, 256 or 384 bytes).
+    // Columns beyond C repeat the last ones of X (their sums are not stored), tokens beyond T the last one (cleared below).
+    auto swap = [](int t) { return W == 4 ? t & 7 : (t >> 1) & 3; };
+    const uint32_t row_bytes = (uint32_t)(a.ld * 2);
+    uint32_t off_a[W], off_b[W];                     // bytes from the tile's first column at the step's first token
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
-        const uint32_t ra = (uint32_t)(wi * 64 + m * 32 + fr), rb = (uint32_t)(wj * 64 + m * 32 + fr);
-        fa_off[m] = ra * 128u;
-        fb_off[m] = rb * 128u + kTileBytes;
+    for (int p = 0; p < W; ++p) {
+        const int q = (wave * W + p) * 64 + lane, t = q / (4 * W), at = q % (4 * W);
+        const int c = 8 * ((((at >> 1) ^ swap(t)) << 1) | (at & 1));
+        off_a[p] = (uint32_t)t * row_bytes + 2 * (uint32_t)(min(i0 + c, a.ld - 8) - i0);
+        off_b[p] = (uint32_t)t * row_bytes + 2 * (uint32_t)(min(j0 + c, a.ld - 8) - j0);
     }
-    const uint32_t fsw = (uint32_t)((fr >> 1) & 7);  // rows of a fragment are 64 w + 32 m + fr: the swizzle depends on fr only
-
-    h16f acc[2][2];
+    const int steps = (int)((a.T + kHsK - 1) / kHsK), last = steps - 1;
+    const int tail = (int)(a.T - (int64_t)last * kHsK);                       // tokens of the last step
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds);
+    auto fetch = [&](int stage, int step) {
+        const uint16_t* xs = a.x + (int64_t)step * kHsK * a.ld;
+        const uint32_t to = lds0 + stage * S::kStage + wave * W * 1024;
+        if (step == last && tail < kHsK) {
 #pragma unroll
-    for (int m = 0; m < 2; ++m)
-#pragma unroll
-        for (int n = 0; n < 2; ++n)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[m][n][r] = 0.f;
-
-    // (a tile on the diagonal loads its rows twice, as both operands: one block in nb + 1, and no special cases below)
-    const int steps = (int)(a.Tp / kHsK);
-    uint4 ra0, ra1, ra2, ra3, rb0, rb1, rb2, rb3;
-#define AMCT_HS_GLOAD(S)                                                                  \
-    {                                                                                     \
-        const int64_t so = (int64_t)(S) * 128;                                            \
-        ra0 = *reinterpret_cast<const uint4*>(ga + so);                                   \
-        ra1 = *reinterpret_cast<const uint4*>(ga + row_step + so);                        \
-        ra2 = *reinterpret_cast<const uint4*>(ga + 2 * row_step + so);                    \
-        ra3 = *reinterpret_cast<const uint4*>(ga + 3 * row_step + so);                    \
-        rb0 = *reinterpret_cast<const uint4*>(gb + so);                                   \
-        rb1 = *reinterpret_cast<const uint4*>(gb + row_step + so);                        \
-        rb2 = *reinterpret_cast<const uint4*>(gb + 2 * row_step + so);                    \
-        rb3 = *reinterpret_cast<const uint4*>(gb + 3 * row_step + so);                    \
-    }
-#define AMCT_HS_LSTORE()                                                                  \
-    {                                                                                     \
-        uint8_t* base = lds + st_off;                                                     \
-        *reinterpret_cast<uint4*>(base) = ra0;                                            \
-        *reinterpret_cast<uint4*>(base + 32 * 128) = ra1;                                 \
-        *reinterpret_cast<uint4*>(base + 64 * 128) = ra2;                                 \
-        *reinterpret_cast<uint4*>(base + 96 * 128) = ra3;                                 \
-        *reinterpret_cast<uint4*>(base + kTileBytes) = rb0;                               \
-        *reinterpret_cast<uint4*>(base + kTileBytes + 32 * 128) = rb1;                    \
-        *reinterpret_cast<uint4*>(base + kTileBytes + 64 * 128) = rb2;                    \
-        *reinterpret_cast<uint4*>(base + kTileBytes + 96 * 128) = rb3;                    \
-    }
-    AMCT_HS_GLOAD(0)
-    AMCT_HS_LSTORE()
-    __syncthreads();
-    for (int s = 0; s < steps; ++s) {
-        if (s + 1 < steps) AMCT_HS_GLOAD(s + 1)      // in flight during this step's MFMAs
-        const uint8_t* st = lds;
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const uint32_t ch = ((uint32_t)(2 * ks + fh) ^ fsw) * 16u;
-            uint4 fa[2], fb[2];
-#pragma unroll
-            for (int m = 0; m < 2; ++m) {
-                fa[m] = *reinterpret_cast<const uint4*>(st + fa_off[m] + ch);
-                fb[m] = *reinterpret_cast<const uint4*>(st + fb_off[m] + ch);
+            for (int p = 0; p < W; ++p) {
+                const int t = ((wave * W + p) * 64 + lane) / (4 * W);
+                const uint32_t back = t < tail ? 0u : (uint32_t)(t - tail + 1) * row_bytes;
+                hs_dma(to + p * 1024, xs + i0, off_a[p] - back);
+                hs_dma(to + p * 1024 + S::kOperand, xs + j0, off_b[p] - back);
             }
-#pragma unroll
-            for (int m = 0; m < 2; ++m)
-#pragma unroll
-                for (int n = 0; n < 2; ++n) acc[m][n] = hs_mfma<F16>(fa[m], fb[n], acc[m][n]);
+            return;
         }
-        __syncthreads();                             // everyone has read this step's tiles
-        if (s + 1 < steps) {
-            AMCT_HS_LSTORE()
-            __syncthreads();
+#pragma unroll
+        for (int p = 0; p < W; ++p) {
+            hs_dma(to + p * 1024, xs + i0, off_a[p]);
+            hs_dma(to + p * 1024 + S::kOperand, xs + j0, off_b[p]);
         }
+    };
+    // the tokens beyond T in the last step's stage, before anyone reads it
+    auto clear_tail = [&](int stage) {
+        const int z0 = tail * S::kRow / 16, z1 = S::kOperand / 16;
+        for (int z = z0 + tid; z < z1; z += kBlock) {
+            *reinterpret_cast<uint4*>(lds + stage * S::kStage + z * 16) = make_uint4(0, 0, 0, 0);
+            *reinterpret_cast<uint4*>(lds + stage * S::kStage + S::kOperand + z * 16) = make_uint4(0, 0, 0, 0);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        hs_meet();
+    };
+
+    // Fragment of 16 columns and 32 tokens: lane l holds column l % 16 and the tokens 4 (l / 16) .. + 3 and 16 more.  Both
+    // operands take the same tokens in the same places, which is all that the contraction asks for.  The lane reads
+    // 4 columns of token 4 (l / 16) + (l % 16) / 4 and is given its own column by the transposition.
+    const int tl = 4 * (lane >> 4) + ((lane & 15) >> 2);
+    int at_a[W], at_b[W];
+#pragma unroll
+    for (int m = 0; m < W; ++m) {
+        at_a[m] = tl * S::kRow + ((wi * W + m) ^ swap(tl)) * 32 + (lane & 3) * 8;
+        at_b[m] = S::kOperand + tl * S::kRow + ((wj * W + m) ^ swap(tl)) * 32 + (lane & 3) * 8;
     }
-#undef AMCT_HS_GLOAD
-#undef AMCT_HS_LSTORE
+    auto fragment = [&](int at) {
+        typedef __attribute__((address_space(3))) h4s lds_h4s;
+        const h4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_h4s*)(lds + at));
+        const h4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_h4s*)(lds + at + 16 * S::kRow));
+        return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+    h8s fa[2][W], fb[2][W];
+    // q < W: rows, else columns, of half u (32 tokens) of a stage
+    auto read_one = [&](int stage, int u, int q) {
+        const int base = stage * S::kStage + u * 32 * S::kRow;
+        if (q < W) fa[u][q] = fragment(base + at_a[q]);
+        else fb[u][q - W] = fragment(base + at_b[q - W]);
+    };
+    h4f acc[W][W];
+#pragma unroll
+    for (int m = 0; m < W; ++m)
+#pragma unroll
+        for (int n = 0; n < W; ++n) acc[m][n] = h4f{0.f, 0.f, 0.f, 0.f};
+    // the products of half u, one fragment of the next half behind every kGap-th of them; the column fragment is the first
+    // operand: a lane's four sums of tile (m, n) are H[16 m + lane % 16][16 n + 4 (lane / 16) + 0 .. 3] of the wave's tile
+    constexpr int kGap = W / 2;
+    auto products = [&](int u, bool more, int stage, int v) {
+#pragma unroll
+        for (int x = 0; x < W * W; ++x) {
+            const int m = x / W, n = x % W;
+            acc[m][n] = hs_mfma<F16>(fb[u][n], fa[u][m], acc[m][n]);
+            __builtin_amdgcn_sched_barrier(0);
+            if (more && x % kGap == 0) {
+                read_one(stage, v, x / kGap);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+
+    if (steps > 0) {
+        constexpr int kPer = 2 * W;                  // loads of a wave and stage
+        // (steps beyond the last repeat it: the counts of the waits stay the same, and nobody reads those stages)
+#pragma unroll
+        for (int s = 0; s < S::kStages; ++s) fetch(s, min(s, last));
+        hs_wait<(S::kStages - 1) * kPer>();
+        hs_meet();
+        if (last == 0 && tail < kHsK) clear_tail(0);
+#pragma unroll
+        for (int q = 0; q < 2 * W; ++q) read_one(0, 0, q);
+        int stage = 0;
+        for (int s = 0; s < last; ++s) {
+            const int next = stage + 1 == S::kStages ? 0 : stage + 1;
+            products(0, true, stage, 1);
+            hs_wait<(S::kStages - 2) * kPer>();       // the next stage is there, this one is in registers
+            hs_meet();
+            if (s + 1 == last && tail < kHsK) clear_tail(next);
+            fetch(stage, min(s + S::kStages, last));
+            products(1, true, next, 0);
+            stage = next;
+        }
+        products(0, true, stage, 1);
+        products(1, false, 0, 0);
+        hs_wait<0>();                                // no load may land after the block has given its LDS back
+    }
 
     // ---- epilogue -------------------------------------------------------------------------------------------
-    // acc[m][n][r]: row 8 (r / 4) + 4 (lane / 32) + r % 4, column lane % 32 of the 32 x 32 tile (m, n) of this wave
-    // Addresses: one block-uniform base per wave plus 32-bit lane offsets (cols < 2^22 is checked by the host), so an
-    // address costs one register and the compiler keeps none of them alive in 64 bits.
+    // The sums go through LDS, a patch per wave, so that H is read and written in whole rows of the wave's tile both ways, and
+    // by loops: unrolled over the registers it was 144 stores with their checks that every wave fetched from memory as
+    // instructions and ran once.  16-byte units of a row are swapped by the row (unit_of): 16 rows' same unit, which
+    // 16 lanes write at a time, lie in different banks.
+    hs_meet();                                       // every wave is done with the stages
+    constexpr int kRows = 16 * W, kUnits = 4 * W;    // of the patch; a unit is 4 columns
+    auto unit_of = [](int row, int u) {
+        return u ^ (W == 4 ? (row ^ (row >> 4)) & 15 : ((row >> 1) ^ (row >> 4)) & 7);
+    };
+    h4f* patch = reinterpret_cast<h4f*>(lds + wave * (S::kLds / 4));
+#pragma unroll
+    for (int m = 0; m < W; ++m)
+#pragma unroll
+        for (int n = 0; n < W; ++n) {
+            h4f v;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = a.alpha * acc[m][n][r];
+            const int row = 16 * m + (lane & 15);
+            patch[row * kUnits + unit_of(row, 4 * n + (lane >> 4))] = v;
+        }
+    // Addresses: one block-uniform base per wave plus 32-bit lane offsets (cols < 2^22 is checked by the host).
     const bool have = a.beta != 0.f;
-    float* patch = reinterpret_cast<float*>(lds) + wave * (64 * 32);          // 8 KB per wave (after the last barrier)
     const uint32_t C32 = (uint32_t)a.C;
-    const int64_t wi0 = i0 + wi * 64, wj0 = j0 + wj * 64;                     // the wave's first row and column
+    const int64_t wi0 = i0 + wi * kRows, wj0 = j0 + wj * kRows;               // the wave's first row and column
     float* hw = a.h + wi0 * a.C + wj0;                                        // H[wi0][wj0]
     float* hm = a.h + wj0 * a.C + wi0;                                        // its mirror image H[wj0][wi0]
-    const int rows_left = (int)min((int64_t)64, a.C - wi0), cols_left = (int)min((int64_t)64, a.C - wj0);   // may be <= 0
-    const uint32_t lane_off = (uint32_t)(4 * fh) * C32 + (uint32_t)fr;
+    const int rows_left = (int)min((int64_t)kRows, a.C - wi0), cols_left = (int)min((int64_t)kRows, a.C - wj0);   // may be <= 0
     bool finite = true;                              // of everything this lane writes (the mirror image repeats it)
+    // VEC: rows of H are 16-byte aligned and a lane takes four columns, which are inside H or outside together; else one.  Lanes
+    // outside read what the first lane does and write nothing: no branches between the loads, of which a lane has kBatch in
+    // flight.  (Element by element, with a branch each, the tiles at the edge of H took 25 us, and a launch waits for its
+    // slowest block.)
+    auto finish = [&](auto vec_tag) {
+        constexpr bool VEC = decltype(vec_tag)::value;
+        constexpr int V = VEC ? 4 : 1, kPieces = kRows / V, kTurns = kRows * kPieces / 64, kBatch = VEC ? 2 * W : 8;
+        static_assert(kTurns % kBatch == 0, "batches");
+        const float* pf = reinterpret_cast<const float*>(patch);
+        auto in_patch = [&](int row, int col) { return (row * kUnits + unit_of(row, col >> 2)) * 4 + (col & 3); };
+#pragma unroll 1
+        for (int b = 0; b < kTurns; b += kBatch) {
+            float old[kBatch][V];
+            if (have) {
 #pragma unroll
-    for (int n = 0; n < 2; ++n) {                    // the wave's columns 32 n .. 32 n + 31
-        const bool col_ok = n * 32 + fr < cols_left;
-        // all of the half's old values first (32 independent loads in flight; one at a time, each behind the store
-        // before it, they cost a trip to memory each), then the arithmetic and the stores
-        h16f old[2];
-#pragma unroll
-        for (int m = 0; m < 2; ++m)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = m * 32 + 8 * (r / 4) + (r % 4);               // + 4 fh
-                const uint32_t idx = lane_off + (uint32_t)row * C32 + (uint32_t)(n * 32);
-                old[m][r] = (have && col_ok && row + 4 * fh < rows_left) ? __builtin_nontemporal_load(hw + idx) : 0.f;
-            }
-#pragma unroll
-        for (int m = 0; m < 2; ++m) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = m * 32 + 8 * (r / 4) + (r % 4);
-                const int lr = row + 4 * fh;                                  // row inside the wave's 64 x 64
-                const uint32_t idx = lane_off + (uint32_t)row * C32 + (uint32_t)(n * 32);
-                float v = a.alpha * acc[m][n][r];
-                if (have) v = old[m][r] * a.beta + v;
-                if (col_ok && lr < rows_left) {
-                    hw[idx] = v;
-                    finite = finite && finite_f(v);
+                for (int x = 0; x < kBatch; ++x) {
+                    const int e = (b + x) * 64 + lane, row = e / kPieces, col = V * (e % kPieces);
+                    const float* from = hw + (row < rows_left && col < cols_left ? (uint32_t)row * C32 + (uint32_t)col : 0u);
+                    if constexpr (VEC) *reinterpret_cast<h4f*>(old[x]) = *reinterpret_cast<const h4f*>(from);
+                    else old[x][0] = *from;
                 }
-                patch[lr * 32 + (fr ^ (lr & 31))] = v;
+            }
+#pragma unroll
+            for (int x = 0; x < kBatch; ++x) {
+                const int e = (b + x) * 64 + lane, row = e / kPieces, col = V * (e % kPieces), at = in_patch(row, col);
+                float v[V];
+                if constexpr (VEC) *reinterpret_cast<h4f*>(v) = patch[at >> 2];
+                else v[0] = pf[at];
+                if (have) {
+#pragma unroll
+                    for (int r = 0; r < V; ++r) v[r] = old[x][r] * a.beta + v[r];
+                    if constexpr (VEC) patch[at >> 2] = *reinterpret_cast<const h4f*>(v);
+                    else reinterpret_cast<float*>(patch)[at] = v[0];
+                }
+                if (row < rows_left && col < cols_left) {
+                    float* to = hw + ((uint32_t)row * C32 + (uint32_t)col);
+                    if constexpr (VEC) *reinterpret_cast<h4f*>(to) = *reinterpret_cast<const h4f*>(v);
+                    else *to = v[0];
+#pragma unroll
+                    for (int r = 0; r < V; ++r) finite = finite && finite_f(v[r]);
+                }
             }
         }
-        if (diag) continue;                          // the tile on the diagonal is its own mirror image
-        // mirror image: H[gj][gi] = H[gi][gj]; lane = row lr of the patch, one column per instruction, so the wave
-        // writes 64 consecutive floats of a row of H.  (The patch is the wave's own: no barrier.)
-        const int lr = lane;
-#pragma unroll 8
-        for (int lc = 0; lc < 32; ++lc) {
-            const float v = patch[lr * 32 + (lc ^ (lr & 31))];
-            if (lr < rows_left && n * 32 + lc < cols_left) hm[(uint32_t)(n * 32 + lc) * C32 + (uint32_t)lr] = v;
+        if (diag) return;                            // the tile on the diagonal is its own mirror image
+        // mirror image: a lane takes V rows of one column of the patch (the patch is the wave's own: no barrier)
+#pragma unroll 1
+        for (int b = 0; b < kTurns; b += 4) {
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+                const int e = (b + x) * 64 + lane, col = e / kPieces, row = V * (e % kPieces);
+                float v[V];
+#pragma unroll
+                for (int r = 0; r < V; ++r) v[r] = pf[in_patch(row + r, col)];
+                if (col < cols_left && row < rows_left) {
+                    float* to = hm + ((uint32_t)col * C32 + (uint32_t)row);
+                    if constexpr (VEC) *reinterpret_cast<h4f*>(to) = *reinterpret_cast<const h4f*>(v);
+                    else *to = v[0];
+                }
+            }
         }
+    };
+    if (rows_left > 0 && cols_left > 0) {
+        if (a.vec) finish(std::true_type{});
+        else finish(std::false_type{});
     }
     if (a.bad && !finite) *a.bad = 1;
 }
@@ -284,9 +353,27 @@ using namespace amct;
 
 static int64_t hs_round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
 
+// The width of the tiles by their number, for 256 CUs.  64 columns while three tiles a CU hold them all (to 2432 columns): short
+// tiles, many of them (2048 tokens of 512 / 2048 columns: 12.9 / 23.4 us, with 128 columns 25.3 / 29.3; at 2560 columns 32.4 and 30.6).
+// Else 128, two a CU.  Where these need a second round for a few more (3969 columns and on) but tiles of 192 columns do with one
+// a CU (to 4224), 192: 4096 columns 50.0 us, with 128 62.2; 3968 columns 49.6 and 40.3; 4480 94.3 and 64.7.
+static int hs_width(int64_t cols) {
+    auto tiles = [cols](int64_t side) { const int64_t nb = (cols + side - 1) / side; return nb * (nb + 1) / 2; };
+    if (tiles(64) <= 3 * 256) return 2;
+    return tiles(128) > 2 * 256 && tiles(192) <= 256 ? 6 : 4;
+}
+
+
+template <bool F16, int W> static void hs_launch(SyrkArgs a, hipStream_t st) {
+    a.nb = (int)((a.C + 32 * W - 1) / (32 * W));
+    a.ntiles = (int64_t)a.nb * (a.nb + 1) / 2;
+    a.per_die = (int)((a.ntiles + 7) / 8);
+    hipLaunchKernelGGL((hess_syrk_k<F16, W>), dim3((unsigned)(8 * (int64_t)a.per_die)), dim3(kBlock), SyrkShape<W>::kLds, st, a);
+}
+
 extern "C" size_t amct_hessian_update_workspace_bytes(int64_t tokens, int64_t cols) {
     if (tokens <= 0 || cols <= 0) return 0;
-    return (size_t)hs_round_up(cols, kHsTile) * (size_t)hs_round_up(tokens, kHsK) * 2;
+    return (size_t)hs_round_up(cols, 128) * (size_t)hs_round_up(tokens, kHsK) * 2;
 }
 
 extern "C" int amct_hessian_update(float* hessian, const void* x, int64_t tokens, int64_t cols, float beta, float alpha,
@@ -299,24 +386,31 @@ extern "C" int amct_hessian_update_checked(float* hessian, const void* x, int64_
     if (tokens < 0 || cols <= 0 || !hessian) return AMCT_E_BADARG;
     if (dtype != AMCT_BF16 && dtype != AMCT_F16) return AMCT_E_UNSUPPORTED;
     if (tokens != 0 && !x) return AMCT_E_BADARG;
-    const int64_t Cp = hs_round_up(cols, kHsTile), Tp = hs_round_up(tokens > 0 ? tokens : 1, kHsK);
-    const int64_t nb = Cp / kHsTile;
     if (cols >= (int64_t(1) << 22)) return AMCT_E_TOO_LARGE;                  // 32-bit offsets inside a tile, block ids
-    if (!workspace || workspace_bytes < (size_t)Cp * (size_t)Tp * 2) return AMCT_E_BADARG;
+    const size_t need = (size_t)hs_round_up(cols, 128) * (size_t)hs_round_up(tokens > 0 ? tokens : 1, kHsK) * 2;
+    if (!workspace || workspace_bytes < need) return AMCT_E_BADARG;
     if (!aligned16(workspace) || (reinterpret_cast<uintptr_t>(hessian) & 3u) != 0 || (reinterpret_cast<uintptr_t>(x) & 1u) != 0)
         return AMCT_E_ALIGN;
     hipStream_t st = (hipStream_t)stream;
-    if (cols % 8 == 0 && aligned16(x))
-        hipLaunchKernelGGL(hess_transpose_vec_k, dim3((unsigned)(Cp / 64), (unsigned)(Tp / 64)), dim3(kBlock), 0, st,
-                           reinterpret_cast<const uint16_t*>(x), reinterpret_cast<uint16_t*>(workspace), tokens, cols, Tp, bad);
-    else
-        hipLaunchKernelGGL(hess_transpose_k, dim3((unsigned)(Cp / 64), (unsigned)(Tp / 64)), dim3(kBlock), 0, st,
-                           reinterpret_cast<const uint16_t*>(x), reinterpret_cast<uint16_t*>(workspace), tokens, cols, Tp, bad);
-    const int64_t ntiles = nb * (nb + 1) / 2, per_die = (ntiles + 7) / 8;
-    SyrkArgs a{reinterpret_cast<const uint16_t*>(workspace), hessian, cols, Tp, (int)nb, (int)per_die, ntiles, beta, alpha, bad};
-    constexpr size_t lds_bytes = 2 * kHsTile * 128;                           // 32 KB
-    const dim3 grid((unsigned)(8 * per_die));
-    if (dtype == AMCT_F16) hipLaunchKernelGGL((hess_syrk_k<true>), grid, dim3(kBlock), lds_bytes, st, a);
-    else hipLaunchKernelGGL((hess_syrk_k<false>), grid, dim3(kBlock), lds_bytes, st, a);
+    SyrkArgs a{reinterpret_cast<const uint16_t*>(x), hessian, tokens, cols, cols, 0, 0, 0, beta, alpha,
+               cols % 4 == 0 && aligned16(hessian), bad};
+    if (bad) hipLaunchKernelGGL(hess_clear_k, dim3(1), dim3(1), 0, st, bad);
+    if (cols % 8 != 0 || !aligned16(x)) {
+        a.ld = hs_round_up(cols, 8);
+        if (tokens > 0)
+            hipLaunchKernelGGL(hess_align_k, dim3((unsigned)((a.ld / 8 + kBlock - 1) / kBlock), (unsigned)(tokens < 65535 ? tokens : 65535)),
+                               dim3(kBlock), 0, st, reinterpret_cast<const uint16_t*>(x), reinterpret_cast<uint16_t*>(workspace), tokens, cols,
+                               a.ld);
+        a.x = reinterpret_cast<const uint16_t*>(workspace);
+    }
+#define AMCT_HS(W)                                              \
+    case W:                                                     \
+        if (dtype == AMCT_F16) hs_launch<true, W>(a, st);       \
+        else hs_launch<false, W>(a, st);                        \
+        break;
+    switch (hs_width(cols)) {
+        AMCT_HS(2) AMCT_HS(4) AMCT_HS(6)
+    }
+#undef AMCT_HS
     return hip_status();
 }

@@ -140,6 +140,27 @@ def test_hessian_update_kernel(dev, dtype, tokens, cols):
     assert torch.equal(hd, hd.t()), "symmetry"
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tokens,cols", [(64, 64), (128, 72), (191, 2432), (1, 2433), (65, 2440), (257, 3968), (130, 3969), (64, 4224), (200, 4225), (449, 4300)])
+def test_hessian_tiles(dev, dtype, tokens, cols):
+    """Both sides of the lines between the tile widths, whole and partial last steps and tiles, X and H that start off a
+    16-byte boundary: sums of small integers are exact, so every element is compared bit for bit; nothing is written behind
+    the matrix."""
+    g = torch.Generator().manual_seed(tokens + cols)
+    for off in (0, 1):
+        x = torch.empty(tokens * cols + 8, dtype=dtype, device=dev)[off:off + tokens * cols].view(tokens, cols)
+        x.copy_(torch.randint(-4, 5, (tokens, cols), generator=g))
+        buf = torch.full((cols * cols + 200,), 7.0, device=dev)
+        h = buf[off:off + cols * cols].view(cols, cols)
+        h.fill_(float('nan'))
+        prod = x.double().t() @ x.double()
+        ops.hessian_update(h, x, 0.0, 1.0)
+        assert torch.equal(h.double(), prod)
+        ops.hessian_update(h, x, 0.5, 2.0)
+        assert torch.equal(h.double(), 2.5 * prod)
+        assert bool((buf[:off] == 7).all()) and bool((buf[off + cols * cols:] == 7).all())
+
+
 def test_update_hessian_on_16_bit_activations(dev):
     """quantize_op.gptq.update_hessian with bf16 activations on the device takes the kernel; against the oracle's
     restatement of the reference (fp32 product of the scaled activations) within the rounding of the two orders of
