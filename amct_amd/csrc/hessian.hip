@@ -25,6 +25,7 @@
 namespace amct {
 
 typedef float h4f __attribute__((ext_vector_type(4)));
+typedef float h16f __attribute__((ext_vector_type(16)));
 typedef __bf16 h8bf __attribute__((ext_vector_type(8)));
 typedef _Float16 h8h __attribute__((ext_vector_type(8)));
 typedef short h4s __attribute__((ext_vector_type(4)));
@@ -64,9 +65,9 @@ struct SyrkArgs {
 };
 
 template <bool F16>
-AMCT_DEV h4f hs_mfma(const h8s& a, const h8s& b, const h4f& c) {
-    if constexpr (F16) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8h, a), __builtin_bit_cast(h8h, b), c, 0, 0, 0);
-    else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(h8bf, a), __builtin_bit_cast(h8bf, b), c, 0, 0, 0);
+AMCT_DEV h16f hs_mfma(const h8s& a, const h8s& b, const h16f& c) {
+    if constexpr (F16) return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8h, a), __builtin_bit_cast(h8h, b), c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(h8bf, a), __builtin_bit_cast(h8bf, b), c, 0, 0, 0);
 }
 
 // A direct-to-LDS load: wave-uniform 64-bit base, a byte offset per lane, lane l's 16 bytes land at lds + 16 l.  (Inline, with
@@ -80,8 +81,8 @@ AMCT_DEV void hs_meet() {
     asm volatile("" ::: "memory");
 }
 
-// W: 16-column tiles per side of a wave (2, 4 or 6); the block's tile is 32 W columns wide.  128-column tiles take two stages so
-// that two blocks fit a CU, and one's epilogue runs under the other's products: X[2048,11008] 293 us, with three stages and
+// W: half the 32-column MFMA tiles per side of a block (2, 4 or 6): W / 2 of them per side of a wave.  128-column tiles take two stages so
+// that two blocks fit a CU, and one's epilogue runs under the other's products: X[2048,11008] 295 us, with three stages and
 // one block 381.
 template <int W> struct SyrkShape {
     static constexpr int kTile = 32 * W;
@@ -134,10 +135,10 @@ __global__ __launch_bounds__(kBlock, SyrkShape<W>::kPerCu) void hess_syrk_k(Syrk
     const int wi = wave >> 1, wj = wave & 1;         // 2 x 2 waves of 16 W x 16 W
 
     // Memory -> LDS: per operand and step 64 tokens x 4 W chunks of 16 bytes, token after token; a wave moves W pieces of 1 KB.
-    // A fragment read takes 16 tokens x 32 bytes at a time: inside a token the 32-byte units are swapped by the token (swap), so
-    // that eight consecutive tokens' units lie in different banks (a token is 128, 256 or 384 bytes).
+    // A fragment read takes 4 tokens x 64 bytes from each half of 8 tokens: the 32-byte units of a token are swapped by the
+    // token, so that four consecutive tokens' pairs of units lie in different banks (a token is 128, 256 or 384 bytes).
     // Columns beyond C repeat the last ones of X (their sums are not stored), tokens beyond T the last one (cleared below).
-    auto swap = [](int t) { return W == 4 ? t & 7 : (t >> 1) & 3; };
+    auto swap = [](int t) { return W == 4 ? 2 * (t & 3) : t & 2; };
     const uint32_t row_bytes = (uint32_t)(a.ld * 2);
     uint32_t off_a[W], off_b[W];                     // bytes from the tile's first column at the step's first token
 #pragma unroll
@@ -180,45 +181,48 @@ __global__ __launch_bounds__(kBlock, SyrkShape<W>::kPerCu) void hess_syrk_k(Syrk
         hs_meet();
     };
 
-    // Fragment of 16 columns and 32 tokens: lane l holds column l % 16 and the tokens 4 (l / 16) .. + 3 and 16 more.  Both
-    // operands take the same tokens in the same places, which is all that the contraction asks for.  The lane reads
-    // 4 columns of token 4 (l / 16) + (l % 16) / 4 and is given its own column by the transposition.
-    const int tl = 4 * (lane >> 4) + ((lane & 15) >> 2);
-    int at_a[W], at_b[W];
+    // Fragment of 32 columns and 16 tokens: lane l holds column l % 32 and the tokens 8 (l / 32) .. + 7, each sum in the order of
+    // the tokens.  Group l / 16 of the lanes reads 4 tokens x 16 columns, a lane 4 columns of token (l % 16) / 4, and is given its
+    // own column by the transposition; then the 4 tokens behind (swapped alike).
+    constexpr int N = W / 2;                         // 32-column tiles per side of a wave
+    const int tl = 8 * (lane >> 5) + ((lane & 15) >> 2), half = (lane >> 4) & 1;
+    int at_a[N], at_b[N];
 #pragma unroll
-    for (int m = 0; m < W; ++m) {
-        at_a[m] = tl * S::kRow + ((wi * W + m) ^ swap(tl)) * 32 + (lane & 3) * 8;
-        at_b[m] = S::kOperand + tl * S::kRow + ((wj * W + m) ^ swap(tl)) * 32 + (lane & 3) * 8;
+    for (int m = 0; m < N; ++m) {
+        at_a[m] = tl * S::kRow + ((wi * W + 2 * m + half) ^ swap(tl)) * 32 + (lane & 3) * 8;
+        at_b[m] = S::kOperand + tl * S::kRow + ((wj * W + 2 * m + half) ^ swap(tl)) * 32 + (lane & 3) * 8;
     }
     auto fragment = [&](int at) {
         typedef __attribute__((address_space(3))) h4s lds_h4s;
         const h4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_h4s*)(lds + at));
-        const h4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_h4s*)(lds + at + 16 * S::kRow));
+        const h4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_h4s*)(lds + at + 4 * S::kRow));
         return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     };
-    h8s fa[2][W], fb[2][W];
-    // q < W: rows, else columns, of half u (32 tokens) of a stage
-    auto read_one = [&](int stage, int u, int q) {
-        const int base = stage * S::kStage + u * 32 * S::kRow;
-        if (q < W) fa[u][q] = fragment(base + at_a[q]);
-        else fb[u][q - W] = fragment(base + at_b[q - W]);
+    h8s fa[2][2][N], fb[2][2][N];                    // [half of a stage: 32 tokens][16 tokens][tile]
+    constexpr int kReads = 4 * N, kProducts = 2 * N * N;
+    auto read_one = [&](int stage, int u, int q) {   // q < 4 N: fragment of half u
+        const int ks = q / (2 * N), x = q % (2 * N), base = stage * S::kStage + (2 * u + ks) * 16 * S::kRow;
+        if (x < N) fa[u][ks][x] = fragment(base + at_a[x]);
+        else fb[u][ks][x - N] = fragment(base + at_b[x - N]);
     };
-    h4f acc[W][W];
+    h16f acc[N][N];
 #pragma unroll
-    for (int m = 0; m < W; ++m)
+    for (int m = 0; m < N; ++m)
 #pragma unroll
-        for (int n = 0; n < W; ++n) acc[m][n] = h4f{0.f, 0.f, 0.f, 0.f};
-    // the products of half u, one fragment of the next half behind every kGap-th of them; the column fragment is the first
-    // operand: a lane's four sums of tile (m, n) are H[16 m + lane % 16][16 n + 4 (lane / 16) + 0 .. 3] of the wave's tile
-    constexpr int kGap = W / 2;
+        for (int n = 0; n < N; ++n)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[m][n][r] = 0.f;
+    // the products of half u, the fragments of the next half dealt out behind them; the column fragment is the first
+    // operand: sums 4 q .. + 3 of tile (m, n) are H[32 m + lane % 32][32 n + 8 q + 4 (lane / 32) + 0 .. 3] of the wave's tile
     auto products = [&](int u, bool more, int stage, int v) {
 #pragma unroll
-        for (int x = 0; x < W * W; ++x) {
-            const int m = x / W, n = x % W;
-            acc[m][n] = hs_mfma<F16>(fb[u][n], fa[u][m], acc[m][n]);
+        for (int x = 0; x < kProducts; ++x) {
+            const int ks = x / (N * N), m = x / N % N, n = x % N;
+            acc[m][n] = hs_mfma<F16>(fb[u][ks][n], fa[u][ks][m], acc[m][n]);
             __builtin_amdgcn_sched_barrier(0);
-            if (more && x % kGap == 0) {
-                read_one(stage, v, x / kGap);
+            if (more) {
+#pragma unroll
+                for (int q = x * kReads / kProducts; q < (x + 1) * kReads / kProducts; ++q) read_one(stage, v, q);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -233,7 +237,7 @@ __global__ __launch_bounds__(kBlock, SyrkShape<W>::kPerCu) void hess_syrk_k(Syrk
         hs_meet();
         if (last == 0 && tail < kHsK) clear_tail(0);
 #pragma unroll
-        for (int q = 0; q < 2 * W; ++q) read_one(0, 0, q);
+        for (int q = 0; q < kReads; ++q) read_one(0, 0, q);
         int stage = 0;
         for (int s = 0; s < last; ++s) {
             const int next = stage + 1 == S::kStages ? 0 : stage + 1;
@@ -262,15 +266,17 @@ __global__ __launch_bounds__(kBlock, SyrkShape<W>::kPerCu) void hess_syrk_k(Syrk
     };
     h4f* patch = reinterpret_cast<h4f*>(lds + wave * (S::kLds / 4));
 #pragma unroll
-    for (int m = 0; m < W; ++m)
+    for (int m = 0; m < N; ++m)
 #pragma unroll
-        for (int n = 0; n < W; ++n) {
-            h4f v;
+        for (int n = 0; n < N; ++n)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] = a.alpha * acc[m][n][r];
-            const int row = 16 * m + (lane & 15);
-            patch[row * kUnits + unit_of(row, 4 * n + (lane >> 4))] = v;
-        }
+            for (int q = 0; q < 4; ++q) {
+                h4f v;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = a.alpha * acc[m][n][4 * q + r];
+                const int row = 32 * m + (lane & 31);
+                patch[row * kUnits + unit_of(row, 8 * n + 2 * q + (lane >> 5))] = v;
+            }
     // Addresses: one block-uniform base per wave plus 32-bit lane offsets (cols < 2^22 is checked by the host).
     const bool have = a.beta != 0.f;
     const uint32_t C32 = (uint32_t)a.C;
@@ -356,11 +362,13 @@ static int64_t hs_round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
 // The width of the tiles by their number, for 256 CUs.  64 columns while three tiles a CU hold them all (to 2432 columns): short
 // tiles, many of them (2048 tokens of 512 / 2048 columns: 12.9 / 23.4 us, with 128 columns 25.3 / 29.3; at 2560 columns 32.4 and 30.6).
 // Else 128, two a CU.  Where these need a second round for a few more (3969 columns and on) but tiles of 192 columns do with one
-// a CU (to 4224), 192: 4096 columns 50.0 us, with 128 62.2; 3968 columns 49.6 and 40.3; 4480 94.3 and 64.7.
-static int hs_width(int64_t cols) {
+// a CU (to 4224), 192: 4096 columns 50.0 us, with 128 62.2; 3968 columns 49.6 and 40.3; 4480 94.3 and 64.7.  Not where rows of H
+// are not 16-byte aligned: a column a lane, four waves a CU take 25 us longer over their H (512 tokens of 4098 columns: 49.5 / 60.0
+// into an empty / a running H, with 128 44.4 / 52.9, from the transposed copy 42.7 / 59.7).
+static int hs_width(int64_t cols, bool vec) {
     auto tiles = [cols](int64_t side) { const int64_t nb = (cols + side - 1) / side; return nb * (nb + 1) / 2; };
     if (tiles(64) <= 3 * 256) return 2;
-    return tiles(128) > 2 * 256 && tiles(192) <= 256 ? 6 : 4;
+    return vec && tiles(128) > 2 * 256 && tiles(192) <= 256 ? 6 : 4;
 }
 
 
@@ -408,7 +416,7 @@ extern "C" int amct_hessian_update_checked(float* hessian, const void* x, int64_
         if (dtype == AMCT_F16) hs_launch<true, W>(a, st);       \
         else hs_launch<false, W>(a, st);                        \
         break;
-    switch (hs_width(cols)) {
+    switch (hs_width(cols, a.vec != 0)) {
         AMCT_HS(2) AMCT_HS(4) AMCT_HS(6)
     }
 #undef AMCT_HS
