@@ -14,10 +14,12 @@
 // A tile is 64, 128 or 192 columns wide, 2 x 2 waves of half that: see hs_width.  The epilogue
 // applies beta and alpha, writes the tile and its mirror image, so H stays exactly symmetric, and notes whether everything
 // it wrote is finite: as library passes over H that check took as long as the update itself (75 us at 4096 columns).
-// X[2048,4096] bf16 into an empty / a running H[4096,4096]: 50 / 54 us (1 PFLOP/s on the 253 tiles), where 128-column tiles fed by a
-// kernel that transposed X first took 75 / 82; 512 columns 12.9 / 13.2 (39 / 40), 2816 30 / 31 (50 / 53), 11008 293 / 348 (350 / 404).
-// At 4096 columns the products take 33 us (21 at the rate of a register-only loop, 8 more are the loads' and LDS's), the
-// rest is the launch and H itself, 64 MB written and half of it read, all tiles at the same time.
+// X[2048,4096] bf16 into an empty / a running H[4096,4096]: 48 / 52 us, where 128-column tiles fed by a kernel that transposed X
+// first took 75 / 82; 512 columns 12 / 12 (39 / 40), 2816 30 / 31 (49 / 53), 11008 295 / 351 (335 / 403).  At 4096 columns the
+// products take about 31 us (21 at the rate of a register-only loop, 8 more are the loads' and LDS's), the rest is the launch
+// and H itself, 64 MB written and half of it read, all tiles at the same time.
+// Every sum runs over the tokens in order, 16 to an instruction, whatever the tile: GPTQ's codes follow the last bits of H
+// (sums of 32 tokens an instruction, as far from the exact ones, moved codes in 7 rows of 100 of a [4096,4096] layer).
 #include <type_traits>
 
 #include "amct_common.h"
@@ -360,11 +362,11 @@ using namespace amct;
 static int64_t hs_round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
 
 // The width of the tiles by their number, for 256 CUs.  64 columns while three tiles a CU hold them all (to 2432 columns): short
-// tiles, many of them (2048 tokens of 512 / 2048 columns: 12.9 / 23.4 us, with 128 columns 25.3 / 29.3; at 2560 columns 32.4 and 30.6).
+// tiles, many of them (2048 tokens of 512 / 2048 columns: 11.9 / 23.4 us, with 128 columns 24.2 / 29.1; at 2560 columns 31.4 and 30.4).
 // Else 128, two a CU.  Where these need a second round for a few more (3969 columns and on) but tiles of 192 columns do with one
-// a CU (to 4224), 192: 4096 columns 50.0 us, with 128 62.2; 3968 columns 49.6 and 40.3; 4480 94.3 and 64.7.  Not where rows of H
-// are not 16-byte aligned: a column a lane, four waves a CU take 25 us longer over their H (512 tokens of 4098 columns: 49.5 / 60.0
-// into an empty / a running H, with 128 44.4 / 52.9, from the transposed copy 42.7 / 59.7).
+// a CU (to 4224), 192: 4096 columns 47.8 us, with 128 62.6; 3968 columns 46.8 and 40.2; 4608 90.1 and 66.8.  Not where rows of H
+// are not 16-byte aligned: a column a lane, four waves a CU take 25 us longer over their H (512 tokens of 4098 columns: 49.0 / 58.8
+// into an empty / a running H, with 128 44.2 / 52.8, from the transposed copy 41.9 / 59.1).
 static int hs_width(int64_t cols, bool vec) {
     auto tiles = [cols](int64_t side) { const int64_t nb = (cols + side - 1) / side; return nb * (nb + 1) / 2; };
     if (tiles(64) <= 3 * 256) return 2;
