@@ -35,6 +35,9 @@ SIGNATURES = {
     "amct_awq_loss_partials": (_I, [_P, _P, _L, _I, _P, _P]),
     "amct_awq_pick": (_I, [_P, _L, _I, _I, _P, _P, _P]),
     "amct_flag_nonfinite": (_I, [_P, _L, _I, _P, _P]),
+    "amct_gptq_block_parts": (_I, [_P, _L, _P, _L, _P, _L, _P, _P, _L, _P, _L, _I, _I, _I, _P, _L, _P, _P]),
+    "amct_gptq_split": (_I, [_P, _P, _L, _L, _P, _P]),
+    "amct_gptq_trail_parts": (_I, [_P, _L, _P, _L, _P, _L, _P, _L, _P, _L, _P, _L, _L, _I, _P]),
     "amct_gptq_trail": (_I, [_P, _L, _P, _L, _P, _L, _L, _L, _I, _P]),
     "amct_gptq_order": (_I, [_P, _P, _P, _P, _L, _L, _I, _I, _P]),
     "amct_gptq_factor_workspace_bytes": (ctypes.c_size_t, [_L]),

@@ -19,6 +19,7 @@
 #include <utility>
 
 #include "amct_common.h"
+#include "gptq_parts.h"
 
 namespace amct {
 
@@ -38,6 +39,9 @@ struct GptqArgs {
     int count;
     int rows_per_wave;
     float qmin, qmax;
+    uint16_t* parts;                                // [rows][3][ld_p]: the errors as three bf16 parts too, or null
+    int64_t ld_p;
+    int32_t* wide;                                  // set where the parts do not hold an error
 };
 
 __global__ __launch_bounds__(kBlock) void gptq_block_k(GptqArgs a) {
@@ -111,6 +115,14 @@ __global__ __launch_bounds__(kBlock) void gptq_block_k(GptqArgs a) {
                 float* er = a.err + n * a.ld_e;
                 if (v0) { wr[c0] = w0[r]; er[c0] = e0[r]; }
                 if (v1) { wr[c1] = w1[r]; er[c1] = e1[r]; }
+                if (a.parts) {
+                    uint16_t* pr = a.parts + n * 3 * a.ld_p;
+                    uint32_t h, m, l;
+                    split_parts(e0[r], e1[r], h, m, l);
+                    if (v0) { pr[c0] = (uint16_t)h; pr[a.ld_p + c0] = (uint16_t)m; pr[2 * a.ld_p + c0] = (uint16_t)l; }
+                    if (v1) { pr[c1] = (uint16_t)(h >> 16); pr[a.ld_p + c1] = (uint16_t)(m >> 16); pr[2 * a.ld_p + c1] = (uint16_t)(l >> 16); }
+                    if ((v0 && !parts_hold(e0[r])) || (v1 && !parts_hold(e1[r]))) *a.wide = 1;
+                }
             }
         }
     }
@@ -413,6 +425,22 @@ __global__ __launch_bounds__(kBlock) void gptq_block_row_k(GptqArgs a) {
             *reinterpret_cast<float4*>(wo + 4 * NL * m) = make_float4(r.w[m][0], r.w[m][1], r.w[m][2], r.w[m][3]);
             *reinterpret_cast<float4*>(er + 4 * NL * m) = make_float4(r.eo[m][0], r.eo[m][1], r.eo[m][2], r.eo[m][3]);
         }
+        if (a.parts) {
+            uint16_t* pr = a.parts + n * 3 * a.ld_p + 4 * q;
+            bool hold = true;
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                uint2 hi, mid, lo;
+                split_parts(r.eo[m][0], r.eo[m][1], hi.x, mid.x, lo.x);
+                split_parts(r.eo[m][2], r.eo[m][3], hi.y, mid.y, lo.y);
+                *reinterpret_cast<uint2*>(pr + 4 * NL * m) = hi;
+                *reinterpret_cast<uint2*>(pr + a.ld_p + 4 * NL * m) = mid;
+                *reinterpret_cast<uint2*>(pr + 2 * a.ld_p + 4 * NL * m) = lo;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) hold = hold && parts_hold(r.eo[m][e]);
+            }
+            if (!hold) *a.wide = 1;
+        }
     }
 }
 
@@ -423,6 +451,16 @@ using namespace amct;
 extern "C" int amct_gptq_block(float* w, int64_t ld_w, float* err, int64_t ld_e, const float* hinv, int64_t ld_h,
                                const float* scale, const int32_t* offset, int64_t scale_stride, const int32_t* gidx,
                                int64_t rows, int count, int qmin, int qmax, amct_stream_t stream) {
+    return amct_gptq_block_parts(w, ld_w, err, ld_e, hinv, ld_h, scale, offset, scale_stride, gidx, rows, count, qmin, qmax, nullptr, 0,
+                                 nullptr, stream);
+}
+
+extern "C" int amct_gptq_block_parts(float* w, int64_t ld_w, float* err, int64_t ld_e, const float* hinv, int64_t ld_h,
+                                     const float* scale, const int32_t* offset, int64_t scale_stride, const int32_t* gidx,
+                                     int64_t rows, int count, int qmin, int qmax, uint16_t* parts, int64_t ld_p, int32_t* wide,
+                                     amct_stream_t stream) {
+    if (parts && (ld_p < count || ld_p % 4 != 0 || !wide)) return AMCT_E_BADARG;
+    if (reinterpret_cast<uintptr_t>(parts) & 7u) return AMCT_E_ALIGN;
     if (rows < 0 || count < 0 || count > kGqMax || qmin > qmax) return AMCT_E_BADARG;
     if (ld_w < count || ld_e < count || ld_h < count || scale_stride < 0) return AMCT_E_BADARG;
     if (rows == 0 || count == 0) return AMCT_OK;
@@ -431,6 +469,7 @@ extern "C" int amct_gptq_block(float* w, int64_t ld_w, float* err, int64_t ld_e,
     a.w = w; a.err = err; a.hinv = hinv; a.scale = scale; a.offset = offset; a.gidx = gidx;
     a.rows = rows; a.ld_w = ld_w; a.ld_e = ld_e; a.ld_h = ld_h; a.scale_stride = scale_stride;
     a.count = count; a.qmin = (float)qmin; a.qmax = (float)qmax;
+    a.parts = parts; a.ld_p = ld_p; a.wide = wide;
     if (count == kGqMax && ld_w % 4 == 0 && ld_e % 4 == 0 && aligned16(w) && aligned16(err) && (rows + 15) / 16 <= 0x7FFFFFFF) {
         const bool wide = rows <= kGqWideRows;
         const int64_t per = (kBlock / 64) * (wide ? 4 : 16);

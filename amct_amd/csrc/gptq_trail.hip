@@ -2,6 +2,7 @@
 // amct_pytorch/quantize_op/gptq_module.py:152-153 `weight[:, i2:] -= err_block @ hinv[i1:i2, i2:]`, :122 `weight[:, perm]` and
 // :155 `weight[:, invperm]`.
 //
+// (Layers of more than 1024 columns are updated from bf16 parts instead: gptq_parts.hip.)
 // gptq_trail_k: one 128 x 64 tile of W per thread block, W <- W - E U with fp32 MFMA: the product is summed first and
 // subtracted once, as in the reference, but W is read and written once instead of three times more for a product that is
 // written, read and subtracted.  E and U come 32 steps of the contraction at a time through LDS, the next 32 wait in

@@ -288,6 +288,43 @@ def gptq_trail(w, err, u, i1, i2):
                                                cols - i2, i2 - i1, _stream(dev)))
 
 
+def gptq_split(u, wide):
+    """The upper triangular u fp32 [C,C] as three bf16 parts, [C, 3, C up to a multiple of 8] (nothing below the diagonal's
+    multiple of 8 is written); wide (int32, one element) becomes 1 where the parts do not hold u."""
+    dev = _dev(u, wide)
+    cols = u.shape[0]
+    _need(u.dim() == 2 and u.shape[1] == cols and u.dtype == torch.float32 and u.is_contiguous(), "gptq_split: u must be a square fp32 matrix")
+    _need(wide.dtype == torch.int32 and wide.numel() == 1, "gptq_split: wide must be one int32 value")
+    parts = torch.empty(cols, 3, (cols + 7) // 8 * 8, dtype=torch.bfloat16, device=dev)
+    with _on(dev):
+        _lib.check(_lib.load().amct_gptq_split(_p(u), _p(parts), cols, parts.shape[2], _p(wide), _stream(dev)))
+    return parts
+
+
+def gptq_trail_parts(w, err, u, err_parts, u_parts, wide, i1, i2, end):
+    """w[:, i2:end] -= err @ u[i1:i2, i2:end] in place from the parts of err and u (gptq_module.py:152-153).  err fp32
+    [N, i2 - i1] and err_parts bf16 [N, 3, i2 - i1] may be the leading columns of wider tensors; i1 and i2 multiples of 32."""
+    dev = _dev(w, err, u, err_parts, u_parts, wide)
+    rows, cols = w.shape
+    count = i2 - i1
+    for name, t, shape in (("w", w, (rows, cols)), ("u", u, (cols, cols))):
+        _need(t.dtype == torch.float32 and tuple(t.shape) == shape and t.is_contiguous(),
+              "gptq_trail_parts: {} must be a contiguous fp32 tensor of shape {}", name, shape)
+    _need(0 <= i1 < i2 <= end <= cols and i1 % 32 == 0 and i2 % 32 == 0, "gptq_trail_parts: no columns {}:{} in {}", i1, i2, cols)
+    _need(err.dtype == torch.float32 and tuple(err.shape) == (rows, count) and err.stride(1) == 1,
+          "gptq_trail_parts: err must be fp32 rows of {} elements", count)
+    _need(err_parts.dtype == torch.bfloat16 and tuple(err_parts.shape) == (rows, 3, count) and err_parts.stride(2) == 1 and
+          err_parts.stride(0) == 3 * err_parts.stride(1), "gptq_trail_parts: err_parts must be bf16 [{}, 3, {}]", rows, count)
+    _need(u_parts.dtype == torch.bfloat16 and tuple(u_parts.shape) == (cols, 3, (cols + 7) // 8 * 8) and u_parts.is_contiguous(),
+          "gptq_trail_parts: u_parts must come from gptq_split")
+    _need(wide.dtype == torch.int32 and wide.numel() == 1, "gptq_trail_parts: wide must be one int32 value")
+    ldp = u_parts.shape[2]
+    with _on(dev):
+        _lib.check(_lib.load().amct_gptq_trail_parts(
+            _p(w) + 4 * i2, cols, _p(err), err.stride(0), _p(u) + 4 * (i1 * cols + i2), cols, _p(err_parts), err_parts.stride(1),
+            _p(u_parts) + 2 * (i1 * 3 * ldp + i2), ldp, _p(wide), rows, end - i2, count, _stream(dev)))
+
+
 def gptq_order(w, perm, dead):
     """w[:, perm] as fp32, the columns of w marked in dead (bool [C]) as zeros."""
     dev = _dev(w, perm, dead)

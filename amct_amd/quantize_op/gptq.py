@@ -1,6 +1,7 @@
 """Host-side mirror of the weight optimisation of amct_pytorch/quantize_op/gptq_module.py (:91-155, :161-186)
 with the tensors resident on the device.  The column loop of each block is one kernel launch (amct_gptq_block), the
-update of the columns behind it another (amct_gptq_trail), the factorisations one call (amct_gptq_factor)."""
+update of the columns behind it another (amct_gptq_trail, of wide layers amct_gptq_trail_parts), the factorisations one call
+(amct_gptq_factor)."""
 import math
 
 import torch
@@ -46,12 +47,25 @@ def update_hessian(hessian, nsamples, input_data, columns):
     return hessian, nsamples
 
 
-def gptq_block(weight_sorted, i1, i2, hinv, scale_w, offset_w, gidx, qmin, qmax):
-    """The column loop of block [i1, i2) in place on weight_sorted [N, columns] fp32; returns err_block."""
+# Columns whose errors are kept for one update of everything behind them; inside, a block's update reaches the end of these
+# columns only.  The weight is read and written once per 512 columns instead of once per 128, and the products of one update
+# are enough to keep the matrix pipe busy.
+_SPAN = 512
+# From how many columns on, and to how many (the parts of the factor are 6 bytes an element: 1.6 GB).  W[1024,1024]: 0.53 ms both
+# ways, of 512 columns 0.33 with spans and 0.31 without (the launches count there), W[1024,5120] 3.30 and 3.42, W[4096,4096]
+# 2.66 and 2.98, W[14336,4096] 4.45 and 5.21.
+_PARTS_COLUMNS = (1025, 16384)
+
+
+def gptq_block(weight_sorted, i1, i2, hinv, scale_w, offset_w, gidx, qmin, qmax, err=None, parts=None, wide=None):
+    """The column loop of block [i1, i2) in place on weight_sorted [N, columns] fp32; returns err_block, written to err, where
+    given: the columns [N, i2 - i1] of a wider matrix.  parts: the same columns of [N, 3, ...] bf16, err_block as the sum of
+    three; wide (int32, one element) becomes 1 where they do not hold it."""
     dev = ops._dev(weight_sorted, hinv, scale_w, offset_w, gidx)
     n, columns = weight_sorted.shape
     count = i2 - i1
-    err = torch.empty(n, count, dtype=torch.float32, device=dev)
+    if err is None:
+        err = torch.empty(n, count, dtype=torch.float32, device=dev)
     if scale_w.numel() == 1:
         stride = 0
     else:
@@ -59,10 +73,11 @@ def gptq_block(weight_sorted, i1, i2, hinv, scale_w, offset_w, gidx, qmin, qmax)
     w_ptr = weight_sorted.data_ptr() + i1 * 4
     h_ptr = hinv.data_ptr() + (i1 * hinv.shape[1] + i1) * 4
     with torch.cuda.device(dev):
-        _lib.check(_lib.load().amct_gptq_block(
-            w_ptr, columns, err.data_ptr(), count, h_ptr, hinv.shape[1], scale_w.data_ptr(),
+        _lib.check(_lib.load().amct_gptq_block_parts(
+            w_ptr, columns, err.data_ptr(), err.stride(0), h_ptr, hinv.shape[1], scale_w.data_ptr(),
             None if offset_w is None else offset_w.data_ptr(), stride, gidx.data_ptr(), n, count, qmin, qmax,
-            torch.cuda.current_stream(dev).cuda_stream))
+            None if parts is None else parts.data_ptr(), 0 if parts is None else parts.stride(1),
+            None if wide is None else wide.data_ptr(), torch.cuda.current_stream(dev).cuda_stream))
     return err
 
 
@@ -75,6 +90,26 @@ def _read_later(flag):
     event = torch.cuda.Event()
     event.record(torch.cuda.current_stream(flag.device))
     return host, event
+
+
+def _by_spans(ws, hinv, scale_w, offset_w, gidx, qmin, qmax, block_size, wide):
+    """The blocks of ws [N, columns] with their updates made by spans of columns, from the parts of the errors and of hinv."""
+    rows, columns = ws.shape
+    span = max(1, _SPAN // block_size) * block_size
+    width = min(span, -(-columns // 32) * 32)
+    hinv_parts = ops.gptq_split(hinv, wide)
+    errors = torch.empty(rows, width, dtype=torch.float32, device=ws.device)
+    parts = torch.empty(rows, 3, width, dtype=torch.bfloat16, device=ws.device)
+    for s1 in range(0, columns, span):
+        s2 = min(s1 + span, columns)
+        for i1 in range(s1, s2, block_size):
+            i2 = min(i1 + block_size, s2)
+            at = slice(i1 - s1, i2 - s1)
+            gptq_block(ws, i1, i2, hinv, scale_w, offset_w, gidx[i1:i2].contiguous(), qmin, qmax, errors[:, at], parts[:, :, at], wide)
+            if i2 < s2:
+                ops.gptq_trail_parts(ws, errors[:, at], hinv, parts[:, :, at], hinv_parts, wide, i1, i2, s2)
+        if s2 < columns:
+            ops.gptq_trail_parts(ws, errors[:, :s2 - s1], hinv, parts[:, :, :s2 - s1], hinv_parts, wide, s1, s2, columns)
 
 
 @torch.no_grad()
@@ -96,12 +131,13 @@ def get_opt_weight_and_quant_factor(weight, hessian, quant_config, block_size=12
     perm = torch.argsort(diag, descending=True)
     # the extrema of the weight with its dead columns at zero, in fp32 like the weight that the reference works on
     weight_min, weight_max = get_weight_min_max_by_granularity(weight.masked_fill(dead, 0), quant_config)
-    # flags that the kernels raise, read when everything is enqueued: a factor not finite, a pivot not positive
-    bad = torch.zeros(2, dtype=torch.int32, device=weight.device)
+    # flags that the kernels raise: a factor not finite, a pivot not positive (read when everything is enqueued), a value that
+    # three bf16 parts do not hold (read by the updates)
+    bad = torch.zeros(3, dtype=torch.int32, device=weight.device)
     scale_w, offset_w = ops.scale_offset(weight_max.float(), weight_min.float(), bits, bool(cfg.get('symmetric')), bad=bad[:1])
     ws = ops.gptq_order(weight, perm, dead)
     # cholesky(cholesky_inverse(cholesky(hs)), upper=True) of the permuted, damped Hessian, as one factorisation
-    hinv = ops.gptq_factor(hessian, perm, perc_damp * torch.mean(diag), bad[1:])
+    hinv = ops.gptq_factor(hessian, perm, perc_damp * torch.mean(diag), bad[1:2])
     flags, factored = _read_later(bad)
     sc = scale_w.reshape(-1).float().contiguous()
     zc = None if offset_w is None else offset_w.reshape(-1).to(torch.int32).contiguous()
@@ -110,11 +146,14 @@ def get_opt_weight_and_quant_factor(weight, hessian, quant_config, block_size=12
     else:
         gidx_all = torch.zeros(columns, dtype=torch.int32, device=weight.device)
     qmin, qmax = -(1 << (bits - 1)), (1 << (bits - 1)) - 1
-    for i1 in range(0, columns, block_size):
-        i2 = min(i1 + block_size, columns)
-        err_block = gptq_block(ws, i1, i2, hinv, sc, zc, gidx_all[i1:i2].contiguous(), qmin, qmax)
-        if i2 < columns:
-            ops.gptq_trail(ws, err_block, hinv, i1, i2)
+    if block_size % 32 == 0 and _PARTS_COLUMNS[0] <= columns <= _PARTS_COLUMNS[1]:
+        _by_spans(ws, hinv, sc, zc, gidx_all, qmin, qmax, block_size, bad[2:])
+    else:
+        for i1 in range(0, columns, block_size):
+            i2 = min(i1 + block_size, columns)
+            err_block = gptq_block(ws, i1, i2, hinv, sc, zc, gidx_all[i1:i2].contiguous(), qmin, qmax)
+            if i2 < columns:
+                ops.gptq_trail(ws, err_block, hinv, i1, i2)
     result = ops.gptq_order_back(ws, perm, weight.dtype).to(out_dtype)
     factored.synchronize()                          # of the copy only: long done when the last block is enqueued
     if int(flags[0]):

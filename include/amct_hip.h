@@ -394,6 +394,24 @@ int amct_gptq_block(float* w, int64_t ld_w, float* err_out, int64_t ld_e, const 
                     const float* scale, const int32_t* offset, int64_t scale_stride, const int32_t* gidx,
                     int64_t rows, int count, int qmin, int qmax, amct_stream_t stream);
 
+/* The same, and the errors as the sums of three bf16 numbers too (exact: 8 + 8 + 8 bits): parts [rows][3][ld_p], bf16,
+ * 8-byte aligned, ld_p a multiple of 4, at the block's first column; null: none.  *wide (int32 on the device) becomes 1
+ * where an error is neither 0 nor in [2^-100, 2^60), which the parts do not hold. */
+int amct_gptq_block_parts(float* w, int64_t ld_w, float* err_out, int64_t ld_e, const float* hinv, int64_t ld_h,
+                          const float* scale, const int32_t* offset, int64_t scale_stride, const int32_t* gidx,
+                          int64_t rows, int count, int qmin, int qmax, uint16_t* parts, int64_t ld_p, int32_t* wide,
+                          amct_stream_t stream);
+/* Such parts of the rows of the upper triangular u [cols, cols] (fp32, dense) from their diagonal on: parts [cols][3][ld],
+ * 16-byte aligned, ld a multiple of 8; *wide as above. */
+int amct_gptq_split(const float* u, uint16_t* parts, int64_t cols, int64_t ld, int32_t* wide, amct_stream_t stream);
+/* amct_gptq_trail from the parts of err and u, count a multiple of 32: six products of parts for one of fp32 numbers, summed in
+ * fp32 over 128 steps at a time (at most as far from the exact sums as fp32 products are).  err and u themselves are read where
+ * *wide is set.  err_parts [rows][3][ld_ep], u_parts [count][3][ld_up] at the first column of w, both 16-byte aligned, their row
+ * lengths multiples of 8; u_parts holds whole groups of 8 columns. */
+int amct_gptq_trail_parts(float* w, int64_t ld_w, const float* err, int64_t ld_e, const float* u, int64_t ld_u,
+                          const uint16_t* err_parts, int64_t ld_ep, const uint16_t* u_parts, int64_t ld_up, const int32_t* wide,
+                          int64_t rows, int64_t cols, int count, amct_stream_t stream);
+
 /* w[rows, cols] -= err[rows, count] @ u[count, cols], all fp32: the products of an element are summed before the one
  * subtraction.  Row strides ld_w, ld_e, ld_u in elements; w must not overlap err or u. */
 int amct_gptq_trail(float* w, int64_t ld_w, const float* err, int64_t ld_e, const float* u, int64_t ld_u, int64_t rows,

@@ -268,3 +268,122 @@ def test_gptq_whole_routine_raises_what_the_kernels_report(dev, columns, sym):
                 gptq.get_opt_weight_and_quant_factor(w.to(dev), h, cfg)
         got = gptq.get_opt_weight_and_quant_factor(w.to(dev), hess, cfg)[0]
         assert bool(torch.isfinite(got).all())
+
+
+def _parts(x, width):
+    """x fp32 [N, K] as three bf16 parts [N, 3, width], the leading K columns of each."""
+    out = torch.empty(x.shape[0], 3, width, dtype=torch.bfloat16, device=x.device)
+    rest = x.clone()
+    for k in range(3):
+        out[:, k, :x.shape[1]] = rest.bfloat16()
+        rest = rest - out[:, k, :x.shape[1]].float()
+    return out[:, :, :x.shape[1]]
+
+
+@pytest.mark.parametrize("n,columns,i1,i2,end", [(1, 65, 0, 32, 65), (63, 200, 32, 64, 136), (64, 192, 0, 128, 192), (65, 321, 96, 256, 321),
+                                                 (300, 1000, 0, 512, 1000), (1100, 777, 64, 608, 777), (130, 900, 160, 192, 193)])
+@pytest.mark.parametrize("spread", [0.0, 2.0])
+def test_gptq_trail_from_parts(dev, n, columns, i1, i2, end, spread):
+    """The update from three bf16 parts against the fp64 product.  Left out of a product: below 2^-25 of it.  A sum of 128
+    steps takes 6 * 128 / 32 additions of a wave's partial sums; the additions inside an instruction are taken to round
+    as often again; two units each bound what the hardware rounds by.  Every 128 steps one more rounding as W is updated.  The
+    products alone (W zero: its rounding every 128 steps is the reference's) are on the whole no further off than those of
+    the fp32 kernel taken 128 steps at a time (of values of one size: with a wide spread a handful of elements decides)."""
+    g = torch.Generator().manual_seed(n + columns)
+    err = (torch.randn(n, i2 - i1, generator=g) * torch.exp(spread * torch.randn(n, i2 - i1, generator=g)) * 0.01).to(dev)
+    err[torch.rand(n, i2 - i1, generator=g).to(dev) < 0.1] = 0.
+    u = torch.triu(torch.randn(columns, columns, generator=g) * torch.exp(spread * torch.randn(columns, columns, generator=g))).to(dev)
+    w = torch.randn(n, columns, generator=g).to(dev)
+    wide = torch.zeros(1, dtype=torch.int32, device=dev)
+    u_parts = ops.gptq_split(u, wide)
+    rows, cols = torch.triu_indices(columns, columns, device=dev)
+    assert torch.equal(u_parts.double().sum(1)[rows, cols], u.double()[rows, cols]) and int(wide) == 0
+    err_parts = _parts(err, (i2 - i1 + 63) // 32 * 32)
+    ref = w.double()
+    ref[:, i2:end] -= err.double() @ u[i1:i2, i2:end].double()
+    mag = err.double().abs() @ u[i1:i2, i2:end].double().abs()
+    for flag in (0, 1):                                   # the parts, the fp32 values themselves
+        got = w.clone()
+        ops.gptq_trail_parts(got, err, u, err_parts, u_parts, torch.full_like(wide, flag), i1, i2, end)
+        assert torch.equal(got[:, :i2], w[:, :i2]) and torch.equal(got[:, end:], w[:, end:])
+        off = (got.double() - ref).abs()[:, i2:end]
+        sums = -(-(i2 - i1) // 128)
+        bound = (2 * 2 * 24 + 2) * 2.0 ** -24 * mag + sums * 2.0 ** -24 * (w[:, i2:end].double().abs() + mag)
+        if flag:
+            bound = bound + 128 * 2.0 ** -24 * mag        # one rounding a step instead
+        assert bool((off <= bound).all()), float((off / bound).max())
+    if spread:
+        return
+    product = ref[:, i2:end] - w[:, i2:end].double()
+    off = []
+    for flag in (0, 1):
+        got = torch.zeros_like(w)
+        ops.gptq_trail_parts(got, err, u, err_parts, u_parts, torch.full_like(wide, flag), i1, i2, end)
+        off.append(float((got[:, i2:end].double() - product).norm()))
+    assert off[0] <= off[1], off
+
+
+@pytest.mark.parametrize("value", [float('inf'), float('nan'), 2.0 ** 60, -2.0 ** 127, 2.0 ** -101, 2.0 ** -140])
+def test_gptq_parts_say_what_they_do_not_hold(dev, value):
+    u = torch.triu(torch.ones(130, 130)).to(dev)
+    for at in ((0, 0), (3, 129), (129, 129)):
+        wide = torch.zeros(1, dtype=torch.int32, device=dev)
+        spoilt = u.clone()
+        spoilt[at] = value
+        ops.gptq_split(spoilt, wide)
+        assert int(wide) == 1
+    for kept in (0.0, -0.0, 2.0 ** -100, -(2.0 ** 60) * (1 - 2.0 ** -24)):
+        wide.zero_()
+        kind = u.clone()
+        kind[5, 77] = kept
+        ops.gptq_split(kind, wide)
+        assert int(wide) == 0
+
+
+@pytest.mark.parametrize("columns,block_size", [(1025, 128), (1300, 96), (1100, 640)])
+def test_gptq_layer_by_spans(dev, monkeypatch, columns, block_size):
+    """Spans of columns updated from parts against one fp32 update per block.  The two differ by roundings, which move a code
+    where one sits on a rounding boundary, and with it codes behind it in its row: few rows, if any, and the layer's error
+    on its inputs is the same to a thousandth."""
+    g = torch.Generator().manual_seed(columns)
+    w = (torch.randn(90, columns, generator=g) * 0.05).to(dev)
+    x = torch.randn(2 * columns, columns, generator=g).to(dev)
+    x[:, ::97] *= 5
+    hess = (x.t() @ x).div(x.shape[0])
+    cfg = {'weights_cfg': {'quant_type': 'int4', 'symmetric': False, 'strategy': 'channel'}}
+    if block_size > 128:
+        with pytest.raises(RuntimeError):
+            gptq.get_opt_weight_and_quant_factor(w, hess, cfg, block_size=block_size)
+        return
+    spans = gptq.get_opt_weight_and_quant_factor(w, hess, cfg, block_size=block_size)
+    monkeypatch.setattr(gptq, '_PARTS_COLUMNS', (1, 0))
+    blocks = gptq.get_opt_weight_and_quant_factor(w, hess, cfg, block_size=block_size)
+    assert torch.equal(spans[1], blocks[1]) and torch.equal(spans[2], blocks[2])
+    moved = ((spans[0] - blocks[0]).abs() > 0.5 * spans[1].reshape(-1, 1)).any(1)
+    assert int(moved.sum()) <= 5
+    # (what the column loop leaves is w - err * hinv[i][i], the code's value up to three roundings of numbers below 32 steps)
+    assert bool(((spans[0] - blocks[0]).abs() <= 2 * 3 * 32 * 2.0 ** -24 * spans[1].reshape(-1, 1))[~moved].all())
+    off = [float((x @ (w - o[0]).t()).double().pow(2).sum()) for o in (spans, blocks)]
+    assert abs(off[0] / off[1] - 1) <= 1e-3
+
+
+@pytest.mark.parametrize("n,count", [(1, 128), (70, 128), (9000, 128), (33, 32), (64, 100)])
+def test_gptq_block_gives_its_errors_in_parts(dev, n, count):
+    g = torch.Generator().manual_seed(n + count)
+    w = torch.randn(n, count, generator=g).to(dev)
+    hinv = _hinv(count, count).to(dev)
+    scale = torch.full((n,), 0.1, device=dev)
+    gidx = torch.zeros(count, dtype=torch.int32, device=dev)
+    want_w = w.clone()
+    want = gptq.gptq_block(want_w, 0, count, hinv, scale, None, gidx, -8, 7)
+    errors = torch.zeros(n, count + 28, device=dev)
+    parts = torch.zeros(n, 3, count + 28, dtype=torch.bfloat16, device=dev)
+    wide = torch.zeros(1, dtype=torch.int32, device=dev)
+    got = gptq.gptq_block(w, 0, count, hinv, scale, None, gidx, -8, 7, errors[:, :count], parts[:, :, :count], wide)
+    assert torch.equal(got, want) and torch.equal(w, want_w) and int(wide) == 0
+    assert torch.equal(parts[:, :, :count].double().sum(1), want.double())
+    assert not bool(errors[:, count:].any()) and not bool(parts[:, :, count:].any())
+    w = want_w.clone()
+    w[n // 2, count // 3] = float('inf')
+    gptq.gptq_block(w, 0, count, hinv, scale, None, gidx, -8, 7, errors[:, :count], parts[:, :, :count], wide)
+    assert int(wide) == 1
