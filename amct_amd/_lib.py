@@ -45,6 +45,7 @@ SIGNATURES = {
     "amct_hessian_update_workspace_bytes": (ctypes.c_size_t, [_L, _L]),
     "amct_hessian_update": (_I, [_P, _P, _L, _L, ctypes.c_float, ctypes.c_float, _I, _P, ctypes.c_size_t, _P]),
     "amct_hessian_update_checked": (_I, [_P, _P, _L, _L, ctypes.c_float, ctypes.c_float, _I, _P, _P, ctypes.c_size_t, _P]),
+    "amct_hessian_update_flag": (_I, [_P, _P, _L, _L, ctypes.c_float, ctypes.c_float, _I, _P, _P, ctypes.c_size_t, _P]),
     "amct_fp8_block_dequant": (_I, [_P, _P, _P, _L, _L, _I, _I, _P]),
     "amct_pack_int4_pairs_n": (_I, [_P, _P, _L, _L, _P]),
     "amct_scale_f32_to_u64": (_I, [_P, _P, _L, _P]),
@@ -54,6 +55,8 @@ SIGNATURES = {
     "amct_awq_loss_workspace_bytes": (ctypes.c_size_t, []),
     "amct_awq_loss": (_I, [_P, _P, _L, _I, _P, _P, ctypes.c_size_t, _P]),
     "amct_scale_offset": (_I, [_P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _P]),
+    "amct_scale_offset_flag": (_I, [_P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _P]),
+    "amct_stream_wait": (_I, [_P]),
     "amct_quant_with_params": (_I, [_P, _P, _P, _P, _P, _I, _P, _I, _L, _L, _I, _I, _I, _I, _I, _I, _P]),
     "amct_fakequant_int": (_I, [_P, _P, _P, _I, _P, _P, _P, _P, _I, _L, _L, _I, _I, _I, _I, _I, _I, _I, _I, _P]),
     "amct_quant_int4_group_pack": (_I, [_P, _P, _P, _I, _P, _P, _P, _P, _I, _L, _L, _I, _I, _I, _P]),

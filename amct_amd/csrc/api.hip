@@ -114,6 +114,12 @@ extern "C" int amct_mfma_yardstick(int bf16, int random_operands, int iters, voi
     return amct::hip_status();
 }
 
+extern "C" int amct_stream_wait(amct_stream_t stream) {
+    if (hipStreamSynchronize((hipStream_t)stream) == hipSuccess) return AMCT_OK;
+    (void)hipGetLastError();
+    return AMCT_E_HIP;
+}
+
 extern "C" int amct_copy_bytes(const void* src, void* dst, int64_t nbytes, amct_stream_t stream) {
     if (nbytes < 0 || (nbytes != 0 && (!src || !dst))) return AMCT_E_BADARG;
     if (nbytes % 16 != 0 || !amct::aligned16(src) || !amct::aligned16(dst)) return AMCT_E_ALIGN;

@@ -561,13 +561,14 @@ __global__ __launch_bounds__(kBlock) void minmax_rows(const void* w, float* mn_o
 
 template <int DT>
 __global__ __launch_bounds__(kBlock) void scale_offset_k(const void* mx, const void* mn, float* scale, int32_t* offset,
-                                                         int32_t* bad, int64_t n, int bits, int symmetric, int scope_rule) {
+                                                         int32_t* bad, int32_t* flag, int64_t n, int bits, int symmetric, int scope_rule) {
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
     const Factors f = make_factors<DT>(load_scalar<DT>(mx, i), load_scalar<DT>(mn, i), bits, symmetric != 0, scope_rule);
     scale[i] = f.s;
     if (offset && !symmetric) offset[i] = (int32_t)f.z;
     if (f.bad && bad) atomicAdd(bad, 1);
+    if (f.bad && flag) *flag = 1;                    // (a store: the flag may be host memory)
 }
 
 // ---------------------------------------------------------------------------
@@ -706,9 +707,8 @@ extern "C" int amct_minmax(const void* w, float* mn, float* mx, int64_t rows, in
     return hip_status();
 }
 
-extern "C" int amct_scale_offset(const void* mx, const void* mn, float* scale, int32_t* offset, int32_t* bad_count,
-                                 int64_t n, int bits, int symmetric, int scope_rule, int in_dtype,
-                                 amct_stream_t stream) {
+static int scale_offset_launch(const void* mx, const void* mn, float* scale, int32_t* offset, int32_t* bad_count, int32_t* flag,
+                               int64_t n, int bits, int symmetric, int scope_rule, int in_dtype, amct_stream_t stream) {
     if (n < 0 || (bits != 4 && bits != 8)) return AMCT_E_BADARG;
     if (n == 0) return AMCT_OK;
     if (!mx || !mn || !scale) return AMCT_E_BADARG;
@@ -717,17 +717,29 @@ extern "C" int amct_scale_offset(const void* mx, const void* mn, float* scale, i
     hipStream_t st = (hipStream_t)stream;
     switch (in_dtype) {
         case AMCT_F32:
-            hipLaunchKernelGGL((scale_offset_k<AMCT_F32>), dim3(nb), dim3(kBlock), 0, st, mx, mn, scale, offset, bad_count, n, bits, symmetric, scope_rule);
+            hipLaunchKernelGGL((scale_offset_k<AMCT_F32>), dim3(nb), dim3(kBlock), 0, st, mx, mn, scale, offset, bad_count, flag, n, bits, symmetric, scope_rule);
             break;
         case AMCT_F16:
-            hipLaunchKernelGGL((scale_offset_k<AMCT_F16>), dim3(nb), dim3(kBlock), 0, st, mx, mn, scale, offset, bad_count, n, bits, symmetric, scope_rule);
+            hipLaunchKernelGGL((scale_offset_k<AMCT_F16>), dim3(nb), dim3(kBlock), 0, st, mx, mn, scale, offset, bad_count, flag, n, bits, symmetric, scope_rule);
             break;
         case AMCT_BF16:
-            hipLaunchKernelGGL((scale_offset_k<AMCT_BF16>), dim3(nb), dim3(kBlock), 0, st, mx, mn, scale, offset, bad_count, n, bits, symmetric, scope_rule);
+            hipLaunchKernelGGL((scale_offset_k<AMCT_BF16>), dim3(nb), dim3(kBlock), 0, st, mx, mn, scale, offset, bad_count, flag, n, bits, symmetric, scope_rule);
             break;
         default: return AMCT_E_BADARG;
     }
     return hip_status();
+}
+
+extern "C" int amct_scale_offset(const void* mx, const void* mn, float* scale, int32_t* offset, int32_t* bad_count,
+                                 int64_t n, int bits, int symmetric, int scope_rule, int in_dtype,
+                                 amct_stream_t stream) {
+    return scale_offset_launch(mx, mn, scale, offset, bad_count, nullptr, n, bits, symmetric, scope_rule, in_dtype, stream);
+}
+
+extern "C" int amct_scale_offset_flag(const void* mx, const void* mn, float* scale, int32_t* offset, int32_t* flag,
+                                      int64_t n, int bits, int symmetric, int scope_rule, int in_dtype,
+                                      amct_stream_t stream) {
+    return scale_offset_launch(mx, mn, scale, offset, nullptr, flag, n, bits, symmetric, scope_rule, in_dtype, stream);
 }
 
 extern "C" int amct_quant_with_params(const void* w, const float* scale, const int32_t* offset, void* dq, void* codes,

@@ -386,13 +386,26 @@ extern "C" size_t amct_hessian_update_workspace_bytes(int64_t tokens, int64_t co
     return (size_t)hs_round_up(cols, 128) * (size_t)hs_round_up(tokens, kHsK) * 2;
 }
 
+static int hessian_launch(float* hessian, const void* x, int64_t tokens, int64_t cols, float beta, float alpha, int dtype, int32_t* bad,
+                          bool clear, void* workspace, size_t workspace_bytes, amct_stream_t stream);
+
 extern "C" int amct_hessian_update(float* hessian, const void* x, int64_t tokens, int64_t cols, float beta, float alpha,
                                    int dtype, void* workspace, size_t workspace_bytes, amct_stream_t stream) {
-    return amct_hessian_update_checked(hessian, x, tokens, cols, beta, alpha, dtype, nullptr, workspace, workspace_bytes, stream);
+    return hessian_launch(hessian, x, tokens, cols, beta, alpha, dtype, nullptr, false, workspace, workspace_bytes, stream);
 }
 
 extern "C" int amct_hessian_update_checked(float* hessian, const void* x, int64_t tokens, int64_t cols, float beta, float alpha,
                                            int dtype, int32_t* bad, void* workspace, size_t workspace_bytes, amct_stream_t stream) {
+    return hessian_launch(hessian, x, tokens, cols, beta, alpha, dtype, bad, true, workspace, workspace_bytes, stream);
+}
+
+extern "C" int amct_hessian_update_flag(float* hessian, const void* x, int64_t tokens, int64_t cols, float beta, float alpha, int dtype,
+                                        int32_t* flag, void* workspace, size_t workspace_bytes, amct_stream_t stream) {
+    return hessian_launch(hessian, x, tokens, cols, beta, alpha, dtype, flag, false, workspace, workspace_bytes, stream);
+}
+
+static int hessian_launch(float* hessian, const void* x, int64_t tokens, int64_t cols, float beta, float alpha, int dtype, int32_t* bad,
+                          bool clear, void* workspace, size_t workspace_bytes, amct_stream_t stream) {
     if (tokens < 0 || cols <= 0 || !hessian) return AMCT_E_BADARG;
     if (dtype != AMCT_BF16 && dtype != AMCT_F16) return AMCT_E_UNSUPPORTED;
     if (tokens != 0 && !x) return AMCT_E_BADARG;
@@ -404,7 +417,7 @@ extern "C" int amct_hessian_update_checked(float* hessian, const void* x, int64_
     hipStream_t st = (hipStream_t)stream;
     SyrkArgs a{reinterpret_cast<const uint16_t*>(x), hessian, tokens, cols, cols, 0, 0, 0, beta, alpha,
                cols % 4 == 0 && aligned16(hessian), bad};
-    if (bad) hipLaunchKernelGGL(hess_clear_k, dim3(1), dim3(1), 0, st, bad);
+    if (bad && clear) hipLaunchKernelGGL(hess_clear_k, dim3(1), dim3(1), 0, st, bad);
     if (cols % 8 != 0 || !aligned16(x)) {
         a.ld = hs_round_up(cols, 8);
         if (tokens > 0)

@@ -212,6 +212,19 @@ def awq_candidates(mean, ratios):
     return out
 
 
+def host_flags(n):
+    """n zeroed int32 values in pinned host memory, for kernels to store to; see read_flags."""
+    return torch.zeros(n, dtype=torch.int32, pin_memory=True)
+
+
+def read_flags(flags, dev):
+    """The values of host_flags() when everything enqueued on dev's current stream has run: no launch that clears them and no copy
+    back (W[4096,4096] fp32, extrema, factors and fake-quantised weight: 56.4 us, with a device tensor and .item() 60.1)."""
+    with _on(dev):
+        _lib.check(_lib.load().amct_stream_wait(_stream(dev)))
+    return flags.tolist()
+
+
 class AwqLosses:
     """mean((y - yhat)^4) of every grid point of a search against one target, nothing read back until winner()."""
 
@@ -237,27 +250,28 @@ class AwqLosses:
             return -1
         dev = self.target.device
         losses = torch.empty(self.grids, dtype=torch.float32, device=dev)
-        at = torch.empty(1, dtype=torch.int32, device=dev)
+        at = host_flags(1)
         with _on(dev):
             _lib.check(self._lib.amct_awq_pick(_p(self._partials), self.target.numel(), dtype_code(self.target.dtype), self.grids,
                                                _p(losses), _p(at), _stream(dev)))
-        return int(at)
+        return read_flags(at, dev)[0]
 
 
 def nonfinite_flags(tensors):
     """One truth value per tensor: whether it holds an infinity or a NaN (one read-back for all of them)."""
     dev = _dev(*tensors)
-    flags = torch.zeros(len(tensors), dtype=torch.int32, device=dev)
+    flags = host_flags(len(tensors))
     with _on(dev):
         for i, t in enumerate(tensors):
             t = _c(t)
             _lib.check(_lib.load().amct_flag_nonfinite(_p(t), t.numel(), dtype_code(t.dtype), flags.data_ptr() + 4 * i, _stream(dev)))
-    return [bool(f) for f in flags.tolist()]
+    return [bool(f) for f in read_flags(flags, dev)]
 
 
-def hessian_update(hessian, x, beta, alpha, bad=None):
+def hessian_update(hessian, x, beta, alpha, bad=None, flag=None):
     """hessian [C,C] fp32 <- beta * hessian + alpha * x^T x in place, x [tokens, C] bf16|f16 (gptq_module.py:176-181).
-    beta == 0 does not read hessian.  bad (int32, one element) becomes 1 if the new hessian is not finite, 0 if it is."""
+    beta == 0 does not read hessian.  bad (int32, one element) becomes 1 if the new hessian is not finite, 0 if it is;
+    flag (of host_flags) becomes 1 in that case and is left alone in the other."""
     dev = _dev(hessian, x, bad)
     _need(bad is None or (bad.dtype == torch.int32 and bad.numel() == 1), "hessian_update: bad must be one int32 value")
     _need(hessian.dim() == 2 and hessian.shape[0] == hessian.shape[1] and hessian.dtype == torch.float32 and
@@ -270,8 +284,9 @@ def hessian_update(hessian, x, beta, alpha, bad=None):
     nbytes = lib.amct_hessian_update_workspace_bytes(tokens, cols)
     ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev)
     with _on(dev):
-        _lib.check(lib.amct_hessian_update_checked(_p(hessian), _p(x), tokens, cols, float(beta), float(alpha),
-                                                   dtype_code(x.dtype), _p(bad), _p(ws), ws.numel(), _stream(dev)))
+        update = lib.amct_hessian_update_checked if flag is None else lib.amct_hessian_update_flag
+        _lib.check(update(_p(hessian), _p(x), tokens, cols, float(beta), float(alpha), dtype_code(x.dtype),
+                          _p(bad if flag is None else flag), _p(ws), ws.numel(), _stream(dev)))
     return hessian
 
 
@@ -371,8 +386,9 @@ def gptq_factor(hessian, perm, damp, bad):
     return u
 
 
-def scale_offset(vmax, vmin, bits, symmetric, scope_rule=SCOPE_AMCT, bad=None):
-    """Elementwise (max, min) -> (scale fp32, offset int32 | None), same shape as the inputs."""
+def scale_offset(vmax, vmin, bits, symmetric, scope_rule=SCOPE_AMCT, bad=None, flag=None):
+    """Elementwise (max, min) -> (scale fp32, offset int32 | None), same shape as the inputs.  bad (int32 on the device) counts the
+    entries that are not finite; flag (of host_flags) becomes 1 if there are any."""
     dev = _dev(vmax, vmin, bad)
     if vmax.dtype != vmin.dtype or vmax.shape != vmin.shape:
         raise RuntimeError("max and min must share dtype and shape")
@@ -380,8 +396,9 @@ def scale_offset(vmax, vmin, bits, symmetric, scope_rule=SCOPE_AMCT, bad=None):
     scale = torch.empty(vmax.shape, dtype=torch.float32, device=dev)
     offset = None if symmetric else torch.empty(vmax.shape, dtype=torch.int32, device=dev)
     with _on(dev):
-        _lib.check(_lib.load().amct_scale_offset(_p(vmax), _p(vmin), _p(scale), _p(offset), _p(bad), vmax.numel(), bits,
-                                                 int(symmetric), scope_rule, dtype_code(vmax.dtype), _stream(dev)))
+        factors = _lib.load().amct_scale_offset if flag is None else _lib.load().amct_scale_offset_flag
+        _lib.check(factors(_p(vmax), _p(vmin), _p(scale), _p(offset), _p(bad if flag is None else flag), vmax.numel(), bits,
+                           int(symmetric), scope_rule, dtype_code(vmax.dtype), _stream(dev)))
     return scale, offset
 
 

@@ -29,9 +29,9 @@ def update_hessian(hessian, nsamples, input_data, columns):
         else:
             beta = nsamples / (nsamples + batch_size)
         nsamples += batch_size
-        bad = torch.empty(1, dtype=torch.int32, device=rows.device)
-        hessian = ops.hessian_update(hessian, rows, beta, 2 / nsamples, bad)
-        finite = not int(bad)
+        flag = ops.host_flags(1)
+        hessian = ops.hessian_update(hessian, rows, beta, 2 / nsamples, flag=flag)
+        finite = not ops.read_flags(flag, rows.device)[0]
     else:
         # fp32 activations keep the fp32 product
         x = rows.t()

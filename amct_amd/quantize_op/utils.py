@@ -28,16 +28,16 @@ def get_int_quant_scope(data_type, symmetric, abs_max_is_negative=False):
 
 def calculate_scale_offset(data_max, data_min, symmetric, data_type, check=True):
     """(scale fp32, offset int32 | None), shaped like data_max (utils.py:75-108).  Raises the
-    reference's RuntimeError when a factor is not finite.  That check reads a flag back from the device, which
-    synchronises the stream: check=False skips it for callers inside a loop (the factors are computed the same
-    way, a non-finite one is simply not reported) -- validate once afterwards with check_scale_offset."""
+    reference's RuntimeError when a factor is not finite.  That check waits for the stream: check=False skips it for
+    callers inside a loop (the factors are computed the same way, a non-finite one is simply not reported) -- validate
+    once afterwards with check_scale_offset."""
     bits = int(data_type.replace('int', ''))
     dev = data_max.device
     if not check:
         return ops.scale_offset(data_max, data_min, bits, bool(symmetric))
-    bad = torch.zeros(2, dtype=torch.int32, device=dev)
-    scale, offset = ops.scale_offset(data_max, data_min, bits, bool(symmetric), bad=bad[:1])
-    if int(bad[0].item()):
+    flag = ops.host_flags(1)
+    scale, offset = ops.scale_offset(data_max, data_min, bits, bool(symmetric), flag=flag)
+    if ops.read_flags(flag, dev)[0]:
         # find which message the reference would give
         check_scale_offset(scale, None)
         raise RuntimeError("Param offset has invalid value inf or nan!")

@@ -6,7 +6,7 @@
  *   - every pointer is a DEVICE pointer unless its name ends in _host;
  *   - tensors are dense and row-major; 16-byte aligned bases take the fast
  *     kernels, anything else a slower general kernel (same results);
- *   - the library never allocates, frees or synchronises: the caller owns all
+ *   - the library never allocates, frees or synchronises (but for amct_stream_wait): the caller owns all
  *     buffers (including workspaces) and supplies the stream; every call only
  *     enqueues work on `stream` and returns (amct_col_minmax_noalloc keeps its
  *     workspace in a fixed device array of the library instead);
@@ -162,6 +162,14 @@ int amct_minmax(const void* w, float* mn, float* mx, int64_t rows, int64_t cols,
 int amct_scale_offset(const void* mx, const void* mn, float* scale, int32_t* offset, int32_t* bad_count,
                       int64_t n, int bits, int symmetric, int scope_rule, int in_dtype,
                       amct_stream_t stream);
+
+/* The same, and *flag = 1 (a store, not a count; never cleared) where an entry is not finite: flag may be pinned host memory,
+ * which the host zeroes beforehand and reads after amct_stream_wait -- no launch that clears it, no copy back. */
+int amct_scale_offset_flag(const void* mx, const void* mn, float* scale, int32_t* offset, int32_t* flag,
+                           int64_t n, int bits, int symmetric, int scope_rule, int in_dtype,
+                           amct_stream_t stream);
+/* Waits until everything enqueued on the stream has run (the one entry point that does). */
+int amct_stream_wait(amct_stream_t stream);
 
 /* ---- A3 / A4 / A5 / A6: quantise with given factors -------------------------------------
  * Replaces quant_dequant_weight (amct_pytorch/utils/quant_util.py:162-188), quant_weight +
@@ -451,6 +459,9 @@ int amct_hessian_update(float* hessian, const void* x, int64_t tokens, int64_t c
 /* The same, and *bad (int32 on the device) = 1 if an element of the new hessian is not finite, 0 if all are. */
 int amct_hessian_update_checked(float* hessian, const void* x, int64_t tokens, int64_t cols, float beta, float alpha, int dtype,
                                 int32_t* bad, void* workspace, size_t workspace_bytes, amct_stream_t stream);
+/* The same with a flag as in amct_scale_offset_flag: set to 1, never cleared, pinned host memory or device memory. */
+int amct_hessian_update_flag(float* hessian, const void* x, int64_t tokens, int64_t cols, float beta, float alpha, int dtype,
+                             int32_t* flag, void* workspace, size_t workspace_bytes, amct_stream_t stream);
 
 /* ---- interchange formats of the checkpoint converter ---------------------------------------
  * (amct_pytorch/experimental/quantization/DeepSeekV3.2/deploy.py)
