@@ -212,17 +212,21 @@ def awq_candidates(mean, ratios):
     return out
 
 
-def host_flags(n):
-    """n zeroed int32 values in pinned host memory, for kernels to store to; see read_flags."""
-    return torch.zeros(n, dtype=torch.int32, pin_memory=True)
-
-
-def read_flags(flags, dev):
-    """The values of host_flags() when everything enqueued on dev's current stream has run: no launch that clears them and no copy
-    back (W[4096,4096] fp32, extrema, factors and fake-quantised weight: 56.4 us, with a device tensor and .item() 60.1)."""
+def with_host_flag(tensor, run):
+    """(run(flag), whether a kernel that it enqueued on the tensor's device has set flag): one zeroed int32 in pinned host memory
+    that kernels store to, read when the stream has got there -- no launch that clears it, no copy back (W[4096,4096] fp32,
+    extrema, factors and fake-quantised weight: 56.4 us, with a device tensor and .item() 60.1).  The stream is waited for also
+    when run raises, since the memory is given back after it.  Where the wait is long the copy back costs nothing (a search of 20
+    AWQ grid points: 1585 us this way, 1560 that way): those callers read a device tensor."""
+    dev = _dev(tensor)
     with _on(dev):
-        _lib.check(_lib.load().amct_stream_wait(_stream(dev)))
-    return flags.tolist()
+        flag = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        try:
+            out = run(flag)
+        finally:
+            status = _lib.load().amct_stream_wait(_stream(dev))
+        _lib.check(status)
+    return out, bool(flag)
 
 
 class AwqLosses:
@@ -250,28 +254,28 @@ class AwqLosses:
             return -1
         dev = self.target.device
         losses = torch.empty(self.grids, dtype=torch.float32, device=dev)
-        at = host_flags(1)
+        at = torch.empty(1, dtype=torch.int32, device=dev)
         with _on(dev):
             _lib.check(self._lib.amct_awq_pick(_p(self._partials), self.target.numel(), dtype_code(self.target.dtype), self.grids,
                                                _p(losses), _p(at), _stream(dev)))
-        return read_flags(at, dev)[0]
+        return int(at)
 
 
 def nonfinite_flags(tensors):
     """One truth value per tensor: whether it holds an infinity or a NaN (one read-back for all of them)."""
     dev = _dev(*tensors)
-    flags = host_flags(len(tensors))
+    flags = torch.zeros(len(tensors), dtype=torch.int32, device=dev)
     with _on(dev):
         for i, t in enumerate(tensors):
             t = _c(t)
             _lib.check(_lib.load().amct_flag_nonfinite(_p(t), t.numel(), dtype_code(t.dtype), flags.data_ptr() + 4 * i, _stream(dev)))
-    return [bool(f) for f in read_flags(flags, dev)]
+    return [bool(f) for f in flags.tolist()]
 
 
 def hessian_update(hessian, x, beta, alpha, bad=None, flag=None):
     """hessian [C,C] fp32 <- beta * hessian + alpha * x^T x in place, x [tokens, C] bf16|f16 (gptq_module.py:176-181).
     beta == 0 does not read hessian.  bad (int32, one element) becomes 1 if the new hessian is not finite, 0 if it is;
-    flag (of host_flags) becomes 1 in that case and is left alone in the other."""
+    flag (pinned, see with_host_flag) becomes 1 in that case and is left alone in the other."""
     dev = _dev(hessian, x, bad)
     _need(bad is None or (bad.dtype == torch.int32 and bad.numel() == 1), "hessian_update: bad must be one int32 value")
     _need(hessian.dim() == 2 and hessian.shape[0] == hessian.shape[1] and hessian.dtype == torch.float32 and
@@ -388,7 +392,7 @@ def gptq_factor(hessian, perm, damp, bad):
 
 def scale_offset(vmax, vmin, bits, symmetric, scope_rule=SCOPE_AMCT, bad=None, flag=None):
     """Elementwise (max, min) -> (scale fp32, offset int32 | None), same shape as the inputs.  bad (int32 on the device) counts the
-    entries that are not finite; flag (of host_flags) becomes 1 if there are any."""
+    entries that are not finite; flag (pinned, see with_host_flag) becomes 1 if there are any."""
     dev = _dev(vmax, vmin, bad)
     if vmax.dtype != vmin.dtype or vmax.shape != vmin.shape:
         raise RuntimeError("max and min must share dtype and shape")

@@ -29,9 +29,9 @@ def update_hessian(hessian, nsamples, input_data, columns):
         else:
             beta = nsamples / (nsamples + batch_size)
         nsamples += batch_size
-        flag = ops.host_flags(1)
-        hessian = ops.hessian_update(hessian, rows, beta, 2 / nsamples, flag=flag)
-        finite = not ops.read_flags(flag, rows.device)[0]
+        hessian, bad = ops.with_host_flag(
+            rows, lambda flag: ops.hessian_update(hessian, rows, beta, 2 / nsamples, flag=flag))
+        finite = not bad
     else:
         # fp32 activations keep the fp32 product
         x = rows.t()

@@ -32,12 +32,11 @@ def calculate_scale_offset(data_max, data_min, symmetric, data_type, check=True)
     callers inside a loop (the factors are computed the same way, a non-finite one is simply not reported) -- validate
     once afterwards with check_scale_offset."""
     bits = int(data_type.replace('int', ''))
-    dev = data_max.device
     if not check:
         return ops.scale_offset(data_max, data_min, bits, bool(symmetric))
-    flag = ops.host_flags(1)
-    scale, offset = ops.scale_offset(data_max, data_min, bits, bool(symmetric), flag=flag)
-    if ops.read_flags(flag, dev)[0]:
+    (scale, offset), bad = ops.with_host_flag(
+        data_max, lambda flag: ops.scale_offset(data_max, data_min, bits, bool(symmetric), flag=flag))
+    if bad:
         # find which message the reference would give
         check_scale_offset(scale, None)
         raise RuntimeError("Param offset has invalid value inf or nan!")

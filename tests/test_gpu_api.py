@@ -501,3 +501,30 @@ def test_awq_pick_and_nonfinite_flags(dev):
             a = x.clone()
             a[0] = float('nan')
             assert ops.nonfinite_flags([x, z, a, torch.ones(size + 1, device=dev, dtype=dtype)[1:]]) == [False, True, True, False]
+
+
+@pytest.mark.parametrize("count", [1, 255, 257, 5000])
+def test_checks_answered_through_host_memory(dev, count):
+    """The flag that a call reads before it returns: left at zero by finite factors and sums, set by one value that is not, in
+    the first and the last place, also on another stream than the default one; the error of a refused launch comes through."""
+    high = torch.rand(count, device=dev) + 1
+    for at in (None, 0, count - 1):
+        top = high.clone()
+        if at is not None:
+            top[at] = float('inf')
+        stream = torch.cuda.Stream()
+        stream.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            (scale, _), bad = ops.with_host_flag(top, lambda flag: ops.scale_offset(top, -top, 8, True, flag=flag))
+        torch.cuda.current_stream().wait_stream(stream)
+        assert bad is (at is not None) and torch.equal(scale, ops.scale_offset(top, -top, 8, True)[0])
+    columns = min(count, 640)
+    x = torch.randn(40, columns, device=dev).bfloat16()
+    hess = torch.empty(columns, columns, device=dev)
+    for at in (None, 0, columns - 1):
+        rows = x.clone()
+        if at is not None:
+            rows[39, at] = float('nan')
+        assert ops.with_host_flag(rows, lambda flag: ops.hessian_update(hess, rows, 0.0, 1.0, flag=flag))[1] is (at is not None)
+    with pytest.raises(RuntimeError):
+        ops.with_host_flag(high, lambda flag: ops.scale_offset(high, high[:0], 8, True, flag=flag))
