@@ -101,6 +101,9 @@ __global__ __launch_bounds__(kBlock) void awq_loss_final_k(const float* partial,
 // mean ** ratio rounded to the activations' dtype and clamped at 1e-4, divided in fp64 by the geometric mean of its extremes,
 // rounded to the dtype and clamped into [1e-4, largest finite].  As thirteen library launches per grid point these took
 // longer than the fake-quantised weight they are for.  The powers are kept in the output between the two passes.
+// 16 waves a block: a grid point is one block's work, and powers and fp64 quotients are long chains (20 points of 4096
+// columns: 15.5 us with 4 waves, now 8.9).
+constexpr int kCandThreads = 1024;
 template <int DT> AMCT_DEV float dtype_max() { return DT == AMCT_F16 ? 65504.f : DT == AMCT_BF16 ? 3.38953138925153547590e38f : 3.40282346638528859812e38f; }
 // torch.clamp of a value of the dtype: NaN stays NaN, the bound is rounded to the dtype
 template <int DT> AMCT_DEV float clamp_low(float v) {
@@ -109,13 +112,13 @@ template <int DT> AMCT_DEV float clamp_low(float v) {
 }
 
 template <int DT>
-__global__ __launch_bounds__(kBlock) void awq_candidates_k(const void* mean, const float* ratios, void* out, int64_t cols) {
-    __shared__ float smx[kBlock / 64], smn[kBlock / 64];
+__global__ __launch_bounds__(kCandThreads) void awq_candidates_k(const void* mean, const float* ratios, void* out, int64_t cols) {
+    __shared__ float smx[kCandThreads / 64], smn[kCandThreads / 64];
     const int tid = threadIdx.x;
     const float ratio = ratios[blockIdx.x];
     const int64_t base = (int64_t)blockIdx.x * cols;
     float mx = -__builtin_inff(), mn = __builtin_inff();
-    for (int64_t c = tid; c < cols; c += kBlock) {
+    for (int64_t c = tid; c < cols; c += kCandThreads) {
         const float x = load_scalar<DT>(mean, c);
         // the square root and the zeroth power as such, as the library's power does
         const float p = ratio == 0.5f ? sqrtf(x) : ratio == 0.f ? 1.f : powf(x, ratio);
@@ -131,12 +134,12 @@ __global__ __launch_bounds__(kBlock) void awq_candidates_k(const void* mean, con
     }
     __syncthreads();
 #pragma unroll
-    for (int w = 0; w < kBlock / 64; ++w) {
+    for (int w = 0; w < kCandThreads / 64; ++w) {
         mx = fmax_nan(mx, smx[w]);
         mn = fmin_nan(mn, smn[w]);
     }
     const double norm = sqrt((double)mx * (double)mn);
-    for (int64_t c = tid; c < cols; c += kBlock) {                 // a thread reads back what it wrote
+    for (int64_t c = tid; c < cols; c += kCandThreads) {                 // a thread reads back what it wrote
         const double q = (double)load_scalar<DT>(out, base + c) / norm;
         const float v = clamp_low<DT>(round_to<DT>((float)q));
         store_scalar<DT>(out, base + c, v > dtype_max<DT>() ? dtype_max<DT>() : v);
@@ -145,28 +148,75 @@ __global__ __launch_bounds__(kBlock) void awq_candidates_k(const void* mean, con
 
 // The losses of a search from the partials of its grid points (kLossBlocks apart), folded as awq_loss_final_k folds them,
 // and the first grid point whose loss is below infinity and below every earlier one: -1 if there is none.
-__global__ __launch_bounds__(kBlock) void awq_pick_k(const float* partials, int nparts, int64_t n, int grids, float* losses, int32_t* winner) {
-    __shared__ float red[kBlock / 64];
-    const int tid = threadIdx.x;
+// One block; a wave folds a quarter of a grid point's partials (lane l of quarter w those of l + 64 w, + 256, ...) with the
+// loads of four quarters in flight, kPickGrids grid points between two barriers.  Bound by the latency of its loads: one grid
+// point after the other, each behind the barriers of the one before, took 19 us for 20 of them, now 4.5 us.
+constexpr int kPickThreads = 1024;
+constexpr int kPickGrids = 64;                      // a lane of the first wave each, for the choice
+constexpr int kPickLoads = kLossBlocks / kBlock;   // partials of a lane at most
+
+__global__ __launch_bounds__(kPickThreads) void awq_pick_k(const float* partials, int nparts, int64_t n, int grids, float* losses, int32_t* winner) {
+    constexpr int W = kBlock / 64, kWaves = kPickThreads / 64, kTasks = 4;
+    __shared__ float red[kPickGrids * W];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     float best = __builtin_inff();
     int at = -1;
-    for (int g = 0; g < grids; ++g) {
-        float t = 0.f;
-        for (int i = tid; i < nparts; i += kBlock) t = t + partials[(int64_t)g * kLossBlocks + i];
+    for (int g0 = 0; g0 < grids; g0 += kPickGrids) {
+        const int count = grids - g0 < kPickGrids ? grids - g0 : kPickGrids;
+        if (g0) __syncthreads();
+        for (int t0 = wave; t0 < count * W; t0 += kWaves * kTasks) {
+            float p[kTasks][kPickLoads];
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) t = t + __shfl_xor(t, off, 64);
-        if (g) __syncthreads();
-        if ((tid & 63) == 0) red[tid >> 6] = t;
+            for (int k = 0; k < kTasks; ++k) {
+                const int t = t0 + k * kWaves < count * W ? t0 + k * kWaves : t0;
+                const float* src = partials + (int64_t)(g0 + t / W) * kLossBlocks;
+#pragma unroll
+                for (int l = 0; l < kPickLoads; ++l) {
+                    const int i = (t % W) * 64 + lane + l * kBlock;
+                    p[k][l] = src[i < nparts ? i : nparts - 1];
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < kTasks; ++k) {
+                const int t = t0 + k * kWaves;
+                if (t >= count * W) break;
+                float sum = 0.f;
+#pragma unroll
+                for (int l = 0; l < kPickLoads; ++l) {
+                    if ((t % W) * 64 + lane + l * kBlock < nparts) sum = sum + p[k][l];
+                }
+#pragma unroll
+                for (int off = 32; off > 0; off >>= 1) sum = sum + __shfl_xor(sum, off, 64);
+                if (lane == 0) red[t] = sum;
+            }
+        }
         __syncthreads();
-        if (tid == 0) {
-            float b = red[0];
+        if (wave == 0) {
+            float b = __builtin_inff();
+            int mine = 0x7FFFFFFF;
+            if (lane < count) {
+                float v = red[lane * W];
 #pragma unroll
-            for (int w = 1; w < kBlock / 64; ++w) b = b + red[w];
-            b = b / (float)n;
-            losses[g] = b;
-            if (b < best) {                          // false for NaN
+                for (int w = 1; w < W; ++w) v = v + red[lane * W + w];
+                v = v / (float)n;
+                losses[g0 + lane] = v;
+                if (v < b) {                         // false for NaN
+                    b = v;
+                    mine = g0 + lane;
+                }
+            }
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) {
+                const float ob = __shfl_xor(b, off, 64);
+                const int om = __shfl_xor(mine, off, 64);
+                if (ob < b || (ob == b && om < mine)) {
+                    b = ob;
+                    mine = om;
+                }
+            }
+            if (b < best) {
                 best = b;
-                at = g;
+                at = mine;
             }
         }
     }
@@ -243,7 +293,7 @@ extern "C" int amct_awq_loss_partials(const void* y, const void* yhat, int64_t n
 
 extern "C" int amct_awq_pick(const float* partials, int64_t n, int dtype, int grids, float* losses, int32_t* winner, amct_stream_t stream) {
     if (!loss_args_ok(n, dtype) || grids <= 0 || !partials || !losses || !winner) return AMCT_E_BADARG;
-    hipLaunchKernelGGL(awq_pick_k, dim3(1), dim3(kBlock), 0, (hipStream_t)stream, partials, loss_blocks(n, dtype), n, grids, losses, winner);
+    hipLaunchKernelGGL(awq_pick_k, dim3(1), dim3(kPickThreads), 0, (hipStream_t)stream, partials, loss_blocks(n, dtype), n, grids, losses, winner);
     return hip_status();
 }
 
@@ -255,9 +305,9 @@ extern "C" int amct_awq_candidates(const void* mean, const float* ratios, void* 
     const dim3 grid((unsigned)grids);
     hipStream_t st = (hipStream_t)stream;
     switch (dtype) {
-        case AMCT_F32: hipLaunchKernelGGL((awq_candidates_k<AMCT_F32>), grid, dim3(kBlock), 0, st, mean, ratios, out, cols); break;
-        case AMCT_F16: hipLaunchKernelGGL((awq_candidates_k<AMCT_F16>), grid, dim3(kBlock), 0, st, mean, ratios, out, cols); break;
-        case AMCT_BF16: hipLaunchKernelGGL((awq_candidates_k<AMCT_BF16>), grid, dim3(kBlock), 0, st, mean, ratios, out, cols); break;
+        case AMCT_F32: hipLaunchKernelGGL((awq_candidates_k<AMCT_F32>), grid, dim3(kCandThreads), 0, st, mean, ratios, out, cols); break;
+        case AMCT_F16: hipLaunchKernelGGL((awq_candidates_k<AMCT_F16>), grid, dim3(kCandThreads), 0, st, mean, ratios, out, cols); break;
+        case AMCT_BF16: hipLaunchKernelGGL((awq_candidates_k<AMCT_BF16>), grid, dim3(kCandThreads), 0, st, mean, ratios, out, cols); break;
         default: return AMCT_E_BADARG;
     }
     return hip_status();

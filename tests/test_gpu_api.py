@@ -528,3 +528,38 @@ def test_checks_answered_through_host_memory(dev, count):
         assert ops.with_host_flag(rows, lambda flag: ops.hessian_update(hess, rows, 0.0, 1.0, flag=flag))[1] is (at is not None)
     with pytest.raises(RuntimeError):
         ops.with_host_flag(high, lambda flag: ops.scale_offset(high, high[:0], 8, True, flag=flag))
+
+
+@pytest.mark.parametrize("grids", [1, 20, 63, 64, 65, 150])
+@pytest.mark.parametrize("n", [1, 4099, 700001, 9000000])
+def test_awq_pick_is_the_first_smallest_loss(dev, grids, n):
+    """Grid points in any number (64 are folded between two barriers), partials from one to the full 1024: the losses of single
+    calls bit for bit, the first of the smallest among them, NaN and infinity never."""
+    y = torch.randn(n, device=dev).bfloat16()
+    losses = ops.AwqLosses(y, grids)
+    g = torch.Generator().manual_seed(grids + n)
+    kinds = torch.randint(0, 6, (grids,), generator=g).tolist()
+    outs = [y + 2.0, y + 1.0, y + 1.5, y * float('nan'), torch.full_like(y, float('inf')), y + 3.0]
+    want = [float(ops.awq_loss(y, o)) for o in outs]
+    for i, k in enumerate(kinds):
+        losses.add(i, outs[k])
+    best, at = float('inf'), -1
+    for i, k in enumerate(kinds):
+        if want[k] < best:
+            best, at = want[k], i
+    assert losses.winner() == at
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("cols", [1, 63, 1023, 1025, 5120])
+def test_awq_candidates_at_the_edges_of_a_block(dev, dtype, cols):
+    """The zeroth power is 1 and its quotient too.  The square root is the device library's, within one unit in the last place:
+    that moves a root by at most eps of the dtype, the geometric mean of two by as much, and the result is rounded once more."""
+    mean = (torch.rand(cols, generator=torch.Generator().manual_seed(cols)) + 0.01).to(dtype)
+    got = ops.awq_candidates(mean.to(dev), [0.0, 0.5]).cpu()
+    low = torch.tensor(1e-4, dtype=dtype)
+    root = torch.maximum(mean.float().sqrt().to(dtype), low)
+    norm = (root.max().double() * root.min().double()).sqrt()
+    assert_bits_equal(got[0], torch.ones(cols, dtype=dtype))
+    want = torch.maximum((root.double() / norm).float().to(dtype), low).double()
+    assert float(((got[1].double() - want).abs() / want).max()) <= 2.5 * torch.finfo(dtype).eps
