@@ -5,6 +5,7 @@
 //   general path : scalar kernel for ragged / unaligned shapes (zero-pad semantics).
 // Reference behaviour: amct_pytorch/quantize_op/utils.py:75-136,
 // amct_pytorch/utils/quant_util.py:56-93,162-188, amct_pytorch/algorithm/awq.py:129-170.
+#include <algorithm>
 #include <type_traits>
 
 #include "amct_common.h"
@@ -338,40 +339,113 @@ __global__ __launch_bounds__(kBlock) void fq_fused(FqArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// params kernel: factors given; flat over 16-byte vectors (cols % VEC == 0).
+// params kernel: factors given; flat over 16-byte vectors (cols % VEC == 0), U consecutive block-wide pieces of them a block.
+// The U vectors of a lane are asked for before anything else, then their factors; the row and group of a vector come from
+// 32-bit products with a reciprocal (one 64-bit division a block, for the block's first row), the quotients from the fma
+// sequence of div_fast where every divisor and value of the wave allows it.  Bound by memory; one vector a lane, each behind a
+// 64-bit division and its factors, reached 3.7 TB/s.  Cold / from the last-level cache, before -> now: W[4096,4096] fp32 36.3 /
+// 24.4 -> 27.3 / 24.8 us, bf16 22.1 / 18.3 -> 18.9 / 16.6; W[4096,11008] fp16 46.8 / 38.7 -> 35.2 / 33.8.  (Loads that stay in the
+// caches: 38.4 / 23.6 for the first; stores that do: 28.4 / 26.7.)
 // ---------------------------------------------------------------------------
-template <int DT, bool VIA_SRC>
-__global__ __launch_bounds__(kBlock) void fq_params(FqArgs a, int64_t nvec) {
+// n / d and n % d for n < 2^32, with magic = min(floor(2^32 / d), 2^32 - 1): the product is short by less than 1
+struct FqDiv {
+    uint32_t d, magic;
+};
+AMCT_DEV uint32_t fq_divide(uint32_t n, const FqDiv& by, uint32_t& rest) {
+    uint32_t q = __umulhi(n, by.magic);
+    rest = n - q * by.d;
+    if (rest >= by.d) {
+        ++q;
+        rest -= by.d;
+    }
+    return q;
+}
+
+template <int DT, bool VIA_SRC, int U>
+__global__ __launch_bounds__(kBlock) void fq_params(FqArgs a, int64_t nvec, FqDiv by_row, FqDiv by_group) {
     constexpr int VEC = Tr<DT>::VEC;
     constexpr int BYTES = Tr<DT>::BYTES;
     const bool asym = a.poffset != nullptr;
-    const int64_t stride = (int64_t)gridDim.x * kBlock;
-    for (int64_t v = (int64_t)blockIdx.x * kBlock + threadIdx.x; v < nvec; v += stride) {
-        const int64_t e0 = v * VEC;
-        const int64_t row = e0 / a.cols;
-        const int64_t c0 = e0 - row * a.cols;
+    const int64_t first = (int64_t)blockIdx.x * (U * kBlock);
+    const int64_t left = nvec - first;              // vectors from the block's first one on
+    uint4 raw[U];
+    uint32_t k[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        k[u] = (uint32_t)min((int64_t)(u * kBlock + threadIdx.x), left - 1);     // (beyond the last: repeats it, not stored)
+        raw[u] = ldg16_nt(reinterpret_cast<const char*>(a.w) + (first + k[u]) * 16);
+    }
+    const int64_t row0 = nvec <= 0xFFFFFFFFll ? (int64_t)((uint32_t)first / by_row.d) : first / by_row.d;
+    const uint32_t at0 = (uint32_t)(first - row0 * by_row.d);
+    float s[U], z[U], x[U][VEC];
+    uint4 craw[U];
+    const bool cols = a.col_mode != AMCT_COL_NONE;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        uint32_t cv, rest;
+        const int64_t row = row0 + fq_divide(at0 + k[u], by_row, cv);
         int64_t pi = 0;
-        if (a.group > 0) pi = row * a.segs_per_row + c0 / a.group;
+        if (a.group > 0) pi = row * a.segs_per_row + fq_divide(cv, by_group, rest);
         else if (a.group == 0) pi = row;
-        const float s = a.pscale[pi];
-        const float z = asym ? (float)a.poffset[pi] : 0.f;
-        float x[VEC], q[VEC], d[VEC];
-        unpack16<DT>(ldg16(reinterpret_cast<const char*>(a.w) + e0 * BYTES), x);
-        float c[VEC];
-        if (a.col_mode != AMCT_COL_NONE) {
-            unpack16<DT>(ldg16(reinterpret_cast<const char*>(a.col) + c0 * BYTES), c);
-            apply_col_pre<DT>(x, c, a.col_mode);
+        s[u] = a.pscale[pi];
+        z[u] = asym ? (float)a.poffset[pi] : 0.f;
+        if (cols) craw[u] = ldg16(reinterpret_cast<const char*>(a.col) + (int64_t)cv * 16);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        unpack16<DT>(raw[u], x[u]);
+        if (cols) {
+            float c[VEC];
+            unpack16<DT>(craw[u], c);
+            apply_col_pre<DT>(x[u], c, a.col_mode);
         }
+    }
+    auto emit = [&](auto stage_tag, auto fast_tag, const Divisor* dv) {
+        constexpr int STAGE = decltype(stage_tag)::value;
+        constexpr bool FAST = decltype(fast_tag)::value;
 #pragma unroll
-        for (int j = 0; j < VEC; ++j) staged_elem<DT, VIA_SRC>(a.stage, x[j], s, z, asym, a.qmin, a.qmax, q[j], d[j]);
-        if (a.codes) store_codes<DT>(a.codes, a.codes_kind, e0, q);
-        if (a.dq) {
-            if (a.col_mode == AMCT_COL_MUL_THEN_DIV) {
+        for (int u = 0; u < U; ++u) {
+            float q[VEC], d[VEC];
 #pragma unroll
-                for (int j = 0; j < VEC; ++j) d[j] = round_to<DT>(d[j]) / c[j];
+            for (int j = 0; j < VEC; ++j) {
+                if constexpr (FAST) {
+                    q[j] = quant_elem<DT, VIA_SRC, true>(x[u][j], dv[u], z[u], asym, a.qmin, a.qmax);
+                    d[j] = dequant_elem(q[j], s[u], z[u], asym);
+                } else {
+                    staged_elem<DT, VIA_SRC>(STAGE, x[u][j], s[u], z[u], asym, a.qmin, a.qmax, q[j], d[j]);
+                }
             }
-            stg16(reinterpret_cast<char*>(a.dq) + e0 * BYTES, pack16<DT>(d));
+            if ((int64_t)(u * kBlock + threadIdx.x) < left) {
+                const int64_t e0 = (first + k[u]) * VEC;
+                if (a.codes) store_codes<DT>(a.codes, a.codes_kind, e0, q);
+                if (a.dq) {
+                    if (a.col_mode == AMCT_COL_MUL_THEN_DIV) {
+                        float c[VEC];
+                        unpack16<DT>(craw[u], c);
+#pragma unroll
+                        for (int j = 0; j < VEC; ++j) d[j] = round_to<DT>(d[j]) / c[j];
+                    }
+                    stg16_nt(reinterpret_cast<char*>(a.dq) + e0 * BYTES, pack16<DT>(d));
+                }
+            }
         }
+    };
+    if (a.stage == AMCT_STAGE_SCALE) emit(std::integral_constant<int, AMCT_STAGE_SCALE>{}, std::false_type{}, nullptr);
+    else if (a.stage == AMCT_STAGE_DEQUANT) emit(std::integral_constant<int, AMCT_STAGE_DEQUANT>{}, std::false_type{}, nullptr);
+    else if (a.stage == AMCT_STAGE_COL) emit(std::integral_constant<int, AMCT_STAGE_COL>{}, std::false_type{}, nullptr);
+    else {
+        Divisor dv[U];
+        bool ok = true;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            dv[u] = make_divisor(s[u]);
+            uint32_t big = 0;
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) big = max(big, __float_as_uint(x[u][j]) & 0x7FFFFFFFu);
+            ok = ok && dv[u].fast && big < 0x5D800000u;
+        }
+        if (wave_all(ok)) emit(std::integral_constant<int, AMCT_STAGE_FULL>{}, std::true_type{}, dv);
+        else emit(std::integral_constant<int, AMCT_STAGE_FULL>{}, std::false_type{}, nullptr);
     }
 }
 
@@ -622,6 +696,10 @@ static int run_fused(FqArgs a, hipStream_t st) {
     return hip_status();
 }
 
+// From how many 16-byte vectors on a lane takes four of them: four blocks of 1024 to a CU.  Below, the launch is what counts and
+// one vector a lane fills more CUs (W[1024,2048] fp32, half of that: 7.4 us either way; 8.8 before).
+constexpr int64_t kFqMany = 4 * 1024 * kBlock;
+
 template <int DT>
 static int run_params(FqArgs a, hipStream_t st) {
     constexpr int VEC = Tr<DT>::VEC;
@@ -629,12 +707,21 @@ static int run_params(FqArgs a, hipStream_t st) {
                         (!a.dq || aligned16(a.dq)) && (!a.codes || aligned16(a.codes)) &&
                         (a.col_mode == AMCT_COL_NONE || aligned16(a.col));
     const bool via = a.via_src && DT != AMCT_F32;
+    const int64_t row_vecs = a.cols / VEC;
+    const int group_vecs = a.group > 0 ? a.group / VEC : 1;
     if (vec_ok) {
-        const int64_t nvec = a.rows * a.cols / VEC;
-        int64_t nb = (nvec + kBlock - 1) / kBlock;
-        if (nb > 65536) nb = 65536;
-        if (via) hipLaunchKernelGGL((fq_params<DT, true>), dim3((unsigned)nb), dim3(kBlock), 0, st, a, nvec);
-        else hipLaunchKernelGGL((fq_params<DT, false>), dim3((unsigned)nb), dim3(kBlock), 0, st, a, nvec);
+        const int64_t nvec = a.rows * row_vecs;
+        auto div_by = [](int64_t d) { return FqDiv{(uint32_t)d, (uint32_t)std::min<int64_t>((int64_t(1) << 32) / d, 0xFFFFFFFFll)}; };
+        const FqDiv by_row = div_by(row_vecs), by_group = div_by(group_vecs);
+        if (nvec >= kFqMany) {
+            const dim3 grid((unsigned)((nvec + 4 * kBlock - 1) / (4 * kBlock)));
+            if (via) hipLaunchKernelGGL((fq_params<DT, true, 4>), grid, dim3(kBlock), 0, st, a, nvec, by_row, by_group);
+            else hipLaunchKernelGGL((fq_params<DT, false, 4>), grid, dim3(kBlock), 0, st, a, nvec, by_row, by_group);
+        } else {
+            const dim3 grid((unsigned)((nvec + kBlock - 1) / kBlock));
+            if (via) hipLaunchKernelGGL((fq_params<DT, true, 1>), grid, dim3(kBlock), 0, st, a, nvec, by_row, by_group);
+            else hipLaunchKernelGGL((fq_params<DT, false, 1>), grid, dim3(kBlock), 0, st, a, nvec, by_row, by_group);
+        }
         return hip_status();
     }
     if (a.rows > 0x7FFFFFFF) return AMCT_E_UNSUPPORTED;

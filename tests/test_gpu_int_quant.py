@@ -328,3 +328,34 @@ def test_column_scaled_fake_quant_beyond_the_largest_fp16(dev, rows, cols, group
     assert sym or bool(want.isinf().any()) and not bool(want.isnan().any())
     got, _, _, _ = ops.fakequant_int(w.to(dev), 4, sym, group=group, col_scale=c.to(dev), col_mode=ops.COL_MUL_THEN_DIV, via_src=True)
     assert_bits_equal(got, want, "awq grid step")
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows,cols,group", [(1, 8, 0), (3, 24, 8), (129, 2040, 0), (1, 2048, 64),        # a vector a lane
+                                             (1024, 8192, 128), (1048577, 8, 0), (1, 8390664, 8), (2051, 4104, 72),   # four
+                                             (50001, 168, -1)])
+def test_given_factors_flat_against_the_general_kernel(dev, dtype, rows, cols, group):
+    """The flat kernel at few and many vectors, rows shorter and longer than a block's piece, pieces that end early, groups that
+    do not divide the row: the bits of the scalar kernel, which takes the same values from an address off 16 bytes.  A scale of 0
+    or 1e-30, infinities, NaN, tiny values and -0.0 send their wave to the divisions."""
+    w = torch.randn(rows, cols, device=dev, generator=torch.Generator(dev).manual_seed(cols)).to(dtype)
+    w.view(-1)[-1] = -0.0
+    w.view(-1)[:4] = torch.tensor([float('inf'), float('nan'), 1e-30, -1e-30], device=dev).to(dtype)
+    count = 1 if group < 0 else rows if group == 0 else rows * -(-cols // group)
+    scale = torch.rand(count, device=dev) * 0.02 + 0.001
+    if count > 9:
+        scale[7], scale[8] = 0.0, 1e-30
+    offset = torch.randint(-8, 8, (count,), device=dev, dtype=torch.int32)
+    col = (torch.rand(cols, device=dev) + 0.5).to(dtype)
+    shifted = torch.empty(rows * cols + 1, device=dev, dtype=dtype)[1:].view(rows, cols)
+    shifted.copy_(w)
+    bits = torch.int32 if dtype == torch.float32 else torch.int16
+    for kw in (dict(codes_kind=ops.CODES_I8), dict(offset=offset, codes_kind=ops.CODES_I32, via_src=True),
+               dict(offset=offset, col_scale=col, col_mode=ops.COL_MUL_THEN_DIV), dict(col_scale=col, col_mode=ops.COL_DIV),
+               dict(offset=offset, stage=ops.STAGE_SCALE), dict(offset=offset, stage=ops.STAGE_DEQUANT)):
+        kw = dict(kw)
+        z = kw.pop("offset", None)
+        got, codes = ops.quant_with_params(w, scale, z, group, -128, 127, **kw)
+        want, want_codes = ops.quant_with_params(shifted, scale, z, group, -128, 127, **kw)
+        assert bool(((got.view(bits) == want.view(bits)) | (got.isnan() & want.isnan())).all()), kw.keys()
+        assert codes is None or torch.equal(codes, want_codes), kw.keys()
