@@ -497,8 +497,10 @@ extern "C" int amct_gptq_factor(const float* hessian, const int64_t* perm, const
     if (cols > kFgMax) return AMCT_E_TOO_LARGE;
     if (workspace_bytes < amct_gptq_factor_workspace_bytes(cols)) return AMCT_E_BADARG;
     if (!aligned16(workspace)) return AMCT_E_ALIGN;
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(gqf_step_k), hipFuncAttributeMaxDynamicSharedMemorySize, kFbLdsAlone) != hipSuccess)
-        return hip_status();
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(gqf_step_k), hipFuncAttributeMaxDynamicSharedMemorySize, kFbLdsAlone) != hipSuccess) {
+        (void)hipGetLastError();
+        return AMCT_E_HIP;
+    }
     hipStream_t st = (hipStream_t)stream;
     const int64_t Cp = (cols + kFb - 1) / kFb * kFb;
     const int n = (int)(Cp / kFb);

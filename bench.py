@@ -519,7 +519,7 @@ def build_cases(dev, only):
                                              wsh.data_ptr(), wsh.numel(), st)
                 assert rc == 0, rc
             cases.append(Case("gptq_hessian_update", "mfma_bf16", work, "flop", launch, 4, "bf16",
-                              "GPTQ Hessian update H[4096,4096] += X^T X, X[2048,4096] bf16 (transpose + symmetric MFMA kernel; "
+                              "GPTQ Hessian update H[4096,4096] += X^T X, X[2048,4096] bf16 (symmetric MFMA kernel; "
                               "flops of the lower triangle)"))
         if want("lib_hessian_update_fp32"):
             def launch(i, xh=xh, hh=hh):
