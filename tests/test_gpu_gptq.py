@@ -387,3 +387,18 @@ def test_gptq_block_gives_its_errors_in_parts(dev, n, count):
     w[n // 2, count // 3] = float('inf')
     gptq.gptq_block(w, 0, count, hinv, scale, None, gidx, -8, 7, errors[:, :count], parts[:, :, :count], wide)
     assert int(wide) == 1
+
+
+@pytest.mark.parametrize("columns", [3, 64, 66, 1020, 1027, 2052, 4100])
+def test_gptq_factor_of_a_matrix_off_16_bytes(dev, columns):
+    """Rows fetched 16 bytes at a time (columns a multiple of 4, an aligned matrix) and word by word hold the same values: the same
+    factor bit for bit, for one piece of a lane's loads and for more."""
+    x = torch.randn(2 * columns, columns, device=dev, generator=torch.Generator(dev).manual_seed(columns))
+    h = x.t() @ x / (2 * columns)
+    h = (h + h.t()) / 2
+    perm = torch.randperm(columns, device=dev)
+    damp = torch.tensor(0.01, device=dev)
+    bad = torch.zeros(1, dtype=torch.int32, device=dev)
+    shifted = torch.empty(columns * columns + 1, device=dev)[1:].view(columns, columns)
+    shifted.copy_(h)
+    assert torch.equal(ops.gptq_factor(h, perm, damp, bad), ops.gptq_factor(shifted, perm, damp, bad)) and int(bad) == 0
